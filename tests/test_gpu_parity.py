@@ -161,6 +161,19 @@ def test_decorations(ctx, flags, ref_tiles, size):
     assert_same(scene, ctx.draw(scene), refcpu.draw(scene))
 
 
+@pytest.mark.parametrize("ref_tiles,size", [
+    (16, (513, 259)), (16, (256, 65)), (1, (320, 129)), (16, (1, 9)), (1, (70, 1)),
+])
+def test_decorations_line_lengths(ctx, ref_tiles, size):
+    """Lines of one pixel, of whole and of broken 64-pixel runs, and borders
+    whose start lies past the frame's edge."""
+    import scene_cases as C
+    scene = C.sphere(w=size[0], h=size[1], eye=(0, 0, 2.4),
+                     flags=C.ALL | _lib.GR_SHOW_TILE_BOUNDS | _lib.GR_SHOW_CROSSHAIR)
+    scene.frame.ref_tiles = ref_tiles
+    assert_same(scene, ctx.draw(scene), refcpu.draw(scene))
+
+
 def test_decorations_batched(ctx):
     """Decorated and plain frames in one batch into shared buffers: each frame
     keeps only its own decorations, and a following draw into the same
