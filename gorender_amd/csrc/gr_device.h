@@ -180,9 +180,7 @@ enum : int32_t {
 struct DevBatchCounters {
     unsigned long long refs_used;  // tile-list entries allocated so far
     uint32_t n_items;              // raster work items (later parts of split tiles)
-    uint32_t next_item;            // next work item to take
     uint32_t n_slabs;              // slabs handed to split tiles
-    uint32_t pad;
     unsigned long long recs_used;  // triangle records the face blocks claimed (k_bin_scan)
 };
 

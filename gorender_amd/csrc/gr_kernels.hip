@@ -2082,8 +2082,8 @@ __device__ __forceinline__ unsigned long long shade_tile(const DevFrame& fr, int
 
 // A tile whose list holds more than part_refs entries, and that k_bin_scan gave
 // a slab, is split into parts of part_refs entries. Parts 1.. are work items
-// that k_raster_parts resolves first, any workgroup taking the next item from
-// the batch queue: each resolves its entries into LDS keys and merges them into
+// that k_raster_parts resolves first, workgroup w taking items w, w + grid, ...:
+// each resolves its entries into LDS keys and merges them into
 // the tile's slab in HBM with a 64-bit max (the (depth, sequence) resolve does
 // not depend on order). k_raster then resolves part 0 of every tile, folds in
 // the slab of a split tile (and clears it) and shades.
@@ -2103,46 +2103,28 @@ void k_raster_parts(const DevFrame* __restrict__ frames, int nframes,
     __shared__ uint32_t lslot[kRasterChunk];
     __shared__ uint32_t qbuf[4][3][128];
     __shared__ unsigned long long red;  // covered fragments of the item
-    __shared__ RasterItem litem;
     const int lane = threadIdx.x & 63, wave = sgpr(threadIdx.x >> 6);
     // Written by k_bin_scan (an earlier kernel).
     const uint32_t n_items = min(counters->n_items, max_items);
     if (n_items == 0u) return;
-    // Every branch around the barriers of this loop is wave-uniform (scalar):
-    // thread-level branches here (a thread-0 fetch, an exit on a value read
-    // from LDS) let the compiler restructure the loop so that thread 0 leaves
-    // it while the other threads go round the barriers again, which hangs.
-    for (;;) {
-        if (wave == 0) {
-            // Lane 0 fetches the next item; the wave publishes it.
-            uint32_t it = kNoSlab;
-            if (lane == 0) {
-                it = __hip_atomic_load(&counters->next_item, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-                if (it < n_items)
-                    it = __hip_atomic_fetch_add(&counters->next_item, 1u, __ATOMIC_RELAXED,
-                                                __HIP_MEMORY_SCOPE_AGENT);
-            }
-            it = (uint32_t)sgpr((int)it);
-            const RasterItem w = it < n_items ? items[it] : RasterItem{kNoSlab, 0u};
-            if (lane == 0) {
-                litem = w;
-                red = 0ull;
-            }
-        }
-        __syncthreads();
-        const uint32_t wtile = (uint32_t)sgpr((int)litem.tile);
-        const uint32_t wpart = (uint32_t)sgpr((int)litem.part);
-        if (wtile == kNoSlab) return;
-        const int tile = (int)wtile;
+    // A fixed stride, not a queue counter: atomics of one cache line are served
+    // one every 12 ns, so the ~6,000 items and 2,048 workgroups of a batch of 8
+    // dense requests waited for the counter (k_raster_parts 414 -> 322 us), and
+    // the items are of one size. Every branch around the barriers of this loop
+    // is wave-uniform (scalar): thread-level branches here let the compiler
+    // restructure the loop so that one thread leaves it while the others go
+    // round the barriers again, which hangs.
+    for (uint32_t it = blockIdx.x; it < n_items; it += gridDim.x) {
+        const int tile = sgpr((int)items[it].tile);
+        const uint32_t wpart = (uint32_t)sgpr((int)items[it].part);
+        if (threadIdx.x == 0) red = 0ull;  // ordered by raster_list's barriers
         const int fi = last_le(nframes, tile, [&](int i) { return frames[i].tile_begin; });
         const DevFrame& fr = frames[fi];
         const int t = tile - fr.tile_begin;
         const int X0 = (t % fr.tiles_x) * TW, Y0 = (t / fr.tiles_x) * TH;
         const uint32_t cnt = tile_counts[tile], beg = wpart * part_refs;
         for (int i = threadIdx.x; i < NPX; i += 256) key[i] = kBackgroundKey;
-        // raster_list's first barrier orders the initialisation (and the read of
-        // litem) before what follows.
+        // raster_list's first barrier orders the initialisation before its use.
         unsigned long long covered =
             raster_list<TW, TH>(fr, X0, Y0, refs + tile_offsets[tile] + beg,
                                 min(cnt - beg, part_refs), key, lrec, lslot, qbuf[wave], lane,
@@ -2157,7 +2139,7 @@ void k_raster_parts(const DevFrame* __restrict__ frames, int nframes,
         if (lane == 0 && cov) atomicAdd(&red, cov);
         __syncthreads();
         if (wave == 0 && lane == 0 && red) atomicAdd(&stats[fi * kNumStats + kStatCovered], red);
-        // litem and red are read before the next item overwrites them.
+        // red and the LDS tile state are read before the next item overwrites them.
         __syncthreads();
     }
 }
@@ -2522,7 +2504,7 @@ static void raster_t(const LaunchParams& p, hipStream_t s, bool parts) {
         // Workgroups of the parts kernel: enough to fill every CU at the
         // raster's occupancy, but no more than the batch has tiles (a single
         // frame rarely splits many); with no work items they return at once,
-        // and any number of them drains the queue.
+        // and any number of them covers the items.
         const uint32_t grid = std::min<uint32_t>(
             std::min<uint32_t>(p.max_items, 256u * (uint32_t)raster_waves(TW * TH)),
             std::max<uint32_t>(256u, (uint32_t)p.total_tiles));
