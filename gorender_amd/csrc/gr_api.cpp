@@ -72,13 +72,12 @@ struct Pipe {
     hipStream_t stream = nullptr;
     // batch: frames | objects | stats | counters | frame_overflow | XCD tables,
     // uploaded with one copy per draw (the counters as zeros).
-    DevBuf batch, rrec, srec, wrec, tile_counts, tiles, wgcount, refs, ctrl;
+    DevBuf batch, rrec, srec, wrec, tile_counts, tiles, blocks, refs, ctrl;
     DevBuf items;  // raster work items (later parts of split tiles)
     DevBuf slabs;  // depth keys of split tiles; zero between draws
     DevBuf okey;   // overlay keys of the frames that draw overlays; zero between draws
     DevBuf orec;   // overlay records per triangle record (batches with overlay frames)
-    DevBuf rbase;  // record pool counters (zero between draws), then each face block's first
-                   // overflow record
+    DevBuf pools;  // record pool counters (zero between draws)
     hipEvent_t raster_done = nullptr;  // after this pipe's last k_raster
     bool raster_pending = false;
 };
@@ -499,7 +498,7 @@ gr_status make_plan(gr_context* c, const gr_batch_frame* bf, int nf, const gr_ob
         d.rrec = nullptr;
         d.srec = nullptr;
         d.wrec = nullptr;
-        d.rbase = nullptr;
+        d.blocks = nullptr;
     }
     P.nobj = nobj;
     P.off_objs = align256((size_t)nf * sizeof(gr::DevFrame));
@@ -529,13 +528,13 @@ struct Bufs {
     char* header = nullptr;  // frames | objects | stats | counters | frame_overflow | XCD tables
     // Triangle records [face blocks * kRecsPerBlock + rec_pools * pool_recs]:
     // each face block's own, then the overflow pools, claimed by the blocks
-    // that need more as they run; rbase [face blocks] holds each block's first
+    // that need more as they run; blocks [face blocks] holds each block's first
     // overflow record, rec_pool the pool counters (zero between draws).
     gr::RasterRec* rrec = nullptr;
     gr::ShadeRec* srec = nullptr;
     gr::WideRec* wrec = nullptr;
     uint32_t rec_pools = 1, pool_recs = 0;
-    uint32_t* rbase = nullptr;
+    gr::FaceBlock* blocks = nullptr;
     uint32_t* rec_pool = nullptr;
     uint32_t* tile_counts = nullptr;  // zero between draws (k_raster re-zeroes)
     uint32_t* tiles = nullptr;        // offsets | cursors | slabs
@@ -544,7 +543,6 @@ struct Bufs {
     unsigned long long* slabs = nullptr;  // zero between draws
     uint32_t max_slabs = 0;
     uint32_t part_refs = 0;
-    uint32_t* wgcount = nullptr;
     uint32_t* refs = nullptr;
     unsigned long long refs_cap = 0;
     gr::DevControl* ctrl = nullptr;  // sticky until read
@@ -577,7 +575,7 @@ void write_header(const Plan& P, const Bufs& B, void* h) {
         d.rrec = B.rrec;
         d.srec = B.srec;
         d.wrec = B.wrec;
-        d.rbase = B.rbase + d.face_block_begin;
+        d.blocks = B.blocks + d.face_block_begin;
     }
     if (P.nobj) std::memcpy((char*)h + P.off_objs, P.dobj, (size_t)P.nobj * sizeof(gr::DevObject));
     std::memcpy((char*)h + P.off_xcd, P.xcd, xcd_ints(P.nf) * sizeof(int));
@@ -605,8 +603,7 @@ gr::LaunchParams launch_params(const Plan& P, const Bufs& B) {
     p.max_slabs = B.max_slabs;
     p.part_refs = B.part_refs;
     p.frame_overflow = (uint32_t*)(bb + P.off_over);
-    p.wg_count = B.wgcount;
-    p.rec_base = B.rbase;
+    p.blocks = B.blocks;
     p.rec_pool = B.rec_pool;
     p.rec_pools = B.rec_pools;
     p.pool_recs = B.pool_recs;
@@ -686,8 +683,7 @@ gr_status size_bufs(gr_context* c, const Plan& P, Pipe& Q, unsigned long long re
     if ((st = ensure(c, Q.rrec, recs * sizeof(gr::RasterRec)))) return st;
     if ((st = ensure(c, Q.srec, recs * sizeof(gr::ShadeRec)))) return st;
     if ((st = ensure(c, Q.wrec, recs * sizeof(gr::WideRec)))) return st;
-    if ((st = ensure_zeroed(c, Q.rbase, (kPoolWords + std::max(P.fblocks, 1)) * sizeof(uint32_t), s)))
-        return st;
+    if ((st = ensure_zeroed(c, Q.pools, kPoolWords * sizeof(uint32_t), s))) return st;
     if ((st = ensure_zeroed(c, Q.tile_counts, (size_t)P.tiles * 4, s))) return st;
     if ((st = ensure(c, Q.tiles, 3 * (size_t)P.tiles * sizeof(uint32_t)))) return st;
     const size_t slab_bytes = (size_t)TW * TH * 8;
@@ -695,7 +691,7 @@ gr_status size_bufs(gr_context* c, const Plan& P, Pipe& Q, unsigned long long re
     split_limits(refs_cap, part_refs, slab_bytes, &max_items, &max_slabs);
     if ((st = ensure(c, Q.items, (size_t)max_items * sizeof(gr::RasterItem)))) return st;
     if ((st = ensure_zeroed(c, Q.slabs, (size_t)max_slabs * slab_bytes, s))) return st;
-    if ((st = ensure(c, Q.wgcount, std::max(P.fblocks, 1) * sizeof(uint32_t)))) return st;
+    if ((st = ensure(c, Q.blocks, std::max(P.fblocks, 1) * sizeof(gr::FaceBlock)))) return st;
     if ((st = ensure(c, Q.refs, refs_cap * sizeof(uint32_t)))) return st;
     if ((st = ensure_zeroed(c, Q.ctrl, sizeof(gr::DevControl), s))) return st;
     if (P.okey_words) {
@@ -708,8 +704,7 @@ gr_status size_bufs(gr_context* c, const Plan& P, Pipe& Q, unsigned long long re
     B.wrec = (gr::WideRec*)Q.wrec.p;
     B.rec_pools = pools;
     B.pool_recs = per;
-    B.rec_pool = (uint32_t*)Q.rbase.p;
-    B.rbase = B.rec_pool + kPoolWords;
+    B.rec_pool = (uint32_t*)Q.pools.p;
     B.tile_counts = (uint32_t*)Q.tile_counts.p;
     B.tiles = (uint32_t*)Q.tiles.p;
     B.items = (gr::RasterItem*)Q.items.p;
@@ -717,7 +712,7 @@ gr_status size_bufs(gr_context* c, const Plan& P, Pipe& Q, unsigned long long re
     B.slabs = (unsigned long long*)Q.slabs.p;
     B.max_slabs = max_slabs;
     B.part_refs = part_refs;
-    B.wgcount = (uint32_t*)Q.wgcount.p;
+    B.blocks = (gr::FaceBlock*)Q.blocks.p;
     B.refs = (uint32_t*)Q.refs.p;
     B.refs_cap = refs_cap;
     B.ctrl = (gr::DevControl*)Q.ctrl.p;
@@ -921,8 +916,8 @@ gr_status present_enqueue(gr_context* c, gr_context::PresentSlot& ps) {
 
 void free_pipe_bufs(Pipe& pp) {
     DevBuf* pb[] = {&pp.batch, &pp.rrec,    &pp.srec, &pp.wrec,  &pp.tile_counts,
-                    &pp.tiles, &pp.wgcount, &pp.refs, &pp.ctrl,  &pp.items,
-                    &pp.slabs, &pp.okey,    &pp.orec,  &pp.rbase};
+                    &pp.tiles, &pp.blocks,  &pp.refs, &pp.ctrl,  &pp.items,
+                    &pp.slabs, &pp.okey,    &pp.orec,  &pp.pools};
     for (DevBuf* b : pb) {
         if (b->p) (void)hipFree(b->p);
         *b = DevBuf{};
@@ -1148,10 +1143,11 @@ gr_status check_request(gr_context* c, const gr_frame* frame, const gr_object* o
 
 // The no-allocation draw. Layout of [base, base + bytes): control words (sticky
 // until gr_synchronize reads them), batch header, texture table, tile counters,
-// tile offsets/cursors/slabs, face-block counts and first records, then what
-// remains shared between triangle records and tile-list entries, as many of
-// each (fewer records when the frame has fewer slots). Tiles are never split
-// (no slabs or work items).
+// tile offsets/cursors/slabs, 8 bytes per face block, then what remains shared
+// between triangle records and tile-list entries, as many of each (fewer records
+// when the frame has fewer slots). Tiles are never split (no slabs or work
+// items). Behind the array's `bytes`, which decide what fits a draw, its tail of
+// kNoAllocTail bytes holds the face blocks' state.
 // Host data reaches the array through kernel arguments (k_put) and zeroing is
 // a fill kernel, so nothing here allocates memory of any kind, and the launch
 // sequence holds no memset or host-buffer copy.
@@ -1191,9 +1187,9 @@ gr_status enqueue_noalloc(gr_context* c, const gr_frame* frame, const gr_object*
         B.textures = (const gr::DevTexture*)take(ntex * sizeof(gr::DevTexture));
         B.tile_counts = (uint32_t*)take((size_t)P.tiles * 4);
         B.tiles = (uint32_t*)take(3 * (size_t)P.tiles * 4);
-        B.wgcount = (uint32_t*)take((size_t)std::max(P.fblocks, 1) * 4);
         B.rec_pool = (uint32_t*)take(kPoolWords * 4);
-        B.rbase = (uint32_t*)take((size_t)std::max(P.fblocks, 1) * 4);
+        off += 2 * align256((size_t)std::max(P.fblocks, 1) * 4);
+        B.blocks = (gr::FaceBlock*)((char*)base + bytes);
         constexpr size_t kRecBytes =
             sizeof(gr::RasterRec) + sizeof(gr::ShadeRec) + sizeof(gr::WideRec);
         const size_t min_refs = 1u << 16;
@@ -1207,6 +1203,8 @@ gr_status enqueue_noalloc(gr_context* c, const gr_frame* frame, const gr_object*
                           "frame too large for the no-allocation draw: needs " +
                               std::to_string(need >> 20) +
                               " MiB of its 32 MiB device array (use gr_draw_device)");
+        if ((size_t)P.fblocks * sizeof(gr::FaceBlock) > kNoAllocTail)
+            return ::fail(GR_ERR_INVALID_ARGUMENT, "frame too large for the no-allocation draw");
         // The rest: kOvfRefs tile-list entries per overflow record.
         const size_t rest = bytes - off - 4 * 256 - own * kRecBytes;
         record_pools(P, rest / (kRecBytes + 4 * gr::kOvfRefs) * gr::kOvfRefs, &B.rec_pools,

@@ -115,11 +115,18 @@ struct DevFrame {
     // Triangle records of the batch. A slot (the draw-order number of a
     // triangle: frame-local face block * kSlotsPerWg + its offset in the
     // block) has its record in the block's own range (offsets below
-    // kRecsPerBlock) or at rbase[block] + offset - kRecsPerBlock.
+    // kRecsPerBlock) or at blocks[block].ovf + offset - kRecsPerBlock.
     struct RasterRec* rrec;
     struct ShadeRec* srec;
     struct WideRec* wrec;
-    const uint32_t* rbase;       // first overflow record of each face block of this frame
+    const struct FaceBlock* blocks;  // the face blocks of this frame
+};
+
+// What k_face leaves of one face block: the slots it filled, its first overflow
+// record, and its counters in 16-bit fields (TPF references | binned triangles
+// << 16, front faces | clip overflows << 16).
+struct alignas(16) FaceBlock {
+    uint32_t count, ovf, c0, c1;
 };
 
 // Per-triangle raster set-up, 80 bytes: what the visibility pass reads. The

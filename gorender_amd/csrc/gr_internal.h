@@ -40,8 +40,9 @@ void set_one_pipe(gr_context* c, bool on);
 // address on `device` (current), and look it up.
 gr_status static_scratch_init(int device);
 void* static_scratch(int device, size_t* bytes);
-// One frame drawn with every per-draw buffer carved from [base, base + bytes):
-// no allocation of any kind on the way.
+// One frame drawn with every per-draw buffer carved from [base, base + bytes +
+// kNoAllocTail): no allocation of any kind on the way.
+constexpr size_t kNoAllocTail = 64u << 10;
 gr_status enqueue_noalloc(gr_context* c, const gr_frame* frame, const gr_object* objs, int32_t no,
                           void* d_rgba, void* d_depth, void* base, size_t bytes);
 

@@ -17,10 +17,10 @@
 
 namespace {
 
-// 32 MiB per GPU, held from the library's load on the device until the
+// 32 MiB (and the tail) per GPU, held from the library's load on the device until the
 // process ends.
 constexpr size_t kScratchBytes = 32u << 20;
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+static __device__ __align__(256) unsigned char scratch[kScratchBytes + gr_internal::kNoAllocTail];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_mu;

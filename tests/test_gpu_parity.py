@@ -174,6 +174,22 @@ def test_decorations_line_lengths(ctx, ref_tiles, size):
     assert_same(scene, ctx.draw(scene), refcpu.draw(scene))
 
 
+@pytest.mark.parametrize("size", [(512, 256), (505, 249), (520, 256), (8, 8), (1, 1)])
+@pytest.mark.parametrize("grid,eye", [((3, 5), 1.1), ((60, 90), 1.3), ((60, 90), 6.0)])
+def test_tile_counting(ctx, size, grid, eye):
+    """Frames of exactly 2,048 tiles, one row and one column short of it, past
+    it and of one tile, with triangles of hundreds of tiles, of a few and of
+    less than one."""
+    import scene_cases as C
+    scene = C.sphere(w=size[0], h=size[1], eye=(0, 0, eye), nlat=grid[0], nlon=grid[1])
+    old = ctx.config()
+    ctx.set_config(tile_w=8, tile_h=8)
+    try:
+        assert_same(scene, ctx.draw(scene), refcpu.draw(scene))
+    finally:
+        ctx.set_config(tile_w=old.tile_w, tile_h=old.tile_h)
+
+
 def test_decorations_batched(ctx):
     """Decorated and plain frames in one batch into shared buffers: each frame
     keeps only its own decorations, and a following draw into the same
