@@ -770,21 +770,41 @@ __device__ uint32_t emit_triangle(const DevFrame& fr, const CV& a, const CV& b, 
                 wr.pad[0] = wr.pad[1] = wr.pad[2] = 0;
                 gstore(&fr.wrec[ri], wr);
             }
-            ShadeRec sr;
-            // u, v as clipped; finalize_record divides them by z (rasterizer.go:132-137).
-            sr.uz[0] = a.u;
-            sr.vz[0] = a.v;
-            sr.uz[1] = b.u;
-            sr.vz[1] = b.v;
-            sr.uz[2] = c.u;
-            sr.vz[2] = c.v;
-            sr.in[0] = a.i;
-            sr.in[1] = b.i;
-            sr.in[2] = c.i;
-            sr.tex = tex;
-            sr.sf = rr.sf;
-            sr.rsf = rr.wide ? kShadeWide : 0u;  // finalize_record sets a reciprocal
-            gstore(&fr.srec[ri], sr);
+            // Nothing reads the shading inputs and reciprocals of an empty box. The
+            // divisions only the raster stage needs are done here, where the
+            // triangle is in registers: in k_bin_fill they cost reading 64 and
+            // writing 48 bytes of every record again (8 requests over 4M resident
+            // triangles: k_bin_fill 177 -> 121 us, k_face unchanged; 32 frames of
+            // 200,000: 50 -> 44 and 116 -> 122 us).
+            if (rr.bx0 <= rr.bx1) {
+                // The reciprocals of the divisors for the exact quotient path, whose
+                // numerators are nonzero int32 edge values and barycentrics with
+                // |alpha|, |beta| >= 2^-41 and gamma = +0 or |gamma| >= 2^-64 (left 0,
+                // i.e. IEEE division, for int64 triangles and divisors outside
+                // rcp_range).
+                if (!rr.wide && rcp_range(rr.sf) && rcp_range(rr.z0) && rcp_range(rr.z1) &&
+                    rcp_range(rr.z2)) {
+                    rr.rsf = 1.0f / rr.sf;
+                    rr.rz0 = 1.0f / rr.z0;
+                    rr.rz1 = 1.0f / rr.z1;
+                    rr.rz2 = 1.0f / rr.z2;
+                }
+                ShadeRec sr;
+                // rasterizer.go:132-137
+                sr.uz[0] = a.u / rr.z0;
+                sr.vz[0] = a.v / rr.z0;
+                sr.uz[1] = b.u / rr.z1;
+                sr.vz[1] = b.v / rr.z1;
+                sr.uz[2] = c.u / rr.z2;
+                sr.vz[2] = c.v / rr.z2;
+                sr.in[0] = a.i;
+                sr.in[1] = b.i;
+                sr.in[2] = c.i;
+                sr.tex = tex;
+                sr.sf = rr.sf;
+                sr.rsf = rr.wide ? kShadeWide : __float_as_uint(rr.rsf);
+                gstore(&fr.srec[ri], sr);
+            }
         }
     }
     gstore(&fr.rrec[ri], rr);
@@ -871,6 +891,15 @@ __device__ __forceinline__ TileRect box_tiles(uint32_t bx, uint32_t by, int twl,
     return t;
 }
 
+// fn(x, y) for every point of a (wave-uniform) rectangle, by the lanes of one
+// wave: a power of two of lanes per row.
+template <typename F>
+__device__ __forceinline__ void wave_rect(int x0, int y0, int x1, int y1, int lane, F fn) {
+    const int l2 = min(x1 == x0 ? 0 : 32 - __builtin_clz((uint32_t)(x1 - x0)), 6);
+    for (int y = y0 + (lane >> l2); y <= y1; y += 64 >> l2)
+        for (int x = x0 + (lane & ((1 << l2) - 1)); x <= x1; x += 1 << l2) fn(x, y);
+}
+
 __device__ __forceinline__ TileRect rec_tiles(const RasterRec* r, int twl, int thl) {
     const uint4 p2 = gload(reinterpret_cast<const uint4*>(r) + 2);
     return box_tiles(p2.x, p2.y, twl, thl);
@@ -879,79 +908,6 @@ __device__ __forceinline__ TileRect rec_tiles(const RasterRec* r, int twl, int t
 // ---------------------------------------------------------------------------
 // k_face
 // ---------------------------------------------------------------------------
-
-// Per-triangle divisions only the raster stage needs, done once per record
-// after the face stage: u/z and v/z (rasterizer.go:132-137; the face stage
-// stores u and v) and the reciprocals of the divisors for the exact quotient
-// path, whose numerators are nonzero int32 edge values and barycentrics with
-// |alpha|, |beta| >= 2^-41 and gamma = +0 or |gamma| >= 2^-64 (left 0, i.e.
-// IEEE division, for int64 triangles and divisors outside rcp_range).
-__device__ __forceinline__ TileRect finalize_record(RasterRec* r, ShadeRec* sr, int twl, int thl) {
-    const float4 d = gload(reinterpret_cast<const float4*>(r));
-    const uint4 p2 = gload(reinterpret_cast<const uint4*>(r) + 2);
-    const TileRect t = box_tiles(p2.x, p2.y, twl, thl);
-    if (t.tx0 > t.tx1) return t;  // not rasterised; no shading inputs were written
-    // Pieces 0 and 1 of the shading record: uz[0..2], vz[0] | vz[1], vz[2], in[0], in[1].
-    static_assert(offsetof(ShadeRec, vz) == 12 && offsetof(ShadeRec, in) == 24,
-                  "shading record pieces");
-    float4 s0 = gload(reinterpret_cast<const float4*>(sr));
-    float4 s1 = gload(reinterpret_cast<const float4*>(sr) + 1);
-    s0.x = s0.x / d.y;  // uz[0]
-    s0.w = s0.w / d.y;  // vz[0]
-    s0.y = s0.y / d.z;  // uz[1]
-    s1.x = s1.x / d.z;  // vz[1]
-    s0.z = s0.z / d.w;  // uz[2]
-    s1.y = s1.y / d.w;  // vz[2]
-    gstore(reinterpret_cast<float4*>(sr), s0);
-    gstore(reinterpret_cast<float4*>(sr) + 1, s1);
-    if (!p2.z && rcp_range(d.x) && rcp_range(d.y) && rcp_range(d.z) && rcp_range(d.w)) {
-        const float4 rc = make_float4(1.0f / d.x, 1.0f / d.y, 1.0f / d.z, 1.0f / d.w);
-        gstore(reinterpret_cast<float4*>(r) + 1, rc);
-        gst(&sr->rsf, __float_as_uint(rc.x));  // the shading pass reads it from here
-    }
-    return t;
-}
-
-// Exclusive block scan of small counts (256 threads = 4 waves).
-// Exclusive scan over the workgroup of per-face fan sizes, which are 0, 1, 2
-// or kMaxFan: the in-wave prefix is counted from three ballots (no cross-lane
-// shuffles, whose lane addresses would need registers at the point where
-// k_face holds the most), the wave totals go through LDS.
-__device__ __forceinline__ int fan_exclusive_scan(int v, int* lds4, int& total) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint64_t b1 = __ballot(v == 1), b2 = __ballot(v == 2), b7 = __ballot(v == kMaxFan);
-    const uint64_t lt = lanemask_lt(lane);
-    const int x = __popcll(b1 & lt) + 2 * __popcll(b2 & lt) + kMaxFan * __popcll(b7 & lt);
-    if (lane == 0) lds4[wave] = __popcll(b1) + 2 * __popcll(b2) + kMaxFan * __popcll(b7);
-    __syncthreads();
-    int base = 0;
-    total = 0;
-    for (int w = 0; w < 4; w++) {
-        const int t = lds4[w];
-        if (w < wave) base += t;
-        total += t;
-    }
-    return base + x;
-}
-
-__device__ __forceinline__ int block_exclusive_scan(int v, int* lds4, int& total) {
-    int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int x = v;
-    for (int o = 1; o < 64; o <<= 1) {
-        int y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-    }
-    if (lane == 63) lds4[wave] = x;
-    __syncthreads();
-    int base = 0;
-    total = 0;
-    for (int w = 0; w < 4; w++) {
-        int t = lds4[w];
-        if (w < wave) base += t;
-        total += t;
-    }
-    return base + x - v;
-}
 
 // Clip-space corner k of a face: MVP * (x, y, z, w) (renderer.go:303-304,318-320).
 __device__ __forceinline__ float4 corner(const DevObject& o, int v) {
@@ -1043,11 +999,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
                 for (int tx = t.tx0; tx <= t.tx1; tx++) add((uint32_t)(ty * fr.tiles_x + tx));
         for (uint64_t big = __ballot(w > 0 && n > kLaneTiles); big; big &= big - 1) {
             const int L = __builtin_ctzll(big);
-            const int bw = __builtin_amdgcn_readlane(w, L), bn = __builtin_amdgcn_readlane(n, L);
-            const int bx = __builtin_amdgcn_readlane(t.tx0, L);
-            const int by = __builtin_amdgcn_readlane(t.ty0, L);
-            for (int k = lane; k < bn; k += 64)
-                add((uint32_t)((by + k / bw) * fr.tiles_x + bx + k % bw));
+            wave_rect(__builtin_amdgcn_readlane(t.tx0, L), __builtin_amdgcn_readlane(t.ty0, L),
+                      __builtin_amdgcn_readlane(t.tx1, L), __builtin_amdgcn_readlane(t.ty1, L),
+                      lane, [&](int tx, int ty) { add((uint32_t)(ty * fr.tiles_x + tx)); });
         }
     };
     const int wg_in_obj = b - o.face_block;
@@ -1571,7 +1525,7 @@ __global__ __launch_bounds__(1024) void k_bin_scan(const DevFrame* __restrict__ 
 // k_bin_fill
 // ---------------------------------------------------------------------------
 
-__global__ __launch_bounds__(kFillThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_bin_fill(const DevObject* __restrict__ objs, int nobj,
+__global__ __launch_bounds__(kFillThreads) void k_bin_fill(const DevObject* __restrict__ objs, int nobj,
                                                   const DevFrame* __restrict__ frames,
                                                   const FaceBlock* __restrict__ blocks,
                                                   const uint32_t* __restrict__ frame_overflow,
@@ -1590,11 +1544,10 @@ __global__ __launch_bounds__(kFillThreads) __attribute__((amdgpu_waves_per_eu(8)
     // The block's slots start at slot0; its records are block_rec(b, ovf, i).
     const uint32_t blk = (uint32_t)(o.seq_block + (b - o.face_block));  // in the frame
     const uint32_t slot0 = blk * kSlotsPerWg;
-    // Tile ranges of the block's first kFillKeep * kFillThreads records stay in
-    // registers from the finalising pass to the placing pass (the records are
-    // read once); later records, if any, are read again in each pass.
-    constexpr int kFillKeep = 4;
-    TileRect tr[kFillKeep];
+    // Tile ranges of the block's first kFillKeep records stay in LDS (the records
+    // are read once); later records, if any, are read again in each pass.
+    constexpr uint32_t kFillKeep = 256;
+    __shared__ uint2 lrange[kFillKeep];  // tx0 | tx1 << 16, ty0 | ty1 << 16
     if (threadIdx.x == 0) {
         lrect[0] = 0x7FFFFFFF;
         lrect[1] = -1;
@@ -1602,36 +1555,35 @@ __global__ __launch_bounds__(kFillThreads) __attribute__((amdgpu_waves_per_eu(8)
         lrect[3] = -1;
     }
     int ax = 0x7FFFFFFF, bx = -1, ay = 0x7FFFFFFF, by = -1;
-    auto fold = [&](const TileRect& t) {
-        if (t.tx0 > t.tx1) return;
+    for (uint32_t i = threadIdx.x; i < cnt; i += kFillThreads) {
+        const uint32_t ri = block_rec(b, ovf, i);
+        const TileRect t = rec_tiles(&fr.rrec[ri], twl, thl);
+        if (i < kFillKeep)
+            lrange[i] = make_uint2((uint32_t)t.tx0 | (uint32_t)t.tx1 << 16,
+                                   (uint32_t)t.ty0 | (uint32_t)t.ty1 << 16);
+        if (t.tx0 > t.tx1) continue;
         ax = min(ax, t.tx0);
         bx = max(bx, t.tx1);
         ay = min(ay, t.ty0);
         by = max(by, t.ty1);
-    };
-#pragma unroll
-    for (int k = 0; k < kFillKeep; k++) {
-        const uint32_t i = threadIdx.x + (uint32_t)(k * kFillThreads);
-        tr[k] = TileRect{1, 0, 1, 0};
-        if (i < cnt) {
-            const uint32_t ri = block_rec(b, ovf, i);
-            tr[k] = finalize_record(&fr.rrec[ri], &fr.srec[ri], twl, thl);
-            fold(tr[k]);
-        }
     }
-    for (uint32_t i = threadIdx.x + kFillKeep * kFillThreads; i < cnt; i += kFillThreads) {
-        const uint32_t ri = block_rec(b, ovf, i);
-        fold(finalize_record(&fr.rrec[ri], &fr.srec[ri], twl, thl));
-    }
-    // Every tile range of record i, from registers or read again.
+    // fn(t, i) for the tile range of every record i, 64 records at a time by all
+    // lanes of the wave (empty past the last record).
     auto each_range = [&](auto&& fn) {
-#pragma unroll
-        for (int k = 0; k < kFillKeep; k++) {
-            const uint32_t i = threadIdx.x + (uint32_t)(k * kFillThreads);
-            if (i < cnt) fn(tr[k], i);
+        for (uint32_t i0 = 0; i0 < cnt; i0 += kFillThreads) {
+            const uint32_t i = i0 + threadIdx.x;
+            TileRect t{1, 0, 1, 0};
+            if (i < cnt) {
+                if (i < kFillKeep) {
+                    const uint2 v = lrange[i];
+                    t = TileRect{(int)(v.x & 0xFFFFu), (int)(v.x >> 16), (int)(v.y & 0xFFFFu),
+                                 (int)(v.y >> 16)};
+                } else {
+                    t = rec_tiles(&fr.rrec[block_rec(b, ovf, i)], twl, thl);
+                }
+            }
+            fn(t, i);
         }
-        for (uint32_t i = threadIdx.x + kFillKeep * kFillThreads; i < cnt; i += kFillThreads)
-            fn(rec_tiles(&fr.rrec[block_rec(b, ovf, i)], twl, thl), i);
     };
     // The union of the ranges, by LDS atomics.
     __syncthreads();
@@ -1644,43 +1596,53 @@ __global__ __launch_bounds__(kFillThreads) __attribute__((amdgpu_waves_per_eu(8)
     __syncthreads();
     const int rx0 = lrect[0], rx1 = lrect[1], ry0 = lrect[2], ry1 = lrect[3];
     if (rx1 < 0) return;
-    const int rw = rx1 - rx0 + 1, rh = ry1 - ry0 + 1;
-    if (rw * rh > kLdsTiles) {
-        // Very large rectangle: one global atomic per reference.
-        each_range([&](const TileRect& t, uint32_t i) {
-            for (int ty = t.ty0; ty <= t.ty1; ty++)
-                for (int tx = t.tx0; tx <= t.tx1; tx++) {
-                    const uint32_t pos =
-                        atomicAdd(&tile_cursor[fr.tile_begin + ty * fr.tiles_x + tx], 1u);
-                    refs[pos] = slot0 + i;
-                }
-        });
-        return;
-    }
-    for (int i = threadIdx.x; i < rw * rh; i += kFillThreads) lcnt[i] = 0u;
-    __syncthreads();
-    each_range([&](const TileRect& t, uint32_t) {
-        for (int ty = t.ty0; ty <= t.ty1; ty++)
-            for (int tx = t.tx0; tx <= t.tx1; tx++)
-                atomicAdd(&lcnt[(ty - ry0) * rw + (tx - rx0)], 1u);
-    });
-    __syncthreads();
-    // One global reservation per touched tile; lcnt becomes the write cursor.
-    for (int i = threadIdx.x; i < rw * rh; i += kFillThreads) {
-        const uint32_t v = lcnt[i];
-        if (v)
-            lcnt[i] = atomicAdd(&tile_cursor[fr.tile_begin + (ry0 + i / rw) * fr.tiles_x + rx0 +
-                                            i % rw],
-                                v);
-    }
-    __syncthreads();
-    each_range([&](const TileRect& t, uint32_t i) {
-        for (int ty = t.ty0; ty <= t.ty1; ty++)
-            for (int tx = t.tx0; tx <= t.tx1; tx++) {
-                const uint32_t pos = atomicAdd(&lcnt[(ty - ry0) * rw + (tx - rx0)], 1u);
-                refs[pos] = slot0 + i;
+    // The union in windows of at most kLdsTiles tiles (one, but for triangles
+    // that span most of a large frame).
+    const int ww = min(rx1 - rx0 + 1, kLdsTiles), wh = min(ry1 - ry0 + 1, kLdsTiles / ww);
+    for (int wy = ry0; wy <= ry1; wy += wh)
+        for (int wx = rx0; wx <= rx1; wx += ww) {
+            const int xe = min(wx + ww - 1, rx1), ye = min(wy + wh - 1, ry1);
+            const int n = ww * (ye - wy + 1);
+            // fn(window tile, i) for every reference of record i to a tile of
+            // the window: a few tiles by the record's lane, more by the whole
+            // wave (one lane walking the 2,040 tiles of a full-screen triangle
+            // kept its workgroup 300 us after all others were done).
+            auto each_ref = [&](auto&& fn) {
+                each_range([&](const TileRect& t, uint32_t i) {
+                    const int x0 = max(t.tx0, wx), x1 = min(t.tx1, xe);
+                    const int y0 = max(t.ty0, wy), y1 = min(t.ty1, ye);
+                    const int w = max(x1 - x0 + 1, 0), m = w * max(y1 - y0 + 1, 0);
+                    constexpr int kLaneTiles = 16;
+                    if (m > 0 && m <= kLaneTiles)
+                        for (int ty = y0; ty <= y1; ty++)
+                            for (int tx = x0; tx <= x1; tx++) fn((ty - wy) * ww + tx - wx, i);
+                    for (uint64_t big = __ballot(m > kLaneTiles); big; big &= big - 1) {
+                        const int L = __builtin_ctzll(big);
+                        const uint32_t bi = (uint32_t)__builtin_amdgcn_readlane((int)i, L);
+                        wave_rect(__builtin_amdgcn_readlane(x0, L) - wx,
+                                  __builtin_amdgcn_readlane(y0, L) - wy,
+                                  __builtin_amdgcn_readlane(x1, L) - wx,
+                                  __builtin_amdgcn_readlane(y1, L) - wy, (int)threadIdx.x,
+                                  [&](int tx, int ty) { fn(ty * ww + tx, bi); });
+                    }
+                });
+            };
+            for (int k = threadIdx.x; k < n; k += kFillThreads) lcnt[k] = 0u;
+            __syncthreads();
+            each_ref([&](int t, uint32_t) { atomicAdd(&lcnt[t], 1u); });
+            __syncthreads();
+            // One global reservation per touched tile; lcnt becomes the write
+            // cursor.
+            for (int k = threadIdx.x; k < n; k += kFillThreads) {
+                const uint32_t v = lcnt[k];
+                if (v)
+                    lcnt[k] = atomicAdd(
+                        &tile_cursor[fr.tile_begin + (wy + k / ww) * fr.tiles_x + wx + k % ww], v);
             }
-    });
+            __syncthreads();
+            each_ref([&](int t, uint32_t i) { refs[atomicAdd(&lcnt[t], 1u)] = slot0 + i; });
+            __syncthreads();
+        }
 }
 
 // ---------------------------------------------------------------------------

@@ -190,6 +190,20 @@ def test_tile_counting(ctx, size, grid, eye):
         ctx.set_config(tile_w=old.tile_w, tile_h=old.tile_h)
 
 
+@pytest.mark.parametrize("size", [(8200, 16), (8192, 9), (16, 8200)])
+def test_binning_windows(ctx, size):
+    """Triangles spanning more tiles than one binning window holds, in a row of
+    1,025 tiles (two windows), of 1,024, and in a column."""
+    import scene_cases as C
+    scene = C.sphere(w=size[0], h=size[1], eye=(0, 0, 1.1), nlat=3, nlon=5)
+    old = ctx.config()
+    ctx.set_config(tile_w=8, tile_h=8)
+    try:
+        assert_same(scene, ctx.draw(scene), refcpu.draw(scene))
+    finally:
+        ctx.set_config(tile_w=old.tile_w, tile_h=old.tile_h)
+
+
 def test_decorations_batched(ctx):
     """Decorated and plain frames in one batch into shared buffers: each frame
     keeps only its own decorations, and a following draw into the same
