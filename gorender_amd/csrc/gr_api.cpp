@@ -407,16 +407,27 @@ struct Plan {
     bool raster_persistent = false;  // k_raster as a persistent grid (gr_config.raster_grid 2)
     gr::DevFrame* frames = nullptr;  // [nf], caller storage
     gr::DevObject* dobj = nullptr;   // [nobj], caller storage
-    int* xcd = nullptr;              // [8 * (nf + 1)], caller storage
+    int* xcd = nullptr;              // [table_ints(nf, nobj)], caller storage
     int face_grid = 0;
     size_t off_objs = 0, off_stats = 0, off_counters = 0, off_over = 0, off_xcd = 0;
     size_t header_bytes = 0;
 };
 
-size_t xcd_ints(int nf) { return 8 * ((size_t)nf + 1); }
+// The header's tables: XCD order [8 * (nf + 1)], first tile of each frame [nf],
+// first face block of each object [no].
+size_t table_ints(int nf, int no) { return 8 * ((size_t)nf + 1) + (size_t)nf + (size_t)no; }
+
+// Objects the frames of a batch draw in all (frames may share a range): the
+// entries make_plan fills. A range past the batch's `no` objects, which make_plan
+// refuses, counts as `no`.
+size_t drawn_objects(const gr_batch_frame* bf, int nf, int no) {
+    size_t n = 0;
+    for (int f = 0; f < nf; f++) n += (size_t)std::max(0, std::min(bf[f].num_objects, no));
+    return n;
+}
 
 // Validates the batch and fills the plan. `frames`, `dobj` and `xcd` hold at
-// least nf, no and xcd_ints(nf) entries.
+// least nf, the frames' objects and table_ints(nf, the frames' objects) entries.
 gr_status make_plan(gr_context* c, const gr_batch_frame* bf, int nf, const gr_object* objs,
                     int no, int TW, int TH, gr::DevFrame* frames, gr::DevObject* dobj, int* xcd,
                     Plan& P) {
@@ -506,7 +517,7 @@ gr_status make_plan(gr_context* c, const gr_batch_frame* bf, int nf, const gr_ob
     P.off_counters = P.off_stats + align256((size_t)nf * gr::kNumStats * 8);
     P.off_over = P.off_counters + align256(sizeof(gr::DevBatchCounters));
     P.off_xcd = P.off_over + align256((size_t)nf * 4);
-    P.header_bytes = P.off_xcd + align256(xcd_ints(nf) * sizeof(int));
+    P.header_bytes = P.off_xcd + align256(table_ints(nf, nobj) * sizeof(int));
     int nface[64];
     std::vector<int> nface_big;
     int* nfp = nface;
@@ -516,6 +527,9 @@ gr_status make_plan(gr_context* c, const gr_batch_frame* bf, int nf, const gr_ob
     }
     for (int f = 0; f < nf; f++) nfp[f] = frames[f].face_blocks;
     gr::xcd_tables(nfp, nf, xcd, &P.face_grid);
+    int* first = xcd + 8 * ((size_t)nf + 1);
+    for (int f = 0; f < nf; f++) *first++ = frames[f].tile_begin;
+    for (int k = 0; k < nobj; k++) *first++ = dobj[k].face_block;
     return GR_OK;
 }
 
@@ -578,7 +592,7 @@ void write_header(const Plan& P, const Bufs& B, void* h) {
         d.blocks = B.blocks + d.face_block_begin;
     }
     if (P.nobj) std::memcpy((char*)h + P.off_objs, P.dobj, (size_t)P.nobj * sizeof(gr::DevObject));
-    std::memcpy((char*)h + P.off_xcd, P.xcd, xcd_ints(P.nf) * sizeof(int));
+    std::memcpy((char*)h + P.off_xcd, P.xcd, table_ints(P.nf, P.nobj) * sizeof(int));
 }
 
 gr::LaunchParams launch_params(const Plan& P, const Bufs& B) {
@@ -614,6 +628,8 @@ gr::LaunchParams launch_params(const Plan& P, const Bufs& B) {
     p.counters = (gr::DevBatchCounters*)(bb + P.off_counters);
     p.ctrl = B.ctrl;
     p.xcd_face = (const int*)(bb + P.off_xcd);
+    p.tile_first = p.xcd_face + 8 * ((size_t)P.nf + 1);
+    p.obj_first = p.tile_first + P.nf;
     p.face_grid = P.face_grid;
     p.raster_persistent = P.raster_persistent ? 1 : 0;
     return p;
@@ -748,8 +764,9 @@ gr_status enqueue(gr_context* c, const gr_batch_frame* bf, int nf, const gr_obje
                   int no) {
     const int TW = c->cfg.tile_w, TH = c->cfg.tile_h;
     std::vector<gr::DevFrame> frames(std::max(nf, 1));
-    std::vector<gr::DevObject> dobj(std::max(no, 1));
-    std::vector<int> xcd(xcd_ints(std::max(nf, 1)));
+    const size_t drawn = drawn_objects(bf, nf, no);
+    std::vector<gr::DevObject> dobj(std::max<size_t>(drawn, 1));
+    std::vector<int> xcd(table_ints(std::max(nf, 1), (int)drawn));
     Plan P;
     gr_status st = make_plan(c, bf, nf, objs, no, TW, TH, frames.data(), dobj.data(), xcd.data(), P);
     if (st) return st;
@@ -1169,7 +1186,8 @@ gr_status enqueue_noalloc(gr_context* c, const gr_frame* frame, const gr_object*
         bf.d_depth = d_depth;
         gr::DevFrame frames[1];
         gr::DevObject dobj[kNoAllocMaxObjects];
-        int xcd[16];
+        int xcd[64];
+        static_assert(8 * 2 + 1 + kNoAllocMaxObjects <= 64, "the tables of one frame");
         Plan P;
         gr_status st = make_plan(c, &bf, 1, objs, no, TW, TH, frames, dobj, xcd, P);
         if (st) return st;
@@ -2005,8 +2023,9 @@ gr_status gr_batch_graph_create(gr_context* c, const gr_batch_frame* frames, int
         g->bf.assign(frames, frames + std::max(nf, 0));
         g->objs.assign(objs, objs + std::max(no, 0));
         g->frames.resize(std::max(nf, 1));
-        g->dobj.resize(std::max(no, 1));
-        g->xcd.resize(xcd_ints(std::max(nf, 1)));
+        const size_t drawn = drawn_objects(frames, nf, no);
+        g->dobj.resize(std::max<size_t>(drawn, 1));
+        g->xcd.resize(table_ints(std::max(nf, 1), (int)drawn));
         st = make_plan(c, frames, nf, objs, no, g->TW, g->TH, g->frames.data(), g->dobj.data(),
                        g->xcd.data(), g->P);
         if (!st && (hipStreamCreateWithFlags(&g->cap, hipStreamNonBlocking) != hipSuccess ||

@@ -122,12 +122,15 @@ struct DevFrame {
     const struct FaceBlock* blocks;  // the face blocks of this frame
 };
 
-// What k_face leaves of one face block: the slots it filled, its first overflow
-// record, and its counters in 16-bit fields (TPF references | binned triangles
-// << 16, front faces | clip overflows << 16).
+// What k_face leaves of one face block: the slots it filled, front faces and clip
+// overflows in the fields of c (11, 9 and 9 bits: at most kSlotsPerWg, kFacesPerWg
+// and kFacesPerWg), its first overflow record, TPF references | binned triangles
+// << 16, and its frame.
 struct alignas(16) FaceBlock {
-    uint32_t count, ovf, c0, c1;
+    uint32_t c, ovf, c0, frame;
+    __host__ __device__ uint32_t slots() const { return c & 2047u; }
 };
+static_assert(kSlotsPerWg < 2048 && kFacesPerWg < 512, "FaceBlock fields");
 
 // Per-triangle raster set-up, 80 bytes: what the visibility pass reads. The
 // four divisors and their reciprocals come first (two aligned 16-byte reads).

@@ -246,8 +246,24 @@ __host__ __device__ __forceinline__ int xcd_count(int x, int n) {
     return n > x ? (n - x + 7) >> 3 : 0;
 }
 
-template <typename F>
-__device__ __forceinline__ int last_le(int n, int b, F key);
+// Last index i in [0, n) with key[i] <= b (key[0] <= b, keys ascending), by the
+// 64 lanes of a wave at once: one round trip to memory per factor of 64, where a
+// binary search takes one per factor of 2 (9 for the 512 frames of a batch, on
+// the path of every face block and every tile).
+__device__ __forceinline__ int wave_last_le(const int* key, int n, int b) {
+    if (n == 1) return 0;
+    const int lane = (int)(threadIdx.x & 63u);
+    int lo = 0, len = n;
+    while (len > 64) {
+        const int step = (len + 63) >> 6;
+        const bool le = lane * step < len && gld(&key[lo + lane * step]) <= b;
+        const int k = __popcll(__ballot(le)) - 1;
+        lo += k * step;
+        len = min(step, len - k * step);
+    }
+    const bool le = lane < len && gld(&key[lo + lane]) <= b;
+    return lo + __popcll(__ballot(le)) - 1;
+}
 
 // Workgroup h -> (frame, unit within the frame) in the XCD-aware order: the
 // hardware places workgroup h on XCD h % 8, and XCD x takes units x, x + 8, ...
@@ -259,23 +275,9 @@ __device__ __forceinline__ bool xcd_unit(const int* table, int nframes, int h, i
     const int x = h & 7, k = h >> 3;
     const int* P = table + x * (nframes + 1);
     if (k >= P[nframes]) return false;
-    f = last_le(nframes, k, [&](int i) { return P[i]; });
+    f = wave_last_le(P, nframes, k);
     local = x + 8 * (k - P[f]);
     return true;
-}
-
-// Binary search: last index i in [0, n) with key(i) <= b.
-template <typename F>
-__device__ __forceinline__ int last_le(int n, int b, F key) {
-    int lo = 0, hi = n - 1;
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (key(mid) <= b)
-            lo = mid;
-        else
-            hi = mid - 1;
-    }
-    return lo;
 }
 
 __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v) {
@@ -938,11 +940,12 @@ __device__ __forceinline__ void wave_sync() {
 // at barriers holding registers, and every resident wave works.
 constexpr int kFacesPerLane = kFacesPerWg / 64;
 
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_face(const DevObject* __restrict__ objs, int nobj,
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_face(const DevObject* __restrict__ objs,
                                               const DevFrame* __restrict__ frames,
                                               uint32_t* __restrict__ tile_counts,
                                               FaceBlock* __restrict__ blocks, int twl,
                                               int thl, const int* __restrict__ xcd_face,
+                                              const int* __restrict__ obj_first,
                                               int nframes, uint32_t* __restrict__ rec_pool, uint32_t npools,
                                               uint32_t pool_recs, uint32_t ovf_begin,
                                               DevControl* __restrict__ ctrl,
@@ -962,14 +965,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     int bf, blocal;
     if (!xcd_unit(xcd_face, nframes, (int)blockIdx.x, bf, blocal)) return;
     const int lane = (int)threadIdx.x;
-    // Search only this frame's objects (one step for one object per frame).
+    // Search only this frame's objects.
     const int b = frames[bf].face_block_begin + blocal;
     const int ob0 = frames[bf].obj_begin;
-    const int oi =
-        ob0 + last_le(frames[bf].obj_count, b, [&](int i) { return objs[ob0 + i].face_block; });
+    const int oi = ob0 + wave_last_le(obj_first + ob0, frames[bf].obj_count, b);
     const DevObject& o = objs[oi];
     const DevMesh& m = o.m;
-    const DevFrame& fr = frames[o.frame];
+    const DevFrame& fr = frames[bf];
     lds_u32* const counters = (lds_u32*)lds_tiles;
     const TileTally tally{counters, counters + kTileTable, tile_counts, o.dense != 0};
     const int ntiles = fr.tiles_x * fr.tiles_y;
@@ -1083,7 +1085,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
             if (lane == 0) {
                 atomicMax(&ctrl->refs_needed, end * npools * kOvfRefs);
                 atomicOr(&ctrl->overflow, 1u);
-                atomicOr(&frame_overflow[o.frame], 1u);
+                atomicOr(&frame_overflow[bf], 1u);
             }
             nsurv = 0;
         } else {
@@ -1255,7 +1257,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     {
         const uint32_t c0 = wave_sum_u32((st.packed & 0xFFFFu) | (((st.packed >> 16) & 0xFFu) << 16));
         const uint32_t c1 = wave_sum_u32(((st.packed >> 24) & 0xFu) | ((st.packed >> 28) << 16));
-        if (lane == 0) gstore(&blocks[b], FaceBlock{run, ovf, c0, c1});
+        if (lane == 0)
+            gstore(&blocks[b], FaceBlock{run | (c1 & 0xFFFFu) << 11 | (c1 >> 16) << 20, ovf, c0,
+                                         (uint32_t)bf});
     }
     // Every count is in the table: flush it.
     wave_sync();
@@ -1283,24 +1287,22 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
 // k_overlay: debug overlays of every binned triangle (frames that ask for them)
 // ---------------------------------------------------------------------------
 
-__global__ __launch_bounds__(256) void k_overlay(const DevObject* __restrict__ objs, int nobj,
-                                                 const DevFrame* __restrict__ frames,
+__global__ __launch_bounds__(256) void k_overlay(const DevFrame* __restrict__ frames,
                                                  const FaceBlock* __restrict__ blocks,
                                                  unsigned long long* __restrict__ stats) {
     const int b = blockIdx.x;
-    const int oi = last_le(nobj, b, [&](int i) { return objs[i].face_block; });
-    const DevObject& o = objs[oi];
-    const DevFrame& fr = frames[o.frame];
+    const FaceBlock fb = gload(&blocks[b]);
+    const DevFrame& fr = frames[fb.frame];
     if (!fr.orec) return;
-    const uint32_t cnt = blocks[b].count, ovf = blocks[b].ovf;
-    const uint32_t blk = (uint32_t)(o.seq_block + (b - o.face_block));  // in the frame
+    const uint32_t cnt = fb.slots(), ovf = fb.ovf;
+    const uint32_t blk = (uint32_t)(b - fr.face_block_begin);  // in the frame
     const uint32_t slot0 = blk * kSlotsPerWg;
     for (uint32_t i = threadIdx.x; i < cnt; i += 256) {
         const OverlayRec rec = fr.orec[block_rec(b, ovf, i)];
         // A frame with a line too long is counted on its own, besides the
         // batch's control word, so a caller can tell which frames failed.
         if (rec.binned && !draw_overlays(fr, rec, slot0 + i))
-            atomicAdd(&stats[o.frame * kNumStats + kStatLongLines], 1ull);
+            atomicAdd(&stats[fb.frame * kNumStats + kStatLongLines], 1ull);
     }
 }
 
@@ -1442,8 +1444,8 @@ __global__ __launch_bounds__(1024) void k_bin_scan(const DevFrame* __restrict__ 
         const FaceBlock fb = gload(&blocks[fr.face_block_begin + i]);
         bs[0] += fb.c0 & 0xFFFFu;
         bs[1] += fb.c0 >> 16;
-        bs[2] += fb.c1 & 0xFFFFu;
-        bs[3] += fb.c1 >> 16;
+        bs[2] += (fb.c >> 11) & 511u;
+        bs[3] += fb.c >> 20;
     }
     local = wave_sum_u64(local);
 #pragma unroll
@@ -1525,8 +1527,7 @@ __global__ __launch_bounds__(1024) void k_bin_scan(const DevFrame* __restrict__ 
 // k_bin_fill
 // ---------------------------------------------------------------------------
 
-__global__ __launch_bounds__(kFillThreads) void k_bin_fill(const DevObject* __restrict__ objs, int nobj,
-                                                  const DevFrame* __restrict__ frames,
+__global__ __launch_bounds__(kFillThreads) void k_bin_fill(const DevFrame* __restrict__ frames,
                                                   const FaceBlock* __restrict__ blocks,
                                                   const uint32_t* __restrict__ frame_overflow,
                                                   uint32_t* __restrict__ tile_cursor,
@@ -1535,14 +1536,12 @@ __global__ __launch_bounds__(kFillThreads) void k_bin_fill(const DevObject* __re
     __shared__ uint32_t lcnt[kLdsTiles];
     __shared__ int lrect[4];
     const int b = blockIdx.x;
-    const int oi = last_le(nobj, b, [&](int i) { return objs[i].face_block; });
-    const DevObject& o = objs[oi];
-    if (frame_overflow[o.frame]) return;
-    const DevFrame& fr = frames[o.frame];
-    const uint32_t cnt = blocks[b].count, ovf = blocks[b].ovf;
-    if (cnt == 0) return;
+    const FaceBlock fb = gload(&blocks[b]);
+    const uint32_t cnt = fb.slots(), ovf = fb.ovf;
+    if (cnt == 0 || frame_overflow[fb.frame]) return;
+    const DevFrame& fr = frames[fb.frame];
     // The block's slots start at slot0; its records are block_rec(b, ovf, i).
-    const uint32_t blk = (uint32_t)(o.seq_block + (b - o.face_block));  // in the frame
+    const uint32_t blk = (uint32_t)(b - fr.face_block_begin);  // in the frame
     const uint32_t slot0 = blk * kSlotsPerWg;
     // Tile ranges of the block's first kFillKeep records stay in LDS (the records
     // are read once); later records, if any, are read again in each pass.
@@ -2130,7 +2129,8 @@ __device__ __forceinline__ unsigned long long shade_tile(const DevFrame& fr, int
 // the slab of a split tile (and clears it) and shades.
 template <int TW, int TH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_waves(TW * TH))))
-void k_raster_parts(const DevFrame* __restrict__ frames, int nframes,
+void k_raster_parts(const DevFrame* __restrict__ frames, const int* __restrict__ tile_first,
+                    int nframes,
                     const uint32_t* __restrict__ tile_counts,
                     const uint32_t* __restrict__ tile_offsets,
                     const uint32_t* __restrict__ tile_slab, const uint32_t* __restrict__ refs,
@@ -2159,7 +2159,7 @@ void k_raster_parts(const DevFrame* __restrict__ frames, int nframes,
         const int tile = sgpr((int)items[it].tile);
         const uint32_t wpart = (uint32_t)sgpr((int)items[it].part);
         if (threadIdx.x == 0) red = 0ull;  // ordered by raster_list's barriers
-        const int fi = last_le(nframes, tile, [&](int i) { return frames[i].tile_begin; });
+        const int fi = wave_last_le(tile_first, nframes, tile);
         const DevFrame& fr = frames[fi];
         const int t = tile - fr.tile_begin;
         const int X0 = (t % fr.tiles_x) * TW, Y0 = (t / fr.tiles_x) * TH;
@@ -2189,14 +2189,15 @@ void k_raster_parts(const DevFrame* __restrict__ frames, int nframes,
 // then the deferred shading. Every thread of the workgroup calls it.
 template <int TW, int TH>
 __device__ __forceinline__ void raster_tile(
-    int g, const DevFrame* __restrict__ frames, int nframes, uint32_t* __restrict__ tile_counts,
+    int g, const DevFrame* __restrict__ frames, const int* __restrict__ tile_first, int nframes,
+    uint32_t* __restrict__ tile_counts,
     const uint32_t* __restrict__ tile_offsets, const uint32_t* __restrict__ tile_slab,
     const uint32_t* __restrict__ refs, const DevTexture* __restrict__ textures,
     unsigned long long* __restrict__ stats, unsigned long long* __restrict__ slabs,
     uint32_t part_refs, unsigned long long* key, uint4* lrec, uint32_t* lslot,
     uint32_t (*qbuf)[3][128], unsigned long long (*red)[2], int lane, int wave) {
     constexpr int NPX = TW * TH;
-    const int fi = last_le(nframes, g, [&](int i) { return frames[i].tile_begin; });
+    const int fi = wave_last_le(tile_first, nframes, g);
     const DevFrame& fr = frames[fi];
     const int t = g - fr.tile_begin;
     const int X0 = (t % fr.tiles_x) * TW, Y0 = (t / fr.tiles_x) * TH;
@@ -2252,7 +2253,7 @@ __device__ __forceinline__ int xcd_tile(int h) {
 // of all XCDs; workgroups past the last tile return at once).
 template <int TW, int TH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_waves(TW * TH))))
-void k_raster(const DevFrame* __restrict__ frames, int nframes,
+void k_raster(const DevFrame* __restrict__ frames, const int* __restrict__ tile_first, int nframes,
               uint32_t* __restrict__ tile_counts, const uint32_t* __restrict__ tile_offsets,
               const uint32_t* __restrict__ tile_slab, const uint32_t* __restrict__ refs,
               const DevTexture* __restrict__ textures, unsigned long long* __restrict__ stats,
@@ -2265,7 +2266,7 @@ void k_raster(const DevFrame* __restrict__ frames, int nframes,
     __shared__ uint32_t qbuf[4][3][128];  // per-wave ring: pixel, f12, f20
     __shared__ unsigned long long red[4][2];  // per wave: covered fragments, shaded pixels
     const int lane = threadIdx.x & 63, wave = sgpr(threadIdx.x >> 6);
-    raster_tile<TW, TH>(g, frames, nframes, tile_counts, tile_offsets, tile_slab, refs, textures,
+    raster_tile<TW, TH>(g, frames, tile_first, nframes, tile_counts, tile_offsets, tile_slab, refs, textures,
                         stats, slabs, part_refs, key, lrec, lslot, qbuf, red, lane, wave);
 }
 
@@ -2273,7 +2274,8 @@ void k_raster(const DevFrame* __restrict__ frames, int nframes,
 // workgroup w draws tiles w, w + grid, w + 2 * grid, ...
 template <int TW, int TH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_waves(TW * TH))))
-void k_raster_persistent(const DevFrame* __restrict__ frames, int nframes,
+void k_raster_persistent(const DevFrame* __restrict__ frames,
+                         const int* __restrict__ tile_first, int nframes,
                          uint32_t* __restrict__ tile_counts,
                          const uint32_t* __restrict__ tile_offsets,
                          const uint32_t* __restrict__ tile_slab, const uint32_t* __restrict__ refs,
@@ -2288,7 +2290,7 @@ void k_raster_persistent(const DevFrame* __restrict__ frames, int nframes,
     __shared__ unsigned long long red[4][2];
     const int lane = threadIdx.x & 63, wave = sgpr(threadIdx.x >> 6);
     for (int g = (int)blockIdx.x; g < total_tiles; g += (int)gridDim.x) {
-        raster_tile<TW, TH>(g, frames, nframes, tile_counts, tile_offsets, tile_slab, refs,
+        raster_tile<TW, TH>(g, frames, tile_first, nframes, tile_counts, tile_offsets, tile_slab, refs,
                             textures, stats, slabs, part_refs, key, lrec, lslot, qbuf, red, lane,
                             wave);
         // red and the LDS tile state are rewritten by the next tile.
@@ -2331,9 +2333,9 @@ void launch_face_normals(const float* pos, const int32_t* vi, int F, float* fn, 
 
 void launch_face(const LaunchParams& p, hipStream_t s) {
     if (p.face_blocks == 0) return;
-    hipLaunchKernelGGL(k_face, dim3(p.face_grid), dim3(64), 0, s, p.objs, p.nobj, p.frames,
+    hipLaunchKernelGGL(k_face, dim3(p.face_grid), dim3(64), 0, s, p.objs, p.frames,
                        p.tile_counts, p.blocks, p.tw_log2, p.th_log2, p.xcd_face,
-                       p.nframes, p.rec_pool, p.rec_pools, p.pool_recs,
+                       p.obj_first, p.nframes, p.rec_pool, p.rec_pools, p.pool_recs,
                        p.ovf_begin, p.ctrl, p.frame_overflow);
 }
 
@@ -2364,7 +2366,7 @@ void launch_fog(void* rgba, const void* depth, uint64_t n, float fog_start, floa
 
 void launch_overlay(const LaunchParams& p, hipStream_t s) {
     if (p.face_blocks == 0) return;
-    hipLaunchKernelGGL(k_overlay, dim3(p.face_blocks), dim3(256), 0, s, p.objs, p.nobj, p.frames,
+    hipLaunchKernelGGL(k_overlay, dim3(p.face_blocks), dim3(256), 0, s, p.frames,
                        p.blocks, p.stats);
 }
 
@@ -2377,8 +2379,8 @@ void launch_bin_scan(const LaunchParams& p, hipStream_t s) {
 
 void launch_bin_fill(const LaunchParams& p, hipStream_t s) {
     if (p.face_blocks == 0) return;
-    hipLaunchKernelGGL(k_bin_fill, dim3(p.face_blocks), dim3(kFillThreads), 0, s, p.objs, p.nobj,
-                       p.frames, p.blocks, p.frame_overflow, p.tile_cursor, p.refs,
+    hipLaunchKernelGGL(k_bin_fill, dim3(p.face_blocks), dim3(kFillThreads), 0, s, p.frames,
+                       p.blocks, p.frame_overflow, p.tile_cursor, p.refs,
                        p.tw_log2, p.th_log2);
 }
 
@@ -2551,7 +2553,7 @@ static void raster_t(const LaunchParams& p, hipStream_t s, bool parts) {
             std::max<uint32_t>(256u, (uint32_t)p.total_tiles));
         if (grid)
             hipLaunchKernelGGL((k_raster_parts<TW, TH>), dim3(grid), dim3(256), 0, s, p.frames,
-                               p.nframes, p.tile_counts, p.tile_offsets, p.tile_slab, p.refs,
+                               p.tile_first, p.nframes, p.tile_counts, p.tile_offsets, p.tile_slab, p.refs,
                                p.stats, p.counters, p.items, p.max_items, p.slabs, p.part_refs);
         return;
     }
@@ -2559,13 +2561,13 @@ static void raster_t(const LaunchParams& p, hipStream_t s, bool parts) {
         const uint32_t grid =
             std::min<uint32_t>((uint32_t)p.total_tiles, 256u * (uint32_t)raster_waves(TW * TH));
         hipLaunchKernelGGL((k_raster_persistent<TW, TH>), dim3(grid), dim3(256), 0, s, p.frames,
-                           p.nframes, p.tile_counts, p.tile_offsets, p.tile_slab, p.refs,
+                           p.tile_first, p.nframes, p.tile_counts, p.tile_offsets, p.tile_slab, p.refs,
                            p.textures, p.stats, p.slabs, p.part_refs, p.total_tiles);
         return;
     }
     constexpr int kRound = 8 * kTileRun;
     const uint32_t grid = (uint32_t)((p.total_tiles + kRound - 1) / kRound * kRound);
-    hipLaunchKernelGGL((k_raster<TW, TH>), dim3(grid), dim3(256), 0, s, p.frames, p.nframes,
+    hipLaunchKernelGGL((k_raster<TW, TH>), dim3(grid), dim3(256), 0, s, p.frames, p.tile_first, p.nframes,
                        p.tile_counts, p.tile_offsets, p.tile_slab, p.refs, p.textures, p.stats,
                        p.slabs, p.part_refs, p.total_tiles);
 }

@@ -45,6 +45,8 @@ struct LaunchParams {
     // of frames < f that XCD x runs (blocks x, x + 8, ... of every frame); the
     // grid is 8 * the longest XCD list.
     const int* xcd_face;
+    const int* tile_first;   // [nframes]: first tile of each frame
+    const int* obj_first;    // [nobj]: first face block of each object
     int face_grid;
 };
 

@@ -204,6 +204,44 @@ def test_binning_windows(ctx, size):
         ctx.set_config(tile_w=old.tile_w, tile_h=old.tile_h)
 
 
+@pytest.mark.parametrize("objects", [63, 64, 65, 130])
+def test_many_objects(ctx, objects):
+    """Frames of up to one, and of more than one, wave's worth of objects, some
+    of several face blocks."""
+    import scene_cases as C
+    scene = C.sphere(w=120, h=90, eye=(0, 0, 3.0))
+    big = S.latlong_sphere(20, 32, S.SplitMix64(5))
+    scene.meshes.append(S.with_texture(big, 0))
+    base = scene.objects[0]
+    scene.objects = []
+    for k in range(objects):
+        world = S.world_matrix(scale=(0.2, 0.2, 0.2), rotation=(0.1 * k, 0.2 * k, 0),
+                               translation=((k % 11 - 5) * 0.2, (k // 11 - 5) * 0.2, 0.1 * (k % 3)))
+        scene.objects.append(S.ObjectData(1 if k % 5 == 0 else 0, S.mvp_matrix(
+            base.mvp, S.world_matrix(), world), world))
+    assert_same(scene, ctx.draw(scene), refcpu.draw(scene))
+
+
+def test_frames_sharing_objects(ctx):
+    """Frames of a batch that name the same range of its object array."""
+    import scene_cases as C
+    scene = C.sphere(w=96, h=64)
+    handles = ctx.upload_scene(scene)[0]
+    outs = [ctx.frame_buffers(96, 64) for _ in range(9)]
+    frames, _, objs, total = ctx.prepare_batch(
+        [scene] * 9, [handles] * 9, [(o[0].ptr, o[1].ptr) for o in outs])
+    for f in frames:
+        f.first_object = 0
+    ctx.submit_batch((frames, 9, objs, 1))
+    ctx.synchronize()
+    want = refcpu.draw(scene)
+    for rg, dp in outs:
+        assert np.array_equal(rg.to_numpy(np.uint8, (64, 96, 4)), want[0])
+        assert np.array_equal(dp.to_numpy(np.uint32, (64, 96)), want[1].view(np.uint32))
+        rg.free()
+        dp.free()
+
+
 def test_decorations_batched(ctx):
     """Decorated and plain frames in one batch into shared buffers: each frame
     keeps only its own decorations, and a following draw into the same
