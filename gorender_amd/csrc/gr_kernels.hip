@@ -295,9 +295,37 @@ __device__ __forceinline__ unsigned long long wave_total(unsigned long long v, i
     return wave_sum_u64(v);
 }
 
+// Reduction of v over the wave's 64 lanes (all active) with an associative,
+// commutative f of identity `none`, in vector instructions (data-parallel
+// primitives: shifts within rows of 16, then row broadcasts), no LDS traffic.
+// The result is wave-uniform.
+template <typename F>
+__device__ __forceinline__ uint32_t wave_reduce(uint32_t v, uint32_t none, F f) {
+#define GR_DPP(ctrl, rows) \
+    v = f(v, (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)v, ctrl, rows, 0xF, false))
+    GR_DPP(0x111, 0xF);  // row_shr:1
+    GR_DPP(0x112, 0xF);  // row_shr:2
+    GR_DPP(0x114, 0xF);  // row_shr:4
+    GR_DPP(0x118, 0xF);  // row_shr:8: lane 15 of each row holds its row
+    GR_DPP(0x142, 0xA);  // row_bcast:15 into rows 1 and 3
+    GR_DPP(0x143, 0xC);  // row_bcast:31 into rows 2 and 3
+#undef GR_DPP
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
 __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+    return wave_reduce(v, 0u, [](uint32_t a, uint32_t b) { return a + b; });
+}
+
+// Maximum of each 16-bit half, unsigned.
+__device__ __forceinline__ uint32_t max_u16x2(uint32_t a, uint32_t b) {
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t,
+                              __builtin_elementwise_max(__builtin_bit_cast(u16x2, a),
+                                                        __builtin_bit_cast(u16x2, b)));
+}
+__device__ __forceinline__ uint32_t wave_max_u16x2(uint32_t v) {
+    return wave_reduce(v, 0u, [](uint32_t a, uint32_t b) { return max_u16x2(a, b); });
 }
 
 __device__ __forceinline__ uint64_t lanemask_lt(int lane) { return (1ull << lane) - 1ull; }
@@ -1534,7 +1562,6 @@ __global__ __launch_bounds__(kFillThreads) void k_bin_fill(const DevFrame* __res
                                                   uint32_t* __restrict__ refs, int twl,
                                                   int thl) {
     __shared__ uint32_t lcnt[kLdsTiles];
-    __shared__ int lrect[4];
     const int b = blockIdx.x;
     const FaceBlock fb = gload(&blocks[b]);
     const uint32_t cnt = fb.slots(), ovf = fb.ovf;
@@ -1547,13 +1574,7 @@ __global__ __launch_bounds__(kFillThreads) void k_bin_fill(const DevFrame* __res
     // are read once); later records, if any, are read again in each pass.
     constexpr uint32_t kFillKeep = 256;
     __shared__ uint2 lrange[kFillKeep];  // tx0 | tx1 << 16, ty0 | ty1 << 16
-    if (threadIdx.x == 0) {
-        lrect[0] = 0x7FFFFFFF;
-        lrect[1] = -1;
-        lrect[2] = 0x7FFFFFFF;
-        lrect[3] = -1;
-    }
-    int ax = 0x7FFFFFFF, bx = -1, ay = 0x7FFFFFFF, by = -1;
+    uint32_t ux = 0u, uy = 0u;  // union: last + 1 | (0xFFFF - first) << 16
     for (uint32_t i = threadIdx.x; i < cnt; i += kFillThreads) {
         const uint32_t ri = block_rec(b, ovf, i);
         const TileRect t = rec_tiles(&fr.rrec[ri], twl, thl);
@@ -1561,10 +1582,8 @@ __global__ __launch_bounds__(kFillThreads) void k_bin_fill(const DevFrame* __res
             lrange[i] = make_uint2((uint32_t)t.tx0 | (uint32_t)t.tx1 << 16,
                                    (uint32_t)t.ty0 | (uint32_t)t.ty1 << 16);
         if (t.tx0 > t.tx1) continue;
-        ax = min(ax, t.tx0);
-        bx = max(bx, t.tx1);
-        ay = min(ay, t.ty0);
-        by = max(by, t.ty1);
+        ux = max_u16x2(ux, (uint32_t)(t.tx1 + 1) | (uint32_t)(0xFFFF - t.tx0) << 16);
+        uy = max_u16x2(uy, (uint32_t)(t.ty1 + 1) | (uint32_t)(0xFFFF - t.ty0) << 16);
     }
     // fn(t, i) for the tile range of every record i, 64 records at a time by all
     // lanes of the wave (empty past the last record).
@@ -1584,16 +1603,13 @@ __global__ __launch_bounds__(kFillThreads) void k_bin_fill(const DevFrame* __res
             fn(t, i);
         }
     };
-    // The union of the ranges, by LDS atomics.
-    __syncthreads();
-    if (bx >= 0) {
-        atomicMin(&lrect[0], ax);
-        atomicMax(&lrect[1], bx);
-        atomicMin(&lrect[2], ay);
-        atomicMax(&lrect[3], by);
-    }
-    __syncthreads();
-    const int rx0 = lrect[0], rx1 = lrect[1], ry0 = lrect[2], ry1 = lrect[3];
+    // The union of the ranges, in vector instructions (LDS minima and maxima of
+    // one address by 64 lanes take the lanes one by one: 8 of the 20 us of a
+    // block with many triangles).
+    ux = wave_max_u16x2(ux);
+    uy = wave_max_u16x2(uy);
+    const int rx0 = 0xFFFF - (int)(ux >> 16), rx1 = (int)(ux & 0xFFFFu) - 1;
+    const int ry0 = 0xFFFF - (int)(uy >> 16), ry1 = (int)(uy & 0xFFFFu) - 1;
     if (rx1 < 0) return;
     // The union in windows of at most kLdsTiles tiles (one, but for triangles
     // that span most of a large frame).
