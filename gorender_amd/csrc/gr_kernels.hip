@@ -961,30 +961,38 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// One face block (kFacesPerWg faces of one object) per single-wave workgroup,
-// kFacesPerLane faces per lane. A block's few survivors keep one wave busy
-// through the long per-survivor chain of pass 2 (dependent loads, lighting,
-// clipping, set-up), so the workgroup is that one wave: no sibling waves wait
-// at barriers holding registers, and every resident wave works.
-constexpr int kFacesPerLane = kFacesPerWg / 64;
+// One face block (kFacesPerWg faces of one object) per workgroup of NW waves.
+//
+// NW = 1, kFacesPerLane faces per lane: a block's few survivors keep one wave
+// busy through the long per-survivor chain of pass 2 (dependent loads, lighting,
+// clipping, set-up), so no sibling waves wait at barriers holding registers, and
+// every resident wave works. The form for launches that fill the chip.
+//
+// NW = 4, a face per lane: pass 1 is a quarter as long and pass 2 one round
+// instead of up to four, for launches whose blocks leave most of the chip idle
+// (see launch_face).
+__device__ __forceinline__ int sgpr(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_face(const DevObject* __restrict__ objs,
-                                              const DevFrame* __restrict__ frames,
-                                              uint32_t* __restrict__ tile_counts,
-                                              FaceBlock* __restrict__ blocks, int twl,
-                                              int thl, const int* __restrict__ xcd_face,
-                                              const int* __restrict__ obj_first,
-                                              int nframes, uint32_t* __restrict__ rec_pool, uint32_t npools,
-                                              uint32_t pool_recs, uint32_t ovf_begin,
-                                              DevControl* __restrict__ ctrl,
-                                              uint32_t* __restrict__ frame_overflow) {
-    static_assert(kFacesPerWg == 64 * kFacesPerLane, "whole faces per lane");
-    // Survivors in face order: face offset | first clip plane << 8.
-    __shared__ uint32_t lds_sface[kFacesPerWg];
-    __shared__ CV wpoly[2][kMaxClip];
-    __shared__ CV lds_stage[kStage][kMaxClip];  // clipped polygons of general faces
-    __shared__ int lds_stage_k[kStage], lds_stage_tex[kStage];
-    __shared__ int lds_stage_off[kStage];  // the face's first offset in the block
+template <int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) void k_face(
+    const DevObject* __restrict__ objs, const DevFrame* __restrict__ frames,
+    uint32_t* __restrict__ tile_counts, FaceBlock* __restrict__ blocks, int twl, int thl,
+    const int* __restrict__ xcd_face, const int* __restrict__ obj_first, int nframes,
+    uint32_t* __restrict__ rec_pool, uint32_t npools, uint32_t pool_recs, uint32_t ovf_begin,
+    DevControl* __restrict__ ctrl, uint32_t* __restrict__ frame_overflow) {
+    constexpr int kFacesPerLane = kFacesPerWg / (64 * NW);
+    static_assert(kFacesPerWg == 64 * NW * kFacesPerLane, "whole faces per lane");
+    // What a wave keeps to itself.
+    struct WaveLds {
+        uint32_t sface[64 * kFacesPerLane];  // survivors in face order: offset | clip plane << 8
+        CV poly[2][kMaxClip];
+        CV stage[kStage][kMaxClip];          // clipped polygons of general faces
+        int stage_k[kStage], stage_tex[kStage];
+        int stage_off[kStage];               // the face's first offset in the block
+    };
+    __shared__ WaveLds lds_wave[NW];
+    __shared__ uint32_t lds_sum[4][NW];  // per-wave terms of the block's sums
+    __shared__ uint32_t lds_claim[2];    // the block's claim of overflow records
     // The tile counters (see kTableTiles): 16 bits a tile, or the entry table.
     // A block counts at most kSlotsPerWg references per tile.
     __shared__ uint4 lds_tiles[kTableTiles / 8];
@@ -992,7 +1000,30 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
 
     int bf, blocal;
     if (!xcd_unit(xcd_face, nframes, (int)blockIdx.x, bf, blocal)) return;
-    const int lane = (int)threadIdx.x;
+    const int lane = (int)threadIdx.x & 63, wave = NW > 1 ? sgpr((int)threadIdx.x >> 6) : 0;
+    WaveLds& W = lds_wave[wave];
+    auto block_sync = [&] {
+        if constexpr (NW > 1)
+            __syncthreads();
+        else
+            wave_sync();
+    };
+    // Sum of the waves' v (wave-uniform) before this one's; all of them in total.
+    // Each k is used once.
+    auto wave_prefix = [&](int k, uint32_t v, uint32_t& total) -> uint32_t {
+        total = v;
+        if constexpr (NW == 1) return 0u;
+        if (lane == 0) lds_sum[k][wave] = v;
+        __syncthreads();
+        uint32_t before = 0u;
+        total = 0u;
+        for (int w = 0; w < NW; w++) {
+            const uint32_t t = (uint32_t)sgpr((int)lds_sum[k][w]);
+            before += w < wave ? t : 0u;
+            total += t;
+        }
+        return before;
+    };
     // Search only this frame's objects.
     const int b = frames[bf].face_block_begin + blocal;
     const int ob0 = frames[bf].obj_begin;
@@ -1005,11 +1036,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     const int ntiles = fr.tiles_x * fr.tiles_y;
     const bool table = ntiles <= kTableTiles;  // wave-uniform
     const int groups = table ? (ntiles + 7) >> 3 : 2 * kTileTable / 4;  // uint4 pieces in use
-    for (int i = lane; i < groups; i += 64) {
+    for (int i = (int)threadIdx.x; i < groups; i += 64 * NW) {
         const uint32_t v = !table && i < kTileTable / 4 ? kNoTile : 0u;
         lds_tiles[i] = make_uint4(v, v, v, v);
     }
-    wave_sync();
+    block_sync();
     // Counts the tiles of the lanes' boxes; every lane of the wave calls it. A box
     // of many tiles is counted by the whole wave.
     auto count = [&](const uint2& box) {
@@ -1050,7 +1081,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
         // All the lane's vertex indices, then all its corners, are loaded
         // before any is used: lanes past the mesh's last face read its last
         // face (in bounds) and are not counted.
-        const int face0 = wg_in_obj * kFacesPerWg + lane;
+        const int fo0 = wave * 64 * kFacesPerLane + lane;  // the lane's first face of the block
+        const int face0 = wg_in_obj * kFacesPerWg + fo0;
         int iv[kFacesPerLane][3];
 #pragma unroll
         for (int k = 0; k < kFacesPerLane; k++) {
@@ -1066,7 +1098,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
             for (int c = 0; c < 3; c++) cv[k][c] = corner(o, iv[k][c]);
 #pragma unroll
         for (int k = 0; k < kFacesPerLane; k++) {
-            const int fo = k * 64 + lane;  // face offset in the block
+            const int fo = k * 64 + fo0;  // face offset in the block
             const float4 v0 = cv[k][0], v1 = cv[k][1], v2 = cv[k][2];
             bool survivor = false;
             int p = 6;
@@ -1088,7 +1120,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
             }
             const uint64_t sm = __ballot(survivor);
             if (survivor)
-                lds_sface[nsurv + __popcll(sm & lanemask_lt(lane))] = (uint32_t)fo | ((uint32_t)p << 8);
+                W.sface[nsurv + __popcll(sm & lanemask_lt(lane))] = (uint32_t)fo | ((uint32_t)p << 8);
             nsurv += __popcll(sm);
             nrec += (uint32_t)__popcll(sm) + (kMaxFan - 1) * (uint32_t)__popcll(__ballot(survivor && p < 6));
         }
@@ -1101,24 +1133,28 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     // overflow with a capacity that gives every pool this much (the caller
     // grows the capacity and draws it again); its frame is marked so that its
     // raster draws the background only.
-    uint32_t ovf = 0u;  // wave-uniform
-    if (nsurv > 0 && nrec > (uint32_t)kRecsPerBlock) {
-        const uint32_t extra = nrec - (uint32_t)kRecsPerBlock;
+    uint32_t ovf = 0u;  // block-uniform
+    uint32_t nrec_block;
+    (void)wave_prefix(0, nrec, nrec_block);
+    if (nrec_block > (uint32_t)kRecsPerBlock) {
+        const uint32_t extra = nrec_block - (uint32_t)kRecsPerBlock;
         const uint32_t pool = (uint32_t)b % npools;
-        uint32_t r = 0u;
-        if (lane == 0) r = atomicAdd(&rec_pool[pool * kPoolStride], extra);
-        r = (uint32_t)__builtin_amdgcn_readfirstlane((int)r);
-        const unsigned long long end = (unsigned long long)r + extra;
-        if (end > pool_recs) {
-            if (lane == 0) {
+        if (threadIdx.x == 0) {
+            const uint32_t r = atomicAdd(&rec_pool[pool * kPoolStride], extra);
+            const unsigned long long end = (unsigned long long)r + extra;
+            lds_claim[0] = r;
+            lds_claim[1] = end > pool_recs;
+            if (end > pool_recs) {
                 atomicMax(&ctrl->refs_needed, end * npools * kOvfRefs);
                 atomicOr(&ctrl->overflow, 1u);
                 atomicOr(&frame_overflow[bf], 1u);
             }
-            nsurv = 0;
-        } else {
-            ovf = ovf_begin + pool * pool_recs + r;
         }
+        block_sync();
+        if (sgpr((int)lds_claim[1]))
+            nsurv = 0;
+        else
+            ovf = ovf_begin + pool * pool_recs + (uint32_t)sgpr((int)lds_claim[0]);
     }
 
     // Pass 2, survivor r0 + lane, 64 a round: lighting, texture coordinates,
@@ -1126,8 +1162,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     // wave, 3: one-plane polygon. q[0..nq-1] holds the polygon to emit (the
     // triangle itself for modes 1 and 2), so only one set of corners stays
     // live across the emits.
-    uint32_t run = 0;  // slots of the earlier rounds (wave-uniform)
-    for (int r0 = 0; r0 < nsurv; r0 += 64) {
+    uint32_t run = 0;  // slots of the earlier rounds, or of the block (wave-uniform)
+    for (int r0 = 0; r0 < (NW > 1 ? 1 : nsurv); r0 += 64) {
         int mode = 0;
         int n = 0;
         CV q[4];
@@ -1135,7 +1171,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
         int tex = -1;
         if (r0 + lane < nsurv) {
             CV c0, c1, c2;
-            const uint32_t e = lds_sface[r0 + lane];
+            const uint32_t e = W.sface[r0 + lane];
             const int sf = wg_in_obj * kFacesPerWg + (int)(e & 0xFFu);
             const int sp = (int)(e >> 8);
             const int i0 = gld(&m.vi[3 * sf + 0]), i1 = gld(&m.vi[3 * sf + 1]),
@@ -1218,9 +1254,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
         const uint64_t b1 = __ballot(n == 1), b2 = __ballot(n == 2), b7 = __ballot(n == kMaxFan);
         const uint64_t lt = lanemask_lt(lane);
         // The lane's slots start at offset off of the block's.
-        const uint32_t off = run + (uint32_t)(__popcll(b1 & lt) + 2 * __popcll(b2 & lt) +
-                                              kMaxFan * __popcll(b7 & lt));
-        run += (uint32_t)(__popcll(b1) + 2 * __popcll(b2) + kMaxFan * __popcll(b7));
+        uint32_t total;
+        const uint32_t before = wave_prefix(
+            1, (uint32_t)(__popcll(b1) + 2 * __popcll(b2) + kMaxFan * __popcll(b7)), total);
+        const uint32_t off = run + before + (uint32_t)(__popcll(b1 & lt) + 2 * __popcll(b2 & lt) +
+                                                       kMaxFan * __popcll(b7 & lt));
+        run += total;
         // Fan of q (Polygon.Triangulate, clipping.go:44-62): (P0, P1, P2),
         // then (P0, P2, P3) for a quad.
         {
@@ -1241,8 +1280,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
         // stage (clipping.go:167-236), then one lane per fan slot emits the
         // triangle (P0, P_t+1, P_t+2) of Polygon.Triangulate
         // (clipping.go:44-62) or an empty record.
-        CV* buf0 = wpoly[0];
-        CV* buf1 = wpoly[1];
+        CV* buf0 = W.poly[0];
+        CV* buf1 = W.poly[1];
         for (uint64_t gen = __ballot(mode == 2); gen;) {
             int nst = 0;
             for (; gen && nst < kStage; gen &= gen - 1, nst++) {
@@ -1252,22 +1291,22 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
                 const int sL = __shfl((int)off, L, 64);
                 const int k = wave_clip(buf0, buf1, a, bb, c, fr.znear, fr.zfar, lane);
                 if (k < 0 && lane == L) st.packed += 1u << 28;
-                if (lane < k) lds_stage[nst][lane] = buf0[lane];
+                if (lane < k) W.stage[nst][lane] = buf0[lane];
                 if (lane == 0) {
-                    lds_stage_k[nst] = k;
-                    lds_stage_tex[nst] = texL;
-                    lds_stage_off[nst] = sL;
+                    W.stage_k[nst] = k;
+                    W.stage_tex[nst] = texL;
+                    W.stage_off[nst] = sL;
                 }
                 wave_sync();
             }
             const int r = lane / kMaxFan, t = lane - r * kMaxFan;
             uint2 box = make_uint2(kEmptyBox, 0u);
             if (r < nst) {
-                const int k = lds_stage_k[r];
-                const uint32_t ri = block_rec(b, ovf, (uint32_t)lds_stage_off[r] + (uint32_t)t);
-                const CV* P = lds_stage[r];
+                const int k = W.stage_k[r];
+                const uint32_t ri = block_rec(b, ovf, (uint32_t)W.stage_off[r] + (uint32_t)t);
+                const CV* P = W.stage[r];
                 if (t < k - 2)
-                    add_emit(st, emit_triangle(fr, P[0], P[t + 1], P[t + 2], lds_stage_tex[r],
+                    add_emit(st, emit_triangle(fr, P[0], P[t + 1], P[t + 2], W.stage_tex[r],
                                                ri, box));
                 else
                     empty_record(fr, ri);
@@ -1283,22 +1322,25 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
     // (Added to the frame's counters, one cache line, the blocks queue up: 47 us
     // for the 3,900 blocks of a million faces.)
     {
-        const uint32_t c0 = wave_sum_u32((st.packed & 0xFFFFu) | (((st.packed >> 16) & 0xFFu) << 16));
-        const uint32_t c1 = wave_sum_u32(((st.packed >> 24) & 0xFu) | ((st.packed >> 28) << 16));
-        if (lane == 0)
+        const uint32_t w0 = wave_sum_u32((st.packed & 0xFFFFu) | (((st.packed >> 16) & 0xFFu) << 16));
+        const uint32_t w1 = wave_sum_u32(((st.packed >> 24) & 0xFu) | ((st.packed >> 28) << 16));
+        uint32_t c0, c1;
+        (void)wave_prefix(2, w0, c0);
+        (void)wave_prefix(3, w1, c1);
+        if (threadIdx.x == 0)
             gstore(&blocks[b], FaceBlock{run | (c1 & 0xFFFFu) << 11 | (c1 >> 16) << 20, ovf, c0,
                                          (uint32_t)bf});
     }
-    // Every count is in the table: flush it.
+    // Every count is in the table (the sums' barriers order the waves): flush it.
     wave_sync();
     if (!table) {
-        for (int i = lane; i < kTileTable; i += 64) {
+        for (int i = (int)threadIdx.x; i < kTileTable; i += 64 * NW) {
             const uint32_t v = counters[kTileTable + i];
             if (v) atomicAdd(&tile_counts[counters[i]], v);
         }
         return;
     }
-    for (int i = lane; i < groups; i += 64) {
+    for (int i = (int)threadIdx.x; i < groups; i += 64 * NW) {
         const uint4 v = lds_tiles[i];
         if (!(v.x | v.y | v.z | v.w)) continue;
         uint32_t* dst = tile_counts + fr.tile_begin + 8 * i;
@@ -1765,9 +1807,6 @@ __device__ __forceinline__ uint32_t color_intensity(uint32_t c, float k) {
     uint32_t b = go_uint8((float)((c >> 16) & 0xFFu) * k);
     return r | (g << 8) | (b << 16) | (c & 0xFF000000u);
 }
-
-__device__ __forceinline__ int sgpr(int v) { return __builtin_amdgcn_readfirstlane(v); }
-
 
 // The raster stage reads a staged RasterRec as five 16-byte pieces: divisors,
 // reciprocals, then (box x, box y, wide, A01), (B01, C01, A12, B12),
@@ -2347,12 +2386,24 @@ void launch_face_normals(const float* pos, const int32_t* vi, int F, float* fn, 
     hipLaunchKernelGGL(k_face_normals, dim3((F + 255) / 256), dim3(256), 0, s, pos, vi, F, fn);
 }
 
+constexpr int kWideFaceBlocks = 4096;
 void launch_face(const LaunchParams& p, hipStream_t s) {
     if (p.face_blocks == 0) return;
-    hipLaunchKernelGGL(k_face, dim3(p.face_grid), dim3(64), 0, s, p.objs, p.frames,
-                       p.tile_counts, p.blocks, p.tw_log2, p.th_log2, p.xcd_face,
-                       p.obj_first, p.nframes, p.rec_pool, p.rec_pools, p.pool_recs,
-                       p.ovf_begin, p.ctrl, p.frame_overflow);
+    // Four waves a block for launches that leave the chip part idle, one past
+    // that, whose waves do not wait for each other. The chip holds 4,096 waves (4
+    // on each of 1,024 SIMDs). us with one | four waves: 2 blocks 27.5 | 19.6,
+    // 20 18.8 | 12.1, 157 29.5 | 18.8, 782 33.7 | 30.6, 4,000 57 | 50, 20,000
+    // 254 | 262, 25,000 119 | 266, 38,000 279 | 458.
+    auto launch = [&](auto kernel, int threads) {
+        hipLaunchKernelGGL(kernel, dim3(p.face_grid), dim3(threads), 0, s, p.objs, p.frames,
+                           p.tile_counts, p.blocks, p.tw_log2, p.th_log2, p.xcd_face,
+                           p.obj_first, p.nframes, p.rec_pool, p.rec_pools, p.pool_recs,
+                           p.ovf_begin, p.ctrl, p.frame_overflow);
+    };
+    if (p.face_blocks <= kWideFaceBlocks)
+        launch(k_face<4>, 256);
+    else
+        launch(k_face<1>, 64);
 }
 
 void xcd_tables(const int* n, int nframes, int* table, int* grid) {

@@ -222,6 +222,38 @@ def test_many_objects(ctx, objects):
     assert_same(scene, ctx.draw(scene), refcpu.draw(scene))
 
 
+def test_face_stage_forms(ctx):
+    """The same frames alone (face blocks of four waves) and in a batch of over
+    4,096 face blocks (of one wave): survivors on every wave, blocks of broken
+    length, faces for the full clipper past a block's own records."""
+    import scene_cases as C
+    cases = [C.clip_space_soup(n=700, seed=31), C.inside_sphere(), C.cube_scene(),
+             C.sphere(w=200, h=120, eye=(0, 0, 1.4), nlat=23, nlon=37),
+             C.sphere(w=90, h=70, flags=C.no(_lib.GR_BACKFACE_CULLING), nlat=16, nlon=24)]
+    # A million faces out of view: blocks that emit nothing.
+    pad = C.sphere(w=16, h=16, nlat=600, nlon=900)
+    pad.objects = [S.camera_object(pad.frame, 0, (100.0, 0, 0), (1, 0, 0))]
+    frames = cases + [pad]
+    handles = [ctx.upload_scene(s)[0] for s in frames]
+    outs = [ctx.frame_buffers(s.frame.width, s.frame.height) for s in frames]
+    ctx.draw_batch(frames, handles, [(o[0].ptr, o[1].ptr) for o in outs])
+    ctx.synchronize()
+    stats = ctx.last_stats()
+    for k, s in enumerate(cases):
+        want = refcpu.draw(s)
+        assert_same(s, ctx.draw(s, handles[k]), want)
+        h, w = s.frame.height, s.frame.width
+        got = (outs[k][0].to_numpy(np.uint8, (h, w, 4)), outs[k][1].to_numpy(np.float32, (h, w)),
+               stats[k])
+        assert_same(s, got, want)
+    for rg, dp in outs:
+        rg.free()
+        dp.free()
+    for hs in handles:
+        for h in hs:
+            ctx.destroy_mesh(h)
+
+
 def test_frames_sharing_objects(ctx):
     """Frames of a batch that name the same range of its object array."""
     import scene_cases as C
