@@ -466,8 +466,20 @@ gr_status make_plan(gr_context* c, const gr_batch_frame* bf, int nf, const gr_ob
         d.clear_color = pack_rgba(fr.clear_color);
         d.dot_color = pack_rgba(fr.dot_color);
         d.dot_step = fr.dot_step;
-        for (int t = 0; t < fr.ref_tiles; t++)
-            ref_tile_bounds(t, fr.ref_tiles, fr.width, fr.height, d.ref_tile_rect[t]);
+        // The grid is a product: x bounds from tile % n, y bounds from tile / n.
+        const int ng = fr.ref_tiles == 16 ? 4 : 1;
+        for (int g = 0; g < 4; g++) {
+            const float none = std::nanf("");
+            float col[4] = {none, none, none, none}, row[4] = {none, none, none, none};
+            if (g < ng) {
+                ref_tile_bounds(g, fr.ref_tiles, fr.width, fr.height, col);
+                ref_tile_bounds(g * ng, fr.ref_tiles, fr.width, fr.height, row);
+            }
+            d.ref_cols[g][0] = col[0];
+            d.ref_cols[g][1] = col[2];
+            d.ref_rows[g][0] = row[1];
+            d.ref_rows[g][1] = row[3];
+        }
         d.tiles_x = (fr.width + TW - 1) / TW;
         d.tiles_y = (fr.height + TH - 1) / TH;
         d.tile_begin = P.tiles;

@@ -100,7 +100,9 @@ struct DevFrame {
     float ambient, diffuse, znear, zfar;
     uint32_t face_color, clear_color, dot_color;
     int32_t dot_step;
-    float ref_tile_rect[16][4];  // reference TPF grid (renderer.go:50-76)
+    // Reference TPF grid (renderer.go:50-76): first and last x of its columns, y of
+    // its rows; NaN past a 1x1 grid's first.
+    float ref_cols[4][2], ref_rows[4][2];
     int32_t tiles_x, tiles_y;    // raster tiles of this frame
     int32_t tile_begin;          // first tile in the batch tile arrays
     int32_t face_block_begin;    // first k_face block of this frame

@@ -495,6 +495,9 @@ struct FaceStats {
     uint32_t packed;
 };
 
+// Box words of a record that is not rasterised: first 1, last 0.
+constexpr uint32_t kEmptyBox = 1u;
+
 // ---------------------------------------------------------------------------
 // Debug overlays (renderer.go:191-216): lines and 3x3 rects write colour only,
 // after their triangle's face, in draw order. Each overlay pixel keeps the max
@@ -627,65 +630,69 @@ __device__ __forceinline__ void count_tiles(const DevFrame& fr, const TileTally&
         }
 }
 
+// A record that is never rasterised: its box words, all that is read of it.
+__device__ __forceinline__ void store_empty_box(const DevFrame& fr, uint32_t ri) {
+    gstore(reinterpret_cast<uint4*>(&fr.rrec[ri]) + 2, make_uint4(kEmptyBox, kEmptyBox, 0u, 0u));
+}
+
 // Writes the set-up of one post-clip triangle into record ri (renderer.go:361-394
 // then the per-triangle part of rasterizer.go:98-137). Returns the TPF
 // references in the low 16 bits and 1 << 16 when the triangle was binned, and the
 // record's box words (bx0 | bx1 << 16, by0 | by1 << 16).
-__device__ uint32_t emit_triangle(const DevFrame& fr, const CV& a, const CV& b, const CV& c,
-                                  int tex, uint32_t ri, uint2& box) {
-    uint32_t tpf = 0, tris = 0;
-    const CV vv[3] = {a, b, c};
-    float sx[3], sy[3], zw[3];
+//
+// k_face is bound by the instructions it issues, and most of them are here. The
+// common triangle (screen coordinates within +-16384) takes 32-bit integers, a
+// reference grid read at once, and one branch for what is rare in its three
+// vertices; with 64-bit coordinates, a loop over the grid and Go's NaN and
+// signed-zero rules worked out per minimum, 64 of them took 3.5 us (k_face for 32
+// frames of 200,000 triangles 120 -> 106 us, for one of 40,000 18.8 -> 15.1).
+__device__ __forceinline__ uint32_t emit_triangle(const DevFrame& fr, const CV& a, const CV& b,
+                                                  const CV& c, int tex, uint32_t ri, uint2& box) {
+    const float zw[3] = {a.w, b.w, c.w}, zz[3] = {a.z, b.z, c.z};
+    const float vx[3] = {a.x, b.x, c.x}, vy[3] = {a.y, b.y, c.y};
+    float sx[3], sy[3], pz[3] = {0.f, 0.f, 0.f};
     // The screen x and y rows use z/w only through screen[2] and screen[6]: when
     // both are zero, z/w matters only by being infinite or NaN (0 * z/w), and the
     // sign of a zero term never changes what the rasteriser does with sx, sy
     // (int(), comparisons). w/w is 1 for finite nonzero w, else NaN.
-    const bool zcol = fr.screen[2] != 0.f || fr.screen[6] != 0.f;
+    bool need_z = fr.screen[2] != 0.f || fr.screen[6] != 0.f;
+#pragma unroll
+    for (int j = 0; j < 3; j++)
+        need_z = need_z || !(__builtin_isfinite(zz[j]) &&
+                             __builtin_fabsf(zz[j]) < __builtin_fabsf(zw[j]) * 0x1p100f);
+    if (need_z) {
+#pragma unroll
+        for (int j = 0; j < 3; j++) pz[j] = zz[j] / zw[j];
+    }
 #pragma unroll
     for (int j = 0; j < 3; j++) {
-        const float w = vv[j].w, z = vv[j].z;
-        const float px = vv[j].x / w, py = vv[j].y / w;
-        const bool wok = __builtin_isfinite(w) && w != 0.f;
-        const float pw = wok ? 1.0f : __builtin_nanf("");
-        float pz = 0.0f;
-        if (zcol || !(__builtin_isfinite(z) && __builtin_fabsf(z) < __builtin_fabsf(w) * 0x1p100f))
-            pz = z / w;
-        sx[j] = fr.screen[0] * px + fr.screen[1] * py + fr.screen[2] * pz + fr.screen[3] * pw;
-        sy[j] = fr.screen[4] * px + fr.screen[5] * py + fr.screen[6] * pz + fr.screen[7] * pw;
-        zw[j] = w;
+        const float w = zw[j];
+        const float px = vx[j] / w, py = vy[j] / w;
+        const float pw = __builtin_isfinite(w) && w != 0.f ? 1.0f : __builtin_nanf("");
+        sx[j] = fr.screen[0] * px + fr.screen[1] * py + fr.screen[2] * pz[j] + fr.screen[3] * pw;
+        sy[j] = fr.screen[4] * px + fr.screen[5] * py + fr.screen[6] * pz[j] + fr.screen[7] * pw;
     }
-    float fminx = go_min(go_min(sx[0], sx[1]), sx[2]);
-    float fmaxx = go_max(go_max(sx[0], sx[1]), sx[2]);
-    float fminy = go_min(go_min(sy[0], sy[1]), sy[2]);
-    float fmaxy = go_max(go_max(sy[0], sy[1]), sy[2]);
+    // Go's min and max of the three: only compared below, where the sign of a
+    // zero does not matter and a NaN (which wins in Go) fails every comparison.
+    const bool okx = !(sx[0] != sx[0]) && !(sx[1] != sx[1]) && !(sx[2] != sx[2]);
+    const bool oky = !(sy[0] != sy[0]) && !(sy[1] != sy[1]) && !(sy[2] != sy[2]);
+    const float fminx = __builtin_fminf(__builtin_fminf(sx[0], sx[1]), sx[2]);
+    const float fmaxx = __builtin_fmaxf(__builtin_fmaxf(sx[0], sx[1]), sx[2]);
+    const float fminy = __builtin_fminf(__builtin_fminf(sy[0], sy[1]), sy[2]);
+    const float fmaxy = __builtin_fmaxf(__builtin_fmaxf(sy[0], sy[1]), sy[2]);
     // renderer.go:226-244 against the reference TPF grid. Its tiles are a
     // product grid (x bounds from tile % n, y bounds from tile / n,
     // renderer.go:61-67), so the overlapping tiles are the overlapping columns
-    // times the overlapping rows.
-    {
-        const int ng = fr.ref_tiles == 16 ? 4 : 1;
-        uint32_t cols = 0, rows = 0;
-        for (int c = 0; c < ng; c++) {
-            const float* rx = fr.ref_tile_rect[c];
-            const float* ry = fr.ref_tile_rect[c * ng];
-            cols += (uint32_t)(fmaxx >= rx[0] && fminx <= rx[2]);
-            rows += (uint32_t)(fmaxy >= ry[1] && fminy <= ry[3]);
-        }
-        tpf = cols * rows;
-    }
-    RasterRec rr;
-    rr.bx0 = 1;
-    rr.bx1 = 0;
-    rr.by0 = 1;
-    rr.by1 = 0;
-    rr.wide = 0;
-    rr.sf = 0.f;
-    rr.z0 = rr.z1 = rr.z2 = 0.f;
-    rr.rsf = rr.rz0 = rr.rz1 = rr.rz2 = 0.f;
+    // times the overlapping rows (the bounds past a smaller grid are NaN).
+    uint32_t cols = 0, rows = 0;
 #pragma unroll
-    for (int e = 0; e < 9; e++) rr.e[e] = 0;
-    float W = (float)fr.W, H = (float)fr.H;
-    bool binned = fmaxx >= 0.f && fminx <= W && fmaxy >= 0.f && fminy <= H;
+    for (int g = 0; g < 4; g++) {
+        cols += (uint32_t)(fmaxx >= fr.ref_cols[g][0] && fminx <= fr.ref_cols[g][1]);
+        rows += (uint32_t)(fmaxy >= fr.ref_rows[g][0] && fminy <= fr.ref_rows[g][1]);
+    }
+    const uint32_t tpf = okx && oky ? cols * rows : 0u;
+    const bool binned = okx && oky && fmaxx >= 0.f && fminx <= (float)fr.W && fmaxy >= 0.f &&
+                        fminy <= (float)fr.H;
     if (fr.orec) {
         // Screen positions for the overlay pass (binned triangles only draw them).
         OverlayRec o;
@@ -698,165 +705,159 @@ __device__ uint32_t emit_triangle(const DevFrame& fr, const CV& a, const CV& b, 
         o.pad = 0;
         gstore(&fr.orec[ri], o);
     }
-    if (binned) {
-        tris = 1;
-        int64_t ix[3], iy[3];
+    box = make_uint2(kEmptyBox, kEmptyBox);
+    if (binned && (fr.flags & kShowFaces)) {
+        RasterRec rr;
+        // Edge functions f_e(x,y) = A*x + B*y + C (rasterizer.go:107-117) with the
+        // top-left adjustment folded into C (rasterizer.go:120-129). The pixel
+        // sum fx12 + fx20 + fx01 is the sum of the C's (the A and B terms
+        // cancel).
+        constexpr int i0[3] = {0, 1, 2}, i1[3] = {1, 2, 0};
+        int x0, x1, y0, y1;  // rasterizer.go:99-104 with tile (0,0)-(W,H) of the sequential renderer
+        const float far = __builtin_fmaxf(
+            __builtin_fmaxf(__builtin_fabsf(fminx), __builtin_fabsf(fmaxx)),
+            __builtin_fmaxf(__builtin_fabsf(fminy), __builtin_fabsf(fmaxy)));
+        const bool fast = far < (float)(kFastCoord + 1);
+        if (fast) {
+            // |x|, |y| <= 2^14: 24-bit products, and every value (the sum of
+            // the three C's included) fits int32.
+            int32_t X[3], Y[3], csum = 0;
 #pragma unroll
-        for (int j = 0; j < 3; j++) {
-            ix[j] = go_int(sx[j]);
-            iy[j] = go_int(sy[j]);
+            for (int j = 0; j < 3; j++) {
+                X[j] = (int32_t)sx[j];
+                Y[j] = (int32_t)sy[j];
+            }
+            x0 = max(min(min(X[0], X[1]), X[2]), 0);
+            x1 = min(max(max(X[0], X[1]), X[2]), fr.W - 1);
+            y0 = max(min(min(Y[0], Y[1]), Y[2]), 0);
+            y1 = min(max(max(Y[0], Y[1]), Y[2]), fr.H - 1);
+#pragma unroll
+            for (int e = 0; e < 3; e++) {
+                const int p = i0[e], q = i1[e];
+                const int32_t A = Y[p] - Y[q], B = X[q] - X[p];
+                int32_t C = __mul24(X[p], Y[q]) - __mul24(X[q], Y[p]);
+                C -= (int32_t)!(B > 0 || (B == 0 && A > 0));
+                rr.e[3 * e + 0] = A;
+                rr.e[3 * e + 1] = B;
+                rr.e[3 * e + 2] = C;
+                csum += C;
+            }
+            rr.sf = (float)csum;
+            rr.wide = 0;
+            // A box of at most 2x2 pixels none of which passes the edge
+            // test (the raster's, rasterizer.go:147) yields no fragment: it
+            // stays out of the tile lists. Dense meshes far from the camera
+            // emit mostly such sub-pixel triangles.
+            if (x1 - x0 <= 1 && y1 - y0 <= 1) {
+                int32_t any = 0;
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const int32_t x = min(x0 + (k & 1), x1), y = min(y0 + (k >> 1), y1);
+                    const int32_t f0 = (int32_t)edge24(rr.e[0], x, rr.e[1], y, rr.e[2]);
+                    const int32_t f1 = (int32_t)edge24(rr.e[3], x, rr.e[4], y, rr.e[5]);
+                    const int32_t f2 = (int32_t)edge24(rr.e[6], x, rr.e[7], y, rr.e[8]);
+                    any |= f0 & f1 & f2;
+                }
+                if (any >= 0) x1 = x0 - 1;
+            }
+        } else {
+            // Wrapping int64 arithmetic as the reference's int.
+            int64_t ix[3], iy[3];
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                ix[j] = go_int(sx[j]);
+                iy[j] = go_int(sy[j]);
+            }
+            const int64_t mnx = max(min(min(ix[0], ix[1]), ix[2]), (int64_t)0);
+            const int64_t mxx = min(max(max(ix[0], ix[1]), ix[2]), (int64_t)fr.W - 1);
+            const int64_t mny = max(min(min(iy[0], iy[1]), iy[2]), (int64_t)0);
+            const int64_t mxy = min(max(max(iy[0], iy[1]), iy[2]), (int64_t)fr.H - 1);
+            const bool some = mnx <= mxx && mny <= mxy;
+            x0 = some ? (int)mnx : 1;
+            x1 = some ? (int)mxx : 0;
+            y0 = (int)mny;
+            y1 = (int)mxy;
+            int64_t csum = 0;
+            uint32_t adj = 0;
+#pragma unroll
+            for (int e = 0; e < 3; e++) {
+                const int p = i0[e], q = i1[e];
+                const int64_t A = wsub(iy[p], iy[q]);
+                const int64_t B = wsub(ix[q], ix[p]);
+                int64_t C = wsub(wmul(ix[p], iy[q]), wmul(ix[q], iy[p]));
+                if (!(B > 0 || (B == 0 && A > 0))) {
+                    C = wsub(C, 1);
+                    adj |= 1u << e;
+                }
+                csum = wadd(csum, C);
+            }
+#pragma unroll
+            for (int e = 0; e < 9; e++) rr.e[e] = 0;
+            rr.sf = (float)csum;
+            rr.wide = 1;
+            WideRec wr;
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                wr.x[j] = ix[j];
+                wr.y[j] = iy[j];
+            }
+            wr.adj = adj;
+            wr.pad[0] = wr.pad[1] = wr.pad[2] = 0;
+            if (some) gstore(&fr.wrec[ri], wr);
         }
-        // rasterizer.go:99-104 with tile (0,0)-(W,H) of the sequential renderer.
-        int64_t mnx = max(min(min(ix[0], ix[1]), ix[2]), (int64_t)0);
-        int64_t mxx = min(max(max(ix[0], ix[1]), ix[2]), (int64_t)fr.W - 1);
-        int64_t mny = max(min(min(iy[0], iy[1]), iy[2]), (int64_t)0);
-        int64_t mxy = min(max(max(iy[0], iy[1]), iy[2]), (int64_t)fr.H - 1);
-        if ((fr.flags & kShowFaces) && mnx <= mxx && mny <= mxy) {
-            rr.bx0 = (int16_t)mnx;
-            rr.bx1 = (int16_t)mxx;
-            rr.by0 = (int16_t)mny;
-            rr.by1 = (int16_t)mxy;
+        if (x0 <= x1 && y0 <= y1) {
+            rr.bx0 = (int16_t)x0;
+            rr.bx1 = (int16_t)x1;
+            rr.by0 = (int16_t)y0;
+            rr.by1 = (int16_t)y1;
+            box = make_uint2((uint32_t)x0 | (uint32_t)x1 << 16, (uint32_t)y0 | (uint32_t)y1 << 16);
             rr.z0 = zw[0];
             rr.z1 = zw[1];
             rr.z2 = zw[2];
-            bool fast = true;
-#pragma unroll
-            for (int j = 0; j < 3; j++)
-                fast = fast && ix[j] >= -kFastCoord && ix[j] <= kFastCoord &&
-                       iy[j] >= -kFastCoord && iy[j] <= kFastCoord;
-            // Edge functions f_e(x,y) = A*x + B*y + C (rasterizer.go:107-117) with the
-            // top-left adjustment folded into C (rasterizer.go:120-129). The pixel
-            // sum fx12 + fx20 + fx01 is the sum of the C's (the A and B terms
-            // cancel).
-            const int i0[3] = {0, 1, 2}, i1[3] = {1, 2, 0};
-            if (fast) {
-                // |x|, |y| <= 2^14: 24-bit products, and every value (the sum of
-                // the three C's included) fits int32.
-                int32_t X[3], Y[3], csum = 0;
-#pragma unroll
-                for (int j = 0; j < 3; j++) {
-                    X[j] = (int32_t)ix[j];
-                    Y[j] = (int32_t)iy[j];
-                }
-#pragma unroll
-                for (int e = 0; e < 3; e++) {
-                    const int p = i0[e], q = i1[e];
-                    const int32_t A = Y[p] - Y[q], B = X[q] - X[p];
-                    int32_t C = __mul24(X[p], Y[q]) - __mul24(X[q], Y[p]);
-                    if (!(B > 0 || (B == 0 && A > 0))) C -= 1;
-                    rr.e[3 * e + 0] = A;
-                    rr.e[3 * e + 1] = B;
-                    rr.e[3 * e + 2] = C;
-                    csum += C;
-                }
-                rr.sf = (float)csum;
-                // A box of at most 2x2 pixels none of which passes the edge
-                // test (the raster's, rasterizer.go:147) yields no fragment: it
-                // stays out of the tile lists. Dense meshes far from the camera
-                // emit mostly such sub-pixel triangles.
-                if (mxx - mnx <= 1 && mxy - mny <= 1) {
-                    int32_t any = 0;
-#pragma unroll
-                    for (int k = 0; k < 4; k++) {
-                        const int32_t x = (int32_t)min(mnx + (k & 1), mxx);
-                        const int32_t y = (int32_t)min(mny + (k >> 1), mxy);
-                        const int32_t f0 = (int32_t)edge24(rr.e[0], x, rr.e[1], y, rr.e[2]);
-                        const int32_t f1 = (int32_t)edge24(rr.e[3], x, rr.e[4], y, rr.e[5]);
-                        const int32_t f2 = (int32_t)edge24(rr.e[6], x, rr.e[7], y, rr.e[8]);
-                        any |= f0 & f1 & f2;
-                    }
-                    if (any >= 0) {
-                        rr.bx0 = 1;
-                        rr.bx1 = 0;
-                        rr.by0 = 1;
-                        rr.by1 = 0;
-                    }
-                }
-            } else {
-                // Wrapping int64 arithmetic as the reference's int.
-                int64_t csum = 0;
-                uint32_t adj = 0;
-#pragma unroll
-                for (int e = 0; e < 3; e++) {
-                    const int p = i0[e], q = i1[e];
-                    const int64_t A = wsub(iy[p], iy[q]);
-                    const int64_t B = wsub(ix[q], ix[p]);
-                    int64_t C = wsub(wmul(ix[p], iy[q]), wmul(ix[q], iy[p]));
-                    if (!(B > 0 || (B == 0 && A > 0))) {
-                        C = wsub(C, 1);
-                        adj |= 1u << e;
-                    }
-                    csum = wadd(csum, C);
-                }
-                rr.sf = (float)csum;
-                rr.wide = 1;
-                WideRec wr;
-#pragma unroll
-                for (int j = 0; j < 3; j++) {
-                    wr.x[j] = ix[j];
-                    wr.y[j] = iy[j];
-                }
-                wr.adj = adj;
-                wr.pad[0] = wr.pad[1] = wr.pad[2] = 0;
-                gstore(&fr.wrec[ri], wr);
-            }
-            // Nothing reads the shading inputs and reciprocals of an empty box. The
-            // divisions only the raster stage needs are done here, where the
+            rr.rsf = rr.rz0 = rr.rz1 = rr.rz2 = 0.f;
+            // The divisions only the raster stage needs are done here, where the
             // triangle is in registers: in k_bin_fill they cost reading 64 and
             // writing 48 bytes of every record again (8 requests over 4M resident
             // triangles: k_bin_fill 177 -> 121 us, k_face unchanged; 32 frames of
             // 200,000: 50 -> 44 and 116 -> 122 us).
-            if (rr.bx0 <= rr.bx1) {
-                // The reciprocals of the divisors for the exact quotient path, whose
-                // numerators are nonzero int32 edge values and barycentrics with
-                // |alpha|, |beta| >= 2^-41 and gamma = +0 or |gamma| >= 2^-64 (left 0,
-                // i.e. IEEE division, for int64 triangles and divisors outside
-                // rcp_range).
-                if (!rr.wide && rcp_range(rr.sf) && rcp_range(rr.z0) && rcp_range(rr.z1) &&
-                    rcp_range(rr.z2)) {
-                    rr.rsf = 1.0f / rr.sf;
-                    rr.rz0 = 1.0f / rr.z0;
-                    rr.rz1 = 1.0f / rr.z1;
-                    rr.rz2 = 1.0f / rr.z2;
-                }
-                ShadeRec sr;
-                // rasterizer.go:132-137
-                sr.uz[0] = a.u / rr.z0;
-                sr.vz[0] = a.v / rr.z0;
-                sr.uz[1] = b.u / rr.z1;
-                sr.vz[1] = b.v / rr.z1;
-                sr.uz[2] = c.u / rr.z2;
-                sr.vz[2] = c.v / rr.z2;
-                sr.in[0] = a.i;
-                sr.in[1] = b.i;
-                sr.in[2] = c.i;
-                sr.tex = tex;
-                sr.sf = rr.sf;
-                sr.rsf = rr.wide ? kShadeWide : __float_as_uint(rr.rsf);
-                gstore(&fr.srec[ri], sr);
+            //
+            // The reciprocals of the divisors for the exact quotient path, whose
+            // numerators are nonzero int32 edge values and barycentrics with
+            // |alpha|, |beta| >= 2^-41 and gamma = +0 or |gamma| >= 2^-64 (left 0,
+            // i.e. IEEE division, for int64 triangles and divisors outside
+            // rcp_range).
+            if (!rr.wide && rcp_range(rr.sf) && rcp_range(rr.z0) && rcp_range(rr.z1) &&
+                rcp_range(rr.z2)) {
+                rr.rsf = 1.0f / rr.sf;
+                rr.rz0 = 1.0f / rr.z0;
+                rr.rz1 = 1.0f / rr.z1;
+                rr.rz2 = 1.0f / rr.z2;
             }
+            ShadeRec sr;
+            // rasterizer.go:132-137
+            sr.uz[0] = a.u / rr.z0;
+            sr.vz[0] = a.v / rr.z0;
+            sr.uz[1] = b.u / rr.z1;
+            sr.vz[1] = b.v / rr.z1;
+            sr.uz[2] = c.u / rr.z2;
+            sr.vz[2] = c.v / rr.z2;
+            sr.in[0] = a.i;
+            sr.in[1] = b.i;
+            sr.in[2] = c.i;
+            sr.tex = tex;
+            sr.sf = rr.sf;
+            sr.rsf = rr.wide ? kShadeWide : __float_as_uint(rr.rsf);
+            gstore(&fr.srec[ri], sr);
+            gstore(&fr.rrec[ri], rr);
         }
     }
-    gstore(&fr.rrec[ri], rr);
-    box = make_uint2((uint32_t)(uint16_t)rr.bx0 | (uint32_t)(uint16_t)rr.bx1 << 16,
-                     (uint32_t)(uint16_t)rr.by0 | (uint32_t)(uint16_t)rr.by1 << 16);
-    return tpf | (tris << 16);
+    if (box.x == kEmptyBox) store_empty_box(fr, ri);
+    return tpf | (binned ? 1u << 16 : 0u);
 }
 
-// A slot that holds no triangle (record ri): an empty box, never binned or
-// finalized.
+// A slot that holds no triangle (record ri): an empty box, never binned.
 __device__ __forceinline__ void empty_record(const DevFrame& fr, uint32_t ri) {
-    RasterRec rr;
-    rr.sf = rr.z0 = rr.z1 = rr.z2 = 0.f;
-    rr.rsf = rr.rz0 = rr.rz1 = rr.rz2 = 0.f;
-    rr.bx0 = 1;
-    rr.bx1 = 0;
-    rr.by0 = 1;
-    rr.by1 = 0;
-    rr.wide = 0;
-#pragma unroll
-    for (int e = 0; e < 9; e++) rr.e[e] = 0;
-    gstore(&fr.rrec[ri], rr);
+    store_empty_box(fr, ri);
     if (fr.orec) {
         OverlayRec o = {};
         gstore(&fr.orec[ri], o);
@@ -902,7 +903,6 @@ struct TileRect {
 
 // Tile range of a raster record's box (empty: tx0 > tx1), from the record's
 // piece 2 (bx0 | bx1 << 16, by0 | by1 << 16, wide, A01).
-constexpr uint32_t kEmptyBox = 1u;  // bx0 = 1, bx1 = 0
 __device__ __forceinline__ TileRect box_tiles(uint32_t bx, uint32_t by, int twl, int thl) {
     const int bx0 = (int)(int16_t)(bx & 0xFFFFu), bx1 = (int)(int16_t)(bx >> 16);
     const int by0 = (int)(int16_t)(by & 0xFFFFu), by1 = (int)(int16_t)(by >> 16);
@@ -1262,18 +1262,20 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
         run += total;
         // Fan of q (Polygon.Triangulate, clipping.go:44-62): (P0, P1, P2),
         // then (P0, P2, P3) for a quad.
-        {
-            uint2 box = make_uint2(kEmptyBox, 0u);
-            if (mode == 1 || mode == 3)
-                add_emit(st, emit_triangle(fr, q[0], q[1], q[2], tex, block_rec(b, ovf, off), box));
-            count(box);
-        }
-        if (__ballot(mode == 3 && nq == 4)) {
-            uint2 box = make_uint2(kEmptyBox, 0u);
-            if (mode == 3 && nq == 4)
-                add_emit(st, emit_triangle(fr, q[0], q[2], q[3], tex, block_rec(b, ovf, off + 1),
+        bool emit = mode == 1 || mode == 3;
+#pragma unroll 1
+        for (uint32_t t = 0;; t++) {
+            uint2 box = make_uint2(kEmptyBox, kEmptyBox);
+            if (emit)
+                add_emit(st, emit_triangle(fr, q[0], q[1], q[2], tex, block_rec(b, ovf, off + t),
                                            box));
             count(box);
+            emit = mode == 3 && nq == 4;
+            if (t == 1 || !__ballot(emit)) break;
+            if (emit) {
+                q[1] = q[2];
+                q[2] = q[3];
+            }
         }
 
         // General faces, kStage at a time: the wave clips each one into its
@@ -1300,7 +1302,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
                 wave_sync();
             }
             const int r = lane / kMaxFan, t = lane - r * kMaxFan;
-            uint2 box = make_uint2(kEmptyBox, 0u);
+            uint2 box = make_uint2(kEmptyBox, kEmptyBox);
             if (r < nst) {
                 const int k = W.stage_k[r];
                 const uint32_t ri = block_rec(b, ovf, (uint32_t)W.stage_off[r] + (uint32_t)t);
@@ -1413,8 +1415,9 @@ __global__ __launch_bounds__(kDecorateThreads) void k_decorate(
         constexpr uint32_t kRed = 0xFF0000FFu;  // {255, 0, 0, 255}
         for (int l = wave; l < 4 * fr.ref_tiles; l += kDecorateThreads / 64) {
             // Tile bounds are whole numbers within the frame (at most 16384).
-            const float* r = fr.ref_tile_rect[l >> 2];
-            const int sx = (int)r[0], sy = (int)r[1], ex = (int)r[2], ey = (int)r[3];
+            const int ng = fr.ref_tiles == 16 ? 4 : 1, t = l >> 2;
+            const float *cx = fr.ref_cols[t % ng], *cy = fr.ref_rows[t / ng];
+            const int sx = (int)cx[0], sy = (int)cy[0], ex = (int)cx[1], ey = (int)cy[1];
             switch (l & 3) {
             case 0: fb_axis_line(fr, sx, sy, ex, sy, kRed, lane); break;
             case 1: fb_axis_line(fr, ex, sy, ex, ey, kRed, lane); break;
