@@ -73,7 +73,7 @@ struct Pipe {
     // batch: frames | objects | stats | counters | frame_overflow | XCD tables,
     // uploaded with one copy per draw (the counters as zeros).
     DevBuf batch, rrec, srec, wrec, tile_counts, tiles, blocks, refs, ctrl;
-    DevBuf items;  // raster work items (later parts of split tiles)
+    DevBuf splits;  // first work item and tile of each slab
     DevBuf slabs;  // depth keys of split tiles; zero between draws
     DevBuf okey;   // overlay keys of the frames that draw overlays; zero between draws
     DevBuf orec;   // overlay records per triangle record (batches with overlay frames)
@@ -564,11 +564,12 @@ struct Bufs {
     uint32_t* rec_pool = nullptr;
     uint32_t* tile_counts = nullptr;  // zero between draws (k_raster re-zeroes)
     uint32_t* tiles = nullptr;        // offsets | cursors | slabs
-    gr::RasterItem* items = nullptr;
-    uint32_t max_items = 0;
+    uint32_t* split_first = nullptr;  // [max_slabs + 1]
+    uint32_t* split_tile = nullptr;   // [max_slabs]
     unsigned long long* slabs = nullptr;  // zero between draws
     uint32_t max_slabs = 0;
-    uint32_t part_refs = 0;
+    uint32_t part_refs = 0;   // tile-list entries per raster part
+    uint32_t split_refs = 0;  // the configured tile_split, for the statistics
     uint32_t* refs = nullptr;
     unsigned long long refs_cap = 0;
     gr::DevControl* ctrl = nullptr;  // sticky until read
@@ -577,15 +578,29 @@ struct Bufs {
     const gr::DevTexture* textures = nullptr;
 };
 
-// Split tiles: a tile is split only when its list is longer than part_refs,
-// so the items of a batch number at most refs_cap / part_refs and the split
-// tiles at most refs_cap / (part_refs + 1); slabs are further capped by a
-// memory budget (a tile without a slab is rasterised whole).
-void split_limits(unsigned long long refs_cap, uint32_t part_refs, size_t slab_bytes,
-                  uint32_t* max_items, uint32_t* max_slabs) {
-    *max_items = (uint32_t)std::min<unsigned long long>(refs_cap / part_refs + 1, 0xFFFFFFF0ull);
-    *max_slabs = (uint32_t)std::max<unsigned long long>(
-        1, std::min<unsigned long long>(refs_cap / (part_refs + 1ull) + 1, kSlabBudget / slab_bytes));
+// Entries per raster part. A launch of at most kFineTiles tiles leaves the chip's
+// 2,048 raster workgroups part idle and lasts as long as its longest list: lists
+// are split from kFinePart entries on (one staged chunk) while every tile can have
+// a slab. Larger launches split at the configured tile_split. (us of parts and
+// raster with parts of 512 | 192 | 128 | 64 entries: 64 instances of 1M triangles
+// 109 | 82 | 68 | 53, a frame of 5,000 28 | 28 | 31 | 30; frames of 200,000
+// triangles in flight 66 -> 44 us each with 64.)
+constexpr int kFineTiles = 4096;
+constexpr uint32_t kFinePart = 64;
+uint32_t part_size(const Plan& P, uint32_t tile_split, size_t slab_bytes,
+                   unsigned long long slab_budget) {
+    const bool fine = P.tiles <= kFineTiles && (unsigned long long)P.tiles * slab_bytes <= slab_budget;
+    return fine ? std::min(kFinePart, tile_split) : tile_split;
+}
+
+// Slabs of a batch: a tile is split only when its list is longer than part_refs,
+// so the split tiles number at most refs_cap / (part_refs + 1); slabs are further
+// capped by a memory budget (a tile without a slab is rasterised whole).
+uint32_t slab_limit(const Plan& P, unsigned long long refs_cap, uint32_t part_refs,
+                    size_t slab_bytes) {
+    return (uint32_t)std::max<unsigned long long>(
+        1, std::min<unsigned long long>({refs_cap / (part_refs + 1ull) + 1,
+                                         kSlabBudget / slab_bytes, (unsigned long long)P.tiles}));
 }
 
 // The header as uploaded: device pointers patched in, counters zero.
@@ -623,11 +638,12 @@ gr::LaunchParams launch_params(const Plan& P, const Bufs& B) {
     p.tile_offsets = B.tiles;
     p.tile_cursor = B.tiles + P.tiles;
     p.tile_slab = B.tiles + 2 * (size_t)P.tiles;
-    p.items = B.items;
-    p.max_items = B.max_items;
+    p.split_first = B.split_first;
+    p.split_tile = B.split_tile;
     p.slabs = B.slabs;
     p.max_slabs = B.max_slabs;
     p.part_refs = B.part_refs;
+    p.split_refs = B.split_refs;
     p.frame_overflow = (uint32_t*)(bb + P.off_over);
     p.blocks = B.blocks;
     p.rec_pool = B.rec_pool;
@@ -702,7 +718,7 @@ size_t records_of(const Plan& P, uint32_t pools, uint32_t per) {
 // Device buffers of a plan in a set of growable buffers (a pipe's or a batch
 // graph's); new allocations that must start at zero are zero-filled on s.
 gr_status size_bufs(gr_context* c, const Plan& P, Pipe& Q, unsigned long long refs_cap,
-                    uint32_t part_refs, int TW, int TH, hipStream_t s, Bufs& B) {
+                    uint32_t tile_split, int TW, int TH, hipStream_t s, Bufs& B) {
     gr_status st;
     uint32_t pools, per;
     record_pools(P, refs_cap, &pools, &per);
@@ -715,9 +731,9 @@ gr_status size_bufs(gr_context* c, const Plan& P, Pipe& Q, unsigned long long re
     if ((st = ensure_zeroed(c, Q.tile_counts, (size_t)P.tiles * 4, s))) return st;
     if ((st = ensure(c, Q.tiles, 3 * (size_t)P.tiles * sizeof(uint32_t)))) return st;
     const size_t slab_bytes = (size_t)TW * TH * 8;
-    uint32_t max_items, max_slabs;
-    split_limits(refs_cap, part_refs, slab_bytes, &max_items, &max_slabs);
-    if ((st = ensure(c, Q.items, (size_t)max_items * sizeof(gr::RasterItem)))) return st;
+    const uint32_t part_refs = part_size(P, tile_split, slab_bytes, kSlabBudget);
+    const uint32_t max_slabs = slab_limit(P, refs_cap, part_refs, slab_bytes);
+    if ((st = ensure(c, Q.splits, (2 * (size_t)max_slabs + 1) * sizeof(uint32_t)))) return st;
     if ((st = ensure_zeroed(c, Q.slabs, (size_t)max_slabs * slab_bytes, s))) return st;
     if ((st = ensure(c, Q.blocks, std::max(P.fblocks, 1) * sizeof(gr::FaceBlock)))) return st;
     if ((st = ensure(c, Q.refs, refs_cap * sizeof(uint32_t)))) return st;
@@ -735,11 +751,12 @@ gr_status size_bufs(gr_context* c, const Plan& P, Pipe& Q, unsigned long long re
     B.rec_pool = (uint32_t*)Q.pools.p;
     B.tile_counts = (uint32_t*)Q.tile_counts.p;
     B.tiles = (uint32_t*)Q.tiles.p;
-    B.items = (gr::RasterItem*)Q.items.p;
-    B.max_items = max_items;
+    B.split_first = (uint32_t*)Q.splits.p;
+    B.split_tile = B.split_first + max_slabs + 1;
     B.slabs = (unsigned long long*)Q.slabs.p;
     B.max_slabs = max_slabs;
     B.part_refs = part_refs;
+    B.split_refs = tile_split;
     B.blocks = (gr::FaceBlock*)Q.blocks.p;
     B.refs = (uint32_t*)Q.refs.p;
     B.refs_cap = refs_cap;
@@ -945,7 +962,7 @@ gr_status present_enqueue(gr_context* c, gr_context::PresentSlot& ps) {
 
 void free_pipe_bufs(Pipe& pp) {
     DevBuf* pb[] = {&pp.batch, &pp.rrec,    &pp.srec, &pp.wrec,  &pp.tile_counts,
-                    &pp.tiles, &pp.blocks,  &pp.refs, &pp.ctrl,  &pp.items,
+                    &pp.tiles, &pp.blocks,  &pp.refs, &pp.ctrl,  &pp.splits,
                     &pp.slabs, &pp.okey,    &pp.orec,  &pp.pools};
     for (DevBuf* b : pb) {
         if (b->p) (void)hipFree(b->p);
@@ -1246,8 +1263,7 @@ gr_status enqueue_noalloc(gr_context* c, const gr_frame* frame, const gr_object*
         B.refs = (uint32_t*)((char*)base + off);
         B.refs_cap = std::min<unsigned long long>((bytes - off) / 4, (unsigned long long)kMaxRefs);
         B.part_refs = 0xFFFFFFFFu;  // no split tiles
-        B.items = nullptr;
-        B.max_items = 0;
+        B.split_refs = 0xFFFFFFFFu;
         B.slabs = nullptr;
         B.max_slabs = 0;
 

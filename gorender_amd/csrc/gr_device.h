@@ -190,19 +190,13 @@ enum : int32_t {
 
 // Per-batch counters, uploaded as zeros with the descriptors of every draw.
 struct DevBatchCounters {
-    unsigned long long refs_used;  // tile-list entries allocated so far
-    uint32_t n_items;              // raster work items (later parts of split tiles)
-    uint32_t n_slabs;              // slabs handed to split tiles
+    unsigned long long refs_used;  // tile-list entries allocated so far (batches of several frames)
+    unsigned long long split;      // slabs << 32 | work items handed to split tiles
     unsigned long long recs_used;  // triangle records the face blocks claimed (k_bin_scan)
 };
 
-// Tile not split (no slab); also the end of the raster work queue.
+// Tile not split (no slab).
 constexpr uint32_t kNoSlab = 0xFFFFFFFFu;
-
-// Raster work item: a later part (>= 1) of a split tile.
-struct RasterItem {
-    uint32_t tile, part;
-};
 
 // Sticky control words (cleared by the host when it reads them): set when a
 // frame of any batch needed more tile-list entries or triangle records than

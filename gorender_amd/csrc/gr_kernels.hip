@@ -313,6 +313,25 @@ __device__ __forceinline__ uint32_t wave_reduce(uint32_t v, uint32_t none, F f) 
     return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
+// Inclusive sums over the lanes of the wave (all active), by the same steps.
+__device__ __forceinline__ uint32_t wave_scan_u32(uint32_t v) {
+#define GR_DPP(ctrl, rows) \
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xF, false)
+    GR_DPP(0x111, 0xF);
+    GR_DPP(0x112, 0xF);
+    GR_DPP(0x114, 0xF);
+    GR_DPP(0x118, 0xF);
+    GR_DPP(0x142, 0xA);
+    GR_DPP(0x143, 0xC);
+#undef GR_DPP
+    return v;
+}
+// The same in 64 bits, from the sums of the 16-bit halves.
+__device__ __forceinline__ unsigned long long wave_scan_u64(uint32_t v) {
+    return (unsigned long long)wave_scan_u32(v & 0xFFFFu) +
+           ((unsigned long long)wave_scan_u32(v >> 16) << 16);
+}
+
 __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
     return wave_reduce(v, 0u, [](uint32_t a, uint32_t b) { return a + b; });
 }
@@ -1473,33 +1492,47 @@ __global__ __launch_bounds__(256) void k_fog(uint32_t* __restrict__ rgba,
 // A kernel of its own: a last-block scan inside k_face would need a device-scope
 // release in every face workgroup, which on a multi-XCD part writes back and
 // invalidates L2 each time.
-__global__ __launch_bounds__(1024) void k_bin_scan(const DevFrame* __restrict__ frames,
-                                                   uint32_t* __restrict__ tile_counts,
-                                                   uint32_t* __restrict__ tile_offsets,
-                                                   uint32_t* __restrict__ tile_cursor,
-                                                   uint32_t* __restrict__ frame_overflow,
-                                                   unsigned long long* __restrict__ stats,
-                                                   DevBatchCounters* __restrict__ counters,
-                                                   DevControl* __restrict__ ctrl,
-                                                   unsigned long long refs_capacity,
-                                                   uint32_t* __restrict__ tile_slab,
-                                                   RasterItem* __restrict__ items,
-                                                   uint32_t max_items, uint32_t max_slabs,
-                                                   uint32_t part_refs,
-                                                   uint32_t* __restrict__ rec_pool,
-                                                   const FaceBlock* __restrict__ blocks) {
-    __shared__ unsigned long long wsum[16];
-    __shared__ unsigned long long wstat[16][4];
-    __shared__ unsigned long long base_s;
+//
+// A tile whose list holds more than part_refs entries is split into parts of that
+// many: part 0 stays with the tile's raster workgroup, the others are work items of
+// k_raster_parts. The tile takes a slab (depth keys of its pixels) and split_first[
+// slab] = its first item, split_tile[slab] = the tile; one counter hands out both, so
+// items ascend with slabs and k_raster_parts finds an item's tile by search. With no
+// slab left the tile stays whole (slower, same result).
+constexpr int kScanThreads = 1024;
+__global__ __launch_bounds__(kScanThreads) void k_bin_scan(
+    const DevFrame* __restrict__ frames, int nframes, uint32_t* __restrict__ tile_counts,
+    uint32_t* __restrict__ tile_offsets, uint32_t* __restrict__ tile_cursor,
+    uint32_t* __restrict__ frame_overflow, unsigned long long* __restrict__ stats,
+    DevBatchCounters* __restrict__ counters, DevControl* __restrict__ ctrl,
+    unsigned long long refs_capacity, uint32_t* __restrict__ tile_slab,
+    uint32_t* __restrict__ split_first, uint32_t* __restrict__ split_tile, uint32_t max_slabs,
+    uint32_t part_refs, uint32_t split_refs, uint32_t* __restrict__ rec_pool,
+    const FaceBlock* __restrict__ blocks) {
+    constexpr int NW = kScanThreads / 64;
+    __shared__ unsigned long long wsum[NW], wsplit[NW];
+    __shared__ uint32_t wstat[NW][4];
+    __shared__ unsigned long long base_s, split_s;
     const int f = blockIdx.x;
     const DevFrame& fr = frames[f];
     const int ntiles = fr.tiles_x * fr.tiles_y;
     uint32_t* cnt = tile_counts + fr.tile_begin;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = sgpr(threadIdx.x >> 6);
+
+    // The first tiles of the thread stay in registers from the totals to the
+    // offsets (2,048 tiles in all); later ones are read again.
+    constexpr int kKeep = 2;
+    uint32_t v0[kKeep];
+#pragma unroll
+    for (int k = 0; k < kKeep; k++) {
+        const int i = (int)threadIdx.x + k * kScanThreads;
+        v0[k] = i < ntiles ? gld(&cnt[i]) : 0u;
+    }
 
     // k_face is done with the record pools: their total to the batch counters,
     // and the counters back to zero for the next draw.
-    static_assert(kRecPools % 64 == 0 && kRecPools <= 1024, "whole waves read the pool counters");
+    static_assert(kRecPools % 64 == 0 && kRecPools <= kScanThreads,
+                  "whole waves read the pool counters");
     if (f == 0 && threadIdx.x < kRecPools) {
         uint32_t* pc = &rec_pool[threadIdx.x * kPoolStride];
         const uint32_t v = *pc;
@@ -1508,38 +1541,48 @@ __global__ __launch_bounds__(1024) void k_bin_scan(const DevFrame* __restrict__ 
         if (lane == 0) atomicAdd(&counters->recs_used, t);
     }
 
-    unsigned long long local = 0;
-    for (int i = threadIdx.x; i < ntiles; i += 1024) local += cnt[i];
     // The counters of the frame's face blocks: TPF references, binned
-    // triangles, front faces, clip overflows.
-    unsigned long long bs[4] = {0, 0, 0, 0};
-    for (int i = threadIdx.x; i < fr.face_blocks; i += 1024) {
-        const FaceBlock fb = gload(&blocks[fr.face_block_begin + i]);
-        bs[0] += fb.c0 & 0xFFFFu;
-        bs[1] += fb.c0 >> 16;
-        bs[2] += (fb.c >> 11) & 511u;
-        bs[3] += fb.c >> 20;
-    }
-    local = wave_sum_u64(local);
+    // triangles, front faces, clip overflows, 65536 blocks a round at most, so
+    // that a wave's sums of 16-bit fields fit 32 bits.
+    unsigned long long bt = 0;  // lanes 0..3 of wave 1: the totals
+    for (int r0 = 0; r0 < fr.face_blocks; r0 += 65536) {
+        uint32_t bs[4] = {0, 0, 0, 0};
+        const int end = min(fr.face_blocks, r0 + 65536);
+        for (int i = r0 + (int)threadIdx.x; i < end; i += kScanThreads) {
+            const FaceBlock fb = gload(&blocks[fr.face_block_begin + i]);
+            bs[0] += fb.c0 & 0xFFFFu;
+            bs[1] += fb.c0 >> 16;
+            bs[2] += (fb.c >> 11) & 511u;
+            bs[3] += fb.c >> 20;
+        }
 #pragma unroll
-    for (int k = 0; k < 4; k++) bs[k] = wave_sum_u64(bs[k]);
-    if (lane == 0) {
-        wsum[wave] = local;
-#pragma unroll
-        for (int k = 0; k < 4; k++) wstat[wave][k] = bs[k];
+        for (int k = 0; k < 4; k++) bs[k] = wave_sum_u32(bs[k]);
+        if (r0) __syncthreads();  // the last round's terms are read
+        if (lane < 4) wstat[wave][lane] = lane == 0 ? bs[0] : lane == 1 ? bs[1] : lane == 2 ? bs[2] : bs[3];
+        __syncthreads();
+        if (wave == 1 && lane < 4)
+            for (int w = 0; w < NW; w++) bt += wstat[w][lane];
     }
-    __syncthreads();
-    if (threadIdx.x >= 64 && threadIdx.x < 68) {
-        const int k = (int)threadIdx.x - 64;
+    if (wave == 1 && lane < 4) {
         const int idx[4] = {kStatTpf, kStatTriangles, kStatFront, kStatClipOverflow};
-        unsigned long long t = 0;
-        for (int w = 0; w < 16; w++) t += wstat[w][k];
-        stats[f * kNumStats + idx[k]] = t;
+        stats[f * kNumStats + idx[lane]] = bt;
     }
+
+    // The frame's references, and its range of the lists.
+    unsigned long long local = 0;
+#pragma unroll
+    for (int k = 0; k < kKeep; k++) local += v0[k];
+    for (int i = (int)threadIdx.x + kKeep * kScanThreads; i < ntiles; i += kScanThreads)
+        local += gld(&cnt[i]);
+    local = wave_sum_u64(local);
+    if (lane == 0) wsum[wave] = local;
+    __syncthreads();
     if (threadIdx.x == 0) {
         unsigned long long tot = 0;
-        for (int w = 0; w < 16; w++) tot += wsum[w];
-        const unsigned long long base = atomicAdd(&counters->refs_used, tot);
+        for (int w = 0; w < NW; w++) tot += wsum[w];
+        // One frame starts at 0, without waiting for the counter.
+        unsigned long long base = 0;
+        if (nframes > 1) base = atomicAdd(&counters->refs_used, tot);
         stats[f * kNumStats + kStatRefs] = tot;
         if (base + tot > refs_capacity) {
             frame_overflow[f] = 1u;
@@ -1551,46 +1594,55 @@ __global__ __launch_bounds__(1024) void k_bin_scan(const DevFrame* __restrict__ 
     __syncthreads();
     const bool over = frame_overflow[f] != 0u;
     unsigned long long run = base_s;
-    for (int c = 0; c < ntiles; c += 1024) {
-        const int i = c + threadIdx.x;
-        const uint32_t v = i < ntiles ? cnt[i] : 0u;
-        unsigned long long x = v;
-        for (int s = 1; s < 64; s <<= 1) {
-            unsigned long long y = __shfl_up(x, s, 64);
-            if (lane >= s) x += y;
+    for (int c = 0; c < ntiles; c += kScanThreads) {
+        const int i = c + (int)threadIdx.x;
+        uint32_t v;
+        if (c == 0)
+            v = v0[0];
+        else if (c == kScanThreads)
+            v = v0[1];
+        else
+            v = i < ntiles ? gld(&cnt[i]) : 0u;
+        const bool split = !over && v > part_refs;
+        const uint64_t sm = __ballot(split);
+        const unsigned long long x = wave_scan_u64(v);
+        const uint32_t more = split ? (v - 1u) / part_refs : 0u;  // items of the tile
+        const uint32_t xi = sm ? wave_scan_u32(more) : 0u;
+        if (c) __syncthreads();  // the last round's terms are read
+        if (lane == 63) {
+            wsum[wave] = x;
+            wsplit[wave] = (unsigned long long)__popcll(sm) << 32 | xi;
         }
         __syncthreads();
-        if (lane == 63) wsum[wave] = x;
-        __syncthreads();
-        unsigned long long wbase = 0, ctot = 0;
-        for (int w = 0; w < 16; w++) {
-            if (w < wave) wbase += wsum[w];
+        unsigned long long wbase = 0, ctot = 0, sbase = 0, stot = 0;
+        for (int w = 0; w < NW; w++) {
+            if (w < wave) {
+                wbase += wsum[w];
+                sbase += wsplit[w];
+            }
             ctot += wsum[w];
+            stot += wsplit[w];
         }
         if (i < ntiles) {
-            const unsigned long long offv = run + wbase + x - v;
-            tile_offsets[fr.tile_begin + i] = (uint32_t)offv;
-            tile_cursor[fr.tile_begin + i] = (uint32_t)offv;
+            const uint32_t offv = (uint32_t)(run + wbase + x - v);
+            tile_offsets[fr.tile_begin + i] = offv;
+            tile_cursor[fr.tile_begin + i] = offv;
             if (over) cnt[i] = 0u;  // overflowed frame: raster draws background only
-            if (!over && v > part_refs) {
-                // Split the list into parts of part_refs entries: part 0 stays
-                // with the tile's workgroup, the others become work items. With
-                // no slab left the tile stays whole (slower, same result).
-                const uint32_t np = (v - 1u) / part_refs + 1u;
-                uint32_t slab = atomicAdd(&counters->n_slabs, 1u);
-                if (slab < max_slabs) {
-                    atomicAdd(&stats[f * kNumStats + kStatSplit], 1ull);
-                    // Items of all split tiles number at most refs / part_refs,
-                    // and max_items is sized for the whole tile-list capacity.
-                    const uint32_t ib = atomicAdd(&counters->n_items, np - 1u);
-                    for (uint32_t k = 1; k < np; k++)
-                        if (ib + k - 1u < max_items)
-                            items[ib + k - 1u] = RasterItem{(uint32_t)(fr.tile_begin + i), k};
-                } else {
-                    slab = kNoSlab;
-                }
-                tile_slab[fr.tile_begin + i] = slab;
+        }
+        if (stot) {  // the same in every thread
+            if (threadIdx.x == 0) split_s = atomicAdd(&counters->split, stot);
+            __syncthreads();
+            sbase += split_s;
+            const uint32_t slab = (uint32_t)(sbase >> 32) + (uint32_t)__popcll(sm & lanemask_lt(lane));
+            if (split) {
+                const uint32_t tile = (uint32_t)(fr.tile_begin + i);
+                if (slab <= max_slabs) split_first[slab] = (uint32_t)sbase + xi - more;
+                if (slab < max_slabs) split_tile[slab] = tile;
+                tile_slab[tile] = slab < max_slabs ? slab : kNoSlab;
             }
+            const uint64_t cm = __ballot(split && slab < max_slabs && v > split_refs);
+            if (cm && lane == 0)
+                atomicAdd(&stats[f * kNumStats + kStatSplit], (unsigned long long)__popcll(cm));
         }
         run += ctot;
     }
@@ -2191,11 +2243,11 @@ void k_raster_parts(const DevFrame* __restrict__ frames, const int* __restrict__
                     int nframes,
                     const uint32_t* __restrict__ tile_counts,
                     const uint32_t* __restrict__ tile_offsets,
-                    const uint32_t* __restrict__ tile_slab, const uint32_t* __restrict__ refs,
-                    unsigned long long* __restrict__ stats,
-                    DevBatchCounters* __restrict__ counters, const RasterItem* __restrict__ items,
-                    uint32_t max_items, unsigned long long* __restrict__ slabs,
-                    uint32_t part_refs) {
+                    const uint32_t* __restrict__ refs, unsigned long long* __restrict__ stats,
+                    const DevBatchCounters* __restrict__ counters,
+                    const uint32_t* __restrict__ split_first,
+                    const uint32_t* __restrict__ split_tile, uint32_t max_slabs,
+                    unsigned long long* __restrict__ slabs, uint32_t part_refs) {
     constexpr int NPX = TW * TH;
     __shared__ unsigned long long key[NPX];
     __shared__ uint4 lrec[kRasterChunk * 5];
@@ -2203,9 +2255,13 @@ void k_raster_parts(const DevFrame* __restrict__ frames, const int* __restrict__
     __shared__ uint32_t qbuf[4][3][128];
     __shared__ unsigned long long red;  // covered fragments of the item
     const int lane = threadIdx.x & 63, wave = sgpr(threadIdx.x >> 6);
-    // Written by k_bin_scan (an earlier kernel).
-    const uint32_t n_items = min(counters->n_items, max_items);
-    if (n_items == 0u) return;
+    // Written by k_bin_scan (an earlier kernel); items past the last slab are of
+    // tiles left whole.
+    const unsigned long long split = counters->split;
+    const uint32_t n_slabs = min((uint32_t)(split >> 32), max_slabs);
+    if (n_slabs == 0u) return;
+    const uint32_t n_items = (uint32_t)(split >> 32) > max_slabs ? split_first[max_slabs]
+                                                                 : (uint32_t)split;
     // A fixed stride, not a queue counter: atomics of one cache line are served
     // one every 12 ns, so the ~6,000 items and 2,048 workgroups of a batch of 8
     // dense requests waited for the counter (k_raster_parts 414 -> 322 us), and
@@ -2214,8 +2270,9 @@ void k_raster_parts(const DevFrame* __restrict__ frames, const int* __restrict__
     // restructure the loop so that one thread leaves it while the others go
     // round the barriers again, which hangs.
     for (uint32_t it = blockIdx.x; it < n_items; it += gridDim.x) {
-        const int tile = sgpr((int)items[it].tile);
-        const uint32_t wpart = (uint32_t)sgpr((int)items[it].part);
+        const int slab_i = wave_last_le((const int*)split_first, (int)n_slabs, (int)it);
+        const int tile = sgpr((int)split_tile[slab_i]);
+        const uint32_t wpart = it - (uint32_t)sgpr((int)split_first[slab_i]) + 1u;
         if (threadIdx.x == 0) red = 0ull;  // ordered by raster_list's barriers
         const int fi = wave_last_le(tile_first, nframes, tile);
         const DevFrame& fr = frames[fi];
@@ -2229,7 +2286,7 @@ void k_raster_parts(const DevFrame* __restrict__ frames, const int* __restrict__
                                 min(cnt - beg, part_refs), key, lrec, lslot, qbuf[wave], lane,
                                 wave);
         __syncthreads();
-        unsigned long long* slab = slabs + (size_t)tile_slab[tile] * NPX;
+        unsigned long long* slab = slabs + (size_t)slab_i * NPX;
         for (int i = threadIdx.x; i < NPX; i += 256) {
             const unsigned long long k = key[i];
             if ((uint32_t)k != 0u) atomicMax(&slab[i], k);
@@ -2441,10 +2498,10 @@ void launch_overlay(const LaunchParams& p, hipStream_t s) {
 }
 
 void launch_bin_scan(const LaunchParams& p, hipStream_t s) {
-    hipLaunchKernelGGL(k_bin_scan, dim3(p.nframes), dim3(1024), 0, s, p.frames, p.tile_counts,
-                       p.tile_offsets, p.tile_cursor, p.frame_overflow, p.stats, p.counters,
-                       p.ctrl, p.refs_capacity, p.tile_slab, p.items, p.max_items, p.max_slabs,
-                       p.part_refs, p.rec_pool, p.blocks);
+    hipLaunchKernelGGL(k_bin_scan, dim3(p.nframes), dim3(kScanThreads), 0, s, p.frames, p.nframes,
+                       p.tile_counts, p.tile_offsets, p.tile_cursor, p.frame_overflow, p.stats,
+                       p.counters, p.ctrl, p.refs_capacity, p.tile_slab, p.split_first,
+                       p.split_tile, p.max_slabs, p.part_refs, p.split_refs, p.rec_pool, p.blocks);
 }
 
 void launch_bin_fill(const LaunchParams& p, hipStream_t s) {
@@ -2618,13 +2675,13 @@ static void raster_t(const LaunchParams& p, hipStream_t s, bool parts) {
         // raster's occupancy, but no more than the batch has tiles (a single
         // frame rarely splits many); with no work items they return at once,
         // and any number of them covers the items.
-        const uint32_t grid = std::min<uint32_t>(
-            std::min<uint32_t>(p.max_items, 256u * (uint32_t)raster_waves(TW * TH)),
-            std::max<uint32_t>(256u, (uint32_t)p.total_tiles));
-        if (grid)
+        const uint32_t grid = std::min<uint32_t>(256u * (uint32_t)raster_waves(TW * TH),
+                                                 std::max<uint32_t>(256u, (uint32_t)p.total_tiles));
+        if (p.max_slabs)
             hipLaunchKernelGGL((k_raster_parts<TW, TH>), dim3(grid), dim3(256), 0, s, p.frames,
-                               p.tile_first, p.nframes, p.tile_counts, p.tile_offsets, p.tile_slab, p.refs,
-                               p.stats, p.counters, p.items, p.max_items, p.slabs, p.part_refs);
+                               p.tile_first, p.nframes, p.tile_counts, p.tile_offsets, p.refs,
+                               p.stats, p.counters, p.split_first, p.split_tile, p.max_slabs,
+                               p.slabs, p.part_refs);
         return;
     }
     if (p.raster_persistent) {

@@ -24,11 +24,12 @@ struct LaunchParams {
     uint32_t* tile_offsets;  // [total_tiles]
     uint32_t* tile_cursor;   // [total_tiles]
     uint32_t* tile_slab;     // [total_tiles]: slab of a split tile or kNoSlab
-    RasterItem* items;       // [max_items]: later parts of split tiles
-    uint32_t max_items;
+    uint32_t* split_first;   // [max_slabs + 1]: first work item of each slab's tile
+    uint32_t* split_tile;    // [max_slabs]: the slab's tile
     unsigned long long* slabs;  // [max_slabs][tile pixels] keys; zero between draws
     uint32_t max_slabs;
     uint32_t part_refs;      // tile-list entries per raster part
+    uint32_t split_refs;     // lists longer than this count as split (gr_stats.tiles_split)
     uint32_t* frame_overflow;// [nframes]
     FaceBlock* blocks;       // [face_blocks]
     uint32_t* rec_pool;      // [kRecPools * kPoolStride]: pool counters; zero between draws

@@ -254,6 +254,39 @@ def test_face_stage_forms(ctx):
             ctx.destroy_mesh(h)
 
 
+@pytest.mark.parametrize("split", [64, 100, 512])
+@pytest.mark.parametrize("eye,grid", [(1.2, (40, 64)), (4.0, (90, 144))])
+def test_split_sizes(ctx, split, eye, grid):
+    """A frame alone (its lists in parts of at most 64 entries) and in a batch
+    of over 4,096 tiles (parts of tile_split): the same frame and statistics,
+    for lists of one part, of whole parts and of broken ones."""
+    import scene_cases as C
+    scene = C.sphere(w=160, h=128, eye=(0, 0, eye), nlat=grid[0], nlon=grid[1])
+    pad = C.sphere(w=2048, h=2112)
+    pad.objects = []
+    frames = [scene, pad]
+    handles = [ctx.upload_scene(s)[0] for s in frames]
+    outs = [ctx.frame_buffers(s.frame.width, s.frame.height) for s in frames]
+    want = refcpu.draw(scene)
+    old = ctx.config()
+    ctx.set_config(tile_split=split)
+    try:
+        alone = ctx.draw(scene, handles[0])
+        ctx.draw_batch(frames, handles, [(o[0].ptr, o[1].ptr) for o in outs])
+        ctx.synchronize()
+        stats = ctx.last_stats()[0]
+    finally:
+        ctx.set_config(tile_split=old.tile_split)
+    assert_same(scene, alone, want)
+    got = (outs[0][0].to_numpy(np.uint8, (128, 160, 4)),
+           outs[0][1].to_numpy(np.float32, (128, 160)), stats)
+    assert_same(scene, got, want)
+    assert stats == alone[2]
+    for rg, dp in outs:
+        rg.free()
+        dp.free()
+
+
 def test_frames_sharing_objects(ctx):
     """Frames of a batch that name the same range of its object array."""
     import scene_cases as C
