@@ -73,8 +73,9 @@ struct Pipe {
     // batch: frames | objects | stats | counters | frame_overflow | XCD tables,
     // uploaded with one copy per draw (the counters as zeros).
     DevBuf batch, rrec, srec, wrec, tile_counts, tiles, blocks, refs, ctrl;
-    DevBuf splits;  // first work item and tile of each slab
-    DevBuf slabs;  // depth keys of split tiles; zero between draws
+    DevBuf splits;  // first entry and tile of each slab
+    DevBuf slabs;  // depth keys of split tiles, then their counts of merged parts; zero
+                   // between draws
     DevBuf okey;   // overlay keys of the frames that draw overlays; zero between draws
     DevBuf orec;   // overlay records per triangle record (batches with overlay frames)
     DevBuf pools;  // record pool counters (zero between draws)
@@ -567,8 +568,9 @@ struct Bufs {
     uint32_t* split_first = nullptr;  // [max_slabs + 1]
     uint32_t* split_tile = nullptr;   // [max_slabs]
     unsigned long long* slabs = nullptr;  // zero between draws
+    uint32_t* slab_done = nullptr;        // zero between draws
     uint32_t max_slabs = 0;
-    uint32_t part_refs = 0;   // tile-list entries per raster part
+    uint32_t part_refs = 0;   // least tile-list entries per raster part
     uint32_t split_refs = 0;  // the configured tile_split, for the statistics
     uint32_t* refs = nullptr;
     unsigned long long refs_cap = 0;
@@ -641,6 +643,7 @@ gr::LaunchParams launch_params(const Plan& P, const Bufs& B) {
     p.split_first = B.split_first;
     p.split_tile = B.split_tile;
     p.slabs = B.slabs;
+    p.slab_done = B.slab_done;
     p.max_slabs = B.max_slabs;
     p.part_refs = B.part_refs;
     p.split_refs = B.split_refs;
@@ -671,10 +674,9 @@ gr_status launch_plan(gr_context* c, const Plan& P, const gr::LaunchParams& p, h
     timed_launch(c, "k_bin_scan", s, [&] { gr::launch_bin_scan(p, s); });
     timed_launch(c, "k_bin_fill", s, [&] { gr::launch_bin_fill(p, s); });
     if (P.okey_words) timed_launch(c, "k_overlay", s, [&] { gr::launch_overlay(p, s); });
-    bool ok = true;
-    timed_launch(c, "k_raster_parts", s, [&] { ok = gr::launch_raster_parts(p, s); });
     if (raster_after) GR_HIP(hipStreamWaitEvent(s, raster_after, 0));
-    if (ok) timed_launch(c, "k_raster", s, [&] { ok = gr::launch_raster(p, s); });
+    bool ok = true;
+    timed_launch(c, "k_raster", s, [&] { ok = gr::launch_raster(p, s); });
     // Drawn over the finished frame, before the event the next batch's raster
     // waits for (it may write the same buffers).
     if (ok && P.decorate) timed_launch(c, "k_decorate", s, [&] { gr::launch_decorate(p, s); });
@@ -734,7 +736,7 @@ gr_status size_bufs(gr_context* c, const Plan& P, Pipe& Q, unsigned long long re
     const uint32_t part_refs = part_size(P, tile_split, slab_bytes, kSlabBudget);
     const uint32_t max_slabs = slab_limit(P, refs_cap, part_refs, slab_bytes);
     if ((st = ensure(c, Q.splits, (2 * (size_t)max_slabs + 1) * sizeof(uint32_t)))) return st;
-    if ((st = ensure_zeroed(c, Q.slabs, (size_t)max_slabs * slab_bytes, s))) return st;
+    if ((st = ensure_zeroed(c, Q.slabs, (size_t)max_slabs * (slab_bytes + 4), s))) return st;
     if ((st = ensure(c, Q.blocks, std::max(P.fblocks, 1) * sizeof(gr::FaceBlock)))) return st;
     if ((st = ensure(c, Q.refs, refs_cap * sizeof(uint32_t)))) return st;
     if ((st = ensure_zeroed(c, Q.ctrl, sizeof(gr::DevControl), s))) return st;
@@ -754,6 +756,7 @@ gr_status size_bufs(gr_context* c, const Plan& P, Pipe& Q, unsigned long long re
     B.split_first = (uint32_t*)Q.splits.p;
     B.split_tile = B.split_first + max_slabs + 1;
     B.slabs = (unsigned long long*)Q.slabs.p;
+    B.slab_done = (uint32_t*)((char*)Q.slabs.p + (size_t)max_slabs * slab_bytes);
     B.max_slabs = max_slabs;
     B.part_refs = part_refs;
     B.split_refs = tile_split;
@@ -974,7 +977,7 @@ void free_pipe_bufs(Pipe& pp) {
 
 // One batch's launch sequence captured in two HIP graphs, with its own device
 // buffers: counter zeroing, k_face, k_bin_scan, k_bin_fill, k_overlay and
-// k_raster_parts in the geometry graph; k_raster and k_decorate in the raster
+// k_overlay in the geometry graph; k_raster and k_decorate in the raster
 // graph, so that a replay's raster can wait for the previous batch's between
 // the two graph launches while its geometry overlaps that raster.
 struct gr_batch_graph {
@@ -1059,7 +1062,7 @@ gr_status graph_build(gr_batch_graph* g) {
              gr::launch_bin_scan(p, s);
              gr::launch_bin_fill(p, s);
              if (P.okey_words) gr::launch_overlay(p, s);
-             return gr::launch_raster_parts(p, s);
+             return true;
          })))
         return st;
     if ((st = capture(g, &g->ras, &g->ras_x, [&] {

@@ -191,7 +191,7 @@ enum : int32_t {
 // Per-batch counters, uploaded as zeros with the descriptors of every draw.
 struct DevBatchCounters {
     unsigned long long refs_used;  // tile-list entries allocated so far (batches of several frames)
-    unsigned long long split;      // slabs << 32 | work items handed to split tiles
+    unsigned long long split;      // slabs << 32 | entries of split tiles
     unsigned long long recs_used;  // triangle records the face blocks claimed (k_bin_scan)
 };
 

@@ -250,7 +250,8 @@ __host__ __device__ __forceinline__ int xcd_count(int x, int n) {
 // 64 lanes of a wave at once: one round trip to memory per factor of 64, where a
 // binary search takes one per factor of 2 (9 for the 512 frames of a batch, on
 // the path of every face block and every tile).
-__device__ __forceinline__ int wave_last_le(const int* key, int n, int b) {
+template <typename T>
+__device__ __forceinline__ int wave_last_le(const T* key, int n, T b) {
     if (n == 1) return 0;
     const int lane = (int)(threadIdx.x & 63u);
     int lo = 0, len = n;
@@ -1493,12 +1494,11 @@ __global__ __launch_bounds__(256) void k_fog(uint32_t* __restrict__ rgba,
 // release in every face workgroup, which on a multi-XCD part writes back and
 // invalidates L2 each time.
 //
-// A tile whose list holds more than part_refs entries is split into parts of that
-// many: part 0 stays with the tile's raster workgroup, the others are work items of
-// k_raster_parts. The tile takes a slab (depth keys of its pixels) and split_first[
-// slab] = its first item, split_tile[slab] = the tile; one counter hands out both, so
-// items ascend with slabs and k_raster_parts finds an item's tile by search. With no
-// slab left the tile stays whole (slower, same result).
+// A tile whose list holds more than part_refs entries may be split over several
+// raster workgroups: it takes a slab (depth keys of its pixels), and its entries a
+// range [split_first[slab], + count) of the split tiles' entries put end to end
+// (split_tile[slab] = the tile). One counter hands out both, so the ranges ascend
+// with the slabs. With no slab left the tile stays whole (slower, same result).
 constexpr int kScanThreads = 1024;
 __global__ __launch_bounds__(kScanThreads) void k_bin_scan(
     const DevFrame* __restrict__ frames, int nframes, uint32_t* __restrict__ tile_counts,
@@ -1606,8 +1606,8 @@ __global__ __launch_bounds__(kScanThreads) void k_bin_scan(
         const bool split = !over && v > part_refs;
         const uint64_t sm = __ballot(split);
         const unsigned long long x = wave_scan_u64(v);
-        const uint32_t more = split ? (v - 1u) / part_refs : 0u;  // items of the tile
-        const uint32_t xi = sm ? wave_scan_u32(more) : 0u;
+        const uint32_t sv = split ? v : 0u;
+        const uint32_t xi = sm ? wave_scan_u32(sv) : 0u;
         if (c) __syncthreads();  // the last round's terms are read
         if (lane == 63) {
             wsum[wave] = x;
@@ -1636,7 +1636,7 @@ __global__ __launch_bounds__(kScanThreads) void k_bin_scan(
             const uint32_t slab = (uint32_t)(sbase >> 32) + (uint32_t)__popcll(sm & lanemask_lt(lane));
             if (split) {
                 const uint32_t tile = (uint32_t)(fr.tile_begin + i);
-                if (slab <= max_slabs) split_first[slab] = (uint32_t)sbase + xi - more;
+                if (slab <= max_slabs) split_first[slab] = (uint32_t)sbase + xi - sv;
                 if (slab < max_slabs) split_tile[slab] = tile;
                 tile_slab[tile] = slab < max_slabs ? slab : kNoSlab;
             }
@@ -1906,7 +1906,7 @@ __device__ __forceinline__ void frag_depth(const uint32_t (*q)[128], uint32_t he
 // LDS of k_raster beyond the key array: 64 staged records (80 B) and slots,
 // the per-wave fragment rings and the stats reduction.
 constexpr int kRasterChunk = 64;
-constexpr int kRasterLdsFixed = kRasterChunk * (80 + 4) + 4 * 3 * 128 * 4 + 4 * 2 * 8;
+constexpr int kRasterLdsFixed = kRasterChunk * (80 + 4) + 4 * 3 * 128 * 4 + 4 * 2 * 8 + 16;
 
 // Waves per SIMD the tile's LDS allows (one wave per SIMD per workgroup), at
 // most 8: the register budget follows from it (512 / waves VGPRs).
@@ -2230,128 +2230,138 @@ __device__ __forceinline__ unsigned long long shade_tile(const DevFrame& fr, int
     return shaded;
 }
 
-// A tile whose list holds more than part_refs entries, and that k_bin_scan gave
-// a slab, is split into parts of part_refs entries. Parts 1.. are work items
-// that k_raster_parts resolves first, workgroup w taking items w, w + grid, ...:
-// each resolves its entries into LDS keys and merges them into
-// the tile's slab in HBM with a 64-bit max (the (depth, sequence) resolve does
-// not depend on order). k_raster then resolves part 0 of every tile, folds in
-// the slab of a split tile (and clears it) and shades.
+// LDS of one raster workgroup.
 template <int TW, int TH>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_waves(TW * TH))))
-void k_raster_parts(const DevFrame* __restrict__ frames, const int* __restrict__ tile_first,
-                    int nframes,
-                    const uint32_t* __restrict__ tile_counts,
-                    const uint32_t* __restrict__ tile_offsets,
-                    const uint32_t* __restrict__ refs, unsigned long long* __restrict__ stats,
-                    const DevBatchCounters* __restrict__ counters,
-                    const uint32_t* __restrict__ split_first,
-                    const uint32_t* __restrict__ split_tile, uint32_t max_slabs,
-                    unsigned long long* __restrict__ slabs, uint32_t part_refs) {
-    constexpr int NPX = TW * TH;
-    __shared__ unsigned long long key[NPX];
-    __shared__ uint4 lrec[kRasterChunk * 5];
-    __shared__ uint32_t lslot[kRasterChunk];
-    __shared__ uint32_t qbuf[4][3][128];
-    __shared__ unsigned long long red;  // covered fragments of the item
-    const int lane = threadIdx.x & 63, wave = sgpr(threadIdx.x >> 6);
-    // Written by k_bin_scan (an earlier kernel); items past the last slab are of
-    // tiles left whole.
+struct RasterLds {
+    unsigned long long key[TW * TH];
+    uint4 lrec[kRasterChunk * 5];  // the staged raster records
+    uint32_t lslot[kRasterChunk];
+    uint32_t qbuf[4][3][128];      // per-wave ring: pixel, f12, f20
+    unsigned long long red[4][2];  // per wave: covered fragments, shaded pixels
+    uint32_t last;                 // the workgroup shades a split tile
+};
+
+// Entries of the batch's split tiles (k_bin_scan) and the size of their parts:
+// part_refs, or what `extra` workgroups need to take one part each. Entries past
+// the last slab are of tiles left whole.
+struct SplitLists {
+    uint32_t n_slabs, entries, part;
+};
+__device__ __forceinline__ SplitLists split_lists(const DevBatchCounters* counters,
+                                                  const uint32_t* split_first, uint32_t max_slabs,
+                                                  uint32_t part_refs, uint32_t extra) {
     const unsigned long long split = counters->split;
-    const uint32_t n_slabs = min((uint32_t)(split >> 32), max_slabs);
-    if (n_slabs == 0u) return;
-    const uint32_t n_items = (uint32_t)(split >> 32) > max_slabs ? split_first[max_slabs]
-                                                                 : (uint32_t)split;
-    // A fixed stride, not a queue counter: atomics of one cache line are served
-    // one every 12 ns, so the ~6,000 items and 2,048 workgroups of a batch of 8
-    // dense requests waited for the counter (k_raster_parts 414 -> 322 us), and
-    // the items are of one size. Every branch around the barriers of this loop
-    // is wave-uniform (scalar): thread-level branches here let the compiler
-    // restructure the loop so that one thread leaves it while the others go
-    // round the barriers again, which hangs.
-    for (uint32_t it = blockIdx.x; it < n_items; it += gridDim.x) {
-        const int slab_i = wave_last_le((const int*)split_first, (int)n_slabs, (int)it);
-        const int tile = sgpr((int)split_tile[slab_i]);
-        const uint32_t wpart = it - (uint32_t)sgpr((int)split_first[slab_i]) + 1u;
-        if (threadIdx.x == 0) red = 0ull;  // ordered by raster_list's barriers
-        const int fi = wave_last_le(tile_first, nframes, tile);
-        const DevFrame& fr = frames[fi];
-        const int t = tile - fr.tile_begin;
-        const int X0 = (t % fr.tiles_x) * TW, Y0 = (t / fr.tiles_x) * TH;
-        const uint32_t cnt = tile_counts[tile], beg = wpart * part_refs;
-        for (int i = threadIdx.x; i < NPX; i += 256) key[i] = kBackgroundKey;
-        // raster_list's first barrier orders the initialisation before its use.
-        unsigned long long covered =
-            raster_list<TW, TH>(fr, X0, Y0, refs + tile_offsets[tile] + beg,
-                                min(cnt - beg, part_refs), key, lrec, lslot, qbuf[wave], lane,
-                                wave);
-        __syncthreads();
-        unsigned long long* slab = slabs + (size_t)slab_i * NPX;
-        for (int i = threadIdx.x; i < NPX; i += 256) {
-            const unsigned long long k = key[i];
-            if ((uint32_t)k != 0u) atomicMax(&slab[i], k);
-        }
-        const unsigned long long cov = wave_total(covered, lane);
-        if (lane == 0 && cov) atomicAdd(&red, cov);
-        __syncthreads();
-        if (wave == 0 && lane == 0 && red) atomicAdd(&stats[fi * kNumStats + kStatCovered], red);
-        // red and the LDS tile state are read before the next item overwrites them.
-        __syncthreads();
-    }
+    const uint32_t n = (uint32_t)(split >> 32);
+    SplitLists s;
+    s.n_slabs = min(n, max_slabs);
+    s.entries = n > max_slabs ? split_first[max_slabs] : (uint32_t)split;
+    s.part = max(part_refs, s.entries / max(extra, 1u) + 1u);
+    return s;
 }
 
-// Screen tile g: part 0 of its list (all of it when the tile is not split),
-// then the deferred shading. Every thread of the workgroup calls it.
+// One part of a tile's list, resolved into LDS keys, and the tile shaded where the
+// part is all of it.
+//
+// The split tiles' entries, put end to end, are cut at every multiple of s.part and
+// at the tiles' ends: item k >= 0 is the part that starts at entry k * s.part, and
+// the tile's own workgroup (item < 0, tile g) takes its first entries, up to the
+// first such multiple. So every workgroup has one part, whatever the lists' lengths.
+// The parts of a tile merge their keys into its slab with a 64-bit max (the (depth,
+// sequence) resolve does not depend on order); the workgroup that merges last takes
+// them back, leaves the slab and its counter cleared for the next draw, and shades.
+// No part waits for another. Every thread of the workgroup calls it.
 template <int TW, int TH>
-__device__ __forceinline__ void raster_tile(
-    int g, const DevFrame* __restrict__ frames, const int* __restrict__ tile_first, int nframes,
-    uint32_t* __restrict__ tile_counts,
-    const uint32_t* __restrict__ tile_offsets, const uint32_t* __restrict__ tile_slab,
-    const uint32_t* __restrict__ refs, const DevTexture* __restrict__ textures,
-    unsigned long long* __restrict__ stats, unsigned long long* __restrict__ slabs,
-    uint32_t part_refs, unsigned long long* key, uint4* lrec, uint32_t* lslot,
-    uint32_t (*qbuf)[3][128], unsigned long long (*red)[2], int lane, int wave) {
+__device__ __forceinline__ void raster_part(
+    const DevFrame* __restrict__ frames, const int* __restrict__ tile_first, int nframes,
+    uint32_t* __restrict__ tile_counts, const uint32_t* __restrict__ tile_offsets,
+    const uint32_t* __restrict__ tile_slab, const uint32_t* __restrict__ refs,
+    const DevTexture* __restrict__ textures, unsigned long long* __restrict__ stats,
+    const uint32_t* __restrict__ split_first, const uint32_t* __restrict__ split_tile,
+    unsigned long long* __restrict__ slabs, uint32_t* __restrict__ slab_done, uint32_t part_refs,
+    int g, int item, const SplitLists& s, RasterLds<TW, TH>& L, int lane, int wave) {
     constexpr int NPX = TW * TH;
+    uint32_t slab_i = kNoSlab, first = 0u, pos = 0u;
+    if (item >= 0) {
+        const unsigned long long at = (unsigned long long)item * s.part;
+        if (at >= s.entries) return;
+        pos = (uint32_t)at;
+        slab_i = (uint32_t)wave_last_le(split_first, (int)s.n_slabs, pos);
+        first = (uint32_t)sgpr((int)split_first[slab_i]);
+        if (pos == first) return;  // the tile's own workgroup starts there
+        g = sgpr((int)split_tile[slab_i]);
+    }
+    const uint32_t cnt = (uint32_t)sgpr((int)tile_counts[g]);
+    if (item < 0 && cnt > part_refs) {
+        slab_i = (uint32_t)sgpr((int)tile_slab[g]);
+        if (slab_i != kNoSlab) pos = first = (uint32_t)sgpr((int)split_first[slab_i]);
+    }
+    // Parts of the tile, and this one's entries [beg, beg + n).
+    uint32_t beg = 0u, n = cnt, parts = 1u;
+    if (slab_i != kNoSlab) {
+        parts += (first + cnt - 1u) / s.part - first / s.part;
+        beg = pos - first;
+        n = min(cnt - beg, s.part - pos % s.part);
+    }
     const int fi = wave_last_le(tile_first, nframes, g);
     const DevFrame& fr = frames[fi];
     const int t = g - fr.tile_begin;
     const int X0 = (t % fr.tiles_x) * TW, Y0 = (t / fr.tiles_x) * TH;
 
-    for (int i = threadIdx.x; i < NPX; i += 256) key[i] = kBackgroundKey;
-
-    const uint32_t cnt = tile_counts[g], off = tile_offsets[g];
-    const uint32_t slab_i = cnt > part_refs ? tile_slab[g] : kNoSlab;
+    for (int i = threadIdx.x; i < NPX; i += 256) L.key[i] = kBackgroundKey;
     // raster_list's first barrier orders the initialisation before its use.
-    const unsigned long long covered = raster_list<TW, TH>(
-        fr, X0, Y0, refs + off, slab_i != kNoSlab ? part_refs : cnt, key, lrec, lslot, qbuf[wave],
-        lane, wave);
+    const unsigned long long covered =
+        raster_list<TW, TH>(fr, X0, Y0, refs + tile_offsets[g] + beg, n, L.key, L.lrec, L.lslot,
+                            L.qbuf[wave], lane, wave);
     __syncthreads();
-    if (slab_i != kNoSlab) {
-        // Fold in the later parts (merged by k_raster_parts; 0 = no fragment)
-        // and leave the slab cleared for the next draw.
+    bool shade = true;
+    if (parts > 1u) {
         unsigned long long* slab = slabs + (size_t)slab_i * NPX;
         for (int i = threadIdx.x; i < NPX; i += 256) {
-            const unsigned long long k = slab[i];
-            if (k > key[i]) key[i] = k;
-            slab[i] = 0ull;
+            const unsigned long long k = L.key[i];
+            if ((uint32_t)k != 0u) atomicMax(&slab[i], k);
         }
+        // Device-scope atomics are performed at memory, and counted as complete
+        // only then: every wave's merges are in the slab before its workgroup
+        // counts itself done. (A device-scope fence would write back and
+        // invalidate the XCD's L2 in every part: 458 -> 1,220 us for 8 dense
+        // requests.)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
+        if (threadIdx.x == 0)
+            L.last = __hip_atomic_fetch_add(&slab_done[slab_i], 1u, __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_AGENT) == parts - 1u;
+        __syncthreads();
+        shade = sgpr((int)L.last) != 0;
+        if (shade) {
+            // Read at memory too (past this XCD's caches).
+            for (int i = threadIdx.x; i < NPX; i += 256) {
+                const unsigned long long k =
+                    __hip_atomic_load(&slab[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                L.key[i] = k ? k : kBackgroundKey;
+                slab[i] = 0ull;
+            }
+            if (threadIdx.x == 0) slab_done[slab_i] = 0u;
+            __syncthreads();
+        }
     }
-    // Tile counts are zero between draws: the face stage of the next draw
-    // accumulates into them again.
-    if (threadIdx.x == 0 && cnt) tile_counts[g] = 0u;
-
-    const unsigned long long shaded = shade_tile<TW, TH>(fr, X0, Y0, key, textures);
+    unsigned long long shaded = 0;
+    if (shade) {
+        // Tile counts are zero between draws: the face stage of the next draw
+        // accumulates into them again.
+        if (threadIdx.x == 0 && cnt) tile_counts[g] = 0u;
+        shaded = shade_tile<TW, TH>(fr, X0, Y0, L.key, textures);
+    }
     const unsigned long long cov = wave_total(covered, lane);
     if (lane == 0) {
-        red[wave][0] = cov;
-        red[wave][1] = shaded;
+        L.red[wave][0] = cov;
+        L.red[wave][1] = shaded;
     }
     __syncthreads();
     if (threadIdx.x < 2) {
-        const unsigned long long s = red[0][threadIdx.x] + red[1][threadIdx.x] +
-                                     red[2][threadIdx.x] + red[3][threadIdx.x];
-        if (s) atomicAdd(&stats[fi * kNumStats + (threadIdx.x ? kStatShaded : kStatCovered)], s);
+        const unsigned long long sum = L.red[0][threadIdx.x] + L.red[1][threadIdx.x] +
+                                       L.red[2][threadIdx.x] + L.red[3][threadIdx.x];
+        if (sum)
+            atomicAdd(&stats[fi * kNumStats + (threadIdx.x ? kStatShaded : kStatCovered)], sum);
     }
 }
 
@@ -2364,51 +2374,56 @@ __device__ __forceinline__ int xcd_tile(int h) {
     return ((j / kTileRun) * 8 + x) * kTileRun + j % kTileRun;
 }
 
-// One workgroup per screen tile (grid: total_tiles rounded up to whole runs
-// of all XCDs; workgroups past the last tile return at once).
+// `extra` workgroups (a multiple of 8) for the later parts of split tiles, one item
+// each, then one per screen tile (total_tiles rounded up to whole runs of all XCDs;
+// workgroups past the last tile or item return at once). One item each, not a loop:
+// what it keeps in scalar registers across items spills (k_raster 295 -> 325 us for
+// 32 frames of 200,000 triangles). Parts in a kernel of their own ahead of the tiles'
+// took 13 us more for a single frame and 75 of 533 us for 8 dense requests.
 template <int TW, int TH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_waves(TW * TH))))
-void k_raster(const DevFrame* __restrict__ frames, const int* __restrict__ tile_first, int nframes,
-              uint32_t* __restrict__ tile_counts, const uint32_t* __restrict__ tile_offsets,
-              const uint32_t* __restrict__ tile_slab, const uint32_t* __restrict__ refs,
-              const DevTexture* __restrict__ textures, unsigned long long* __restrict__ stats,
-              unsigned long long* __restrict__ slabs, uint32_t part_refs, int total_tiles) {
-    const int g = xcd_tile((int)blockIdx.x);
-    if (g >= total_tiles) return;
-    __shared__ unsigned long long key[TW * TH];
-    __shared__ uint4 lrec[kRasterChunk * 5];  // the staged raster records
-    __shared__ uint32_t lslot[kRasterChunk];
-    __shared__ uint32_t qbuf[4][3][128];  // per-wave ring: pixel, f12, f20
-    __shared__ unsigned long long red[4][2];  // per wave: covered fragments, shaded pixels
+void k_raster(
+    const DevFrame* __restrict__ frames, const int* __restrict__ tile_first, int nframes,
+    int total_tiles, uint32_t* __restrict__ tile_counts,
+    const uint32_t* __restrict__ tile_offsets, const uint32_t* __restrict__ tile_slab,
+    const uint32_t* __restrict__ refs, const DevTexture* __restrict__ textures,
+    unsigned long long* __restrict__ stats, const DevBatchCounters* __restrict__ counters,
+    const uint32_t* __restrict__ split_first, const uint32_t* __restrict__ split_tile,
+    unsigned long long* __restrict__ slabs, uint32_t* __restrict__ slab_done, uint32_t max_slabs,
+    uint32_t part_refs, int extra) {
+    __shared__ RasterLds<TW, TH> L;
     const int lane = threadIdx.x & 63, wave = sgpr(threadIdx.x >> 6);
-    raster_tile<TW, TH>(g, frames, tile_first, nframes, tile_counts, tile_offsets, tile_slab, refs, textures,
-                        stats, slabs, part_refs, key, lrec, lslot, qbuf, red, lane, wave);
+    const SplitLists s = split_lists(counters, split_first, max_slabs, part_refs, (uint32_t)extra);
+    const int it = (int)blockIdx.x < extra ? (int)blockIdx.x : -1;
+    const int g = it < 0 ? xcd_tile((int)blockIdx.x - extra) : 0;
+    if (g >= total_tiles) return;
+    raster_part<TW, TH>(frames, tile_first, nframes, tile_counts, tile_offsets, tile_slab, refs,
+                        textures, stats, split_first, split_tile, slabs, slab_done, part_refs, g,
+                        it, s, L, lane, wave);
 }
 
 // Persistent form: a fixed grid (every CU at the raster's occupancy) in which
-// workgroup w draws tiles w, w + grid, w + 2 * grid, ...
+// workgroup w takes w, w + grid, w + 2 * grid, ... of the items and then the tiles.
 template <int TW, int TH>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_waves(TW * TH))))
-void k_raster_persistent(const DevFrame* __restrict__ frames,
-                         const int* __restrict__ tile_first, int nframes,
-                         uint32_t* __restrict__ tile_counts,
-                         const uint32_t* __restrict__ tile_offsets,
-                         const uint32_t* __restrict__ tile_slab, const uint32_t* __restrict__ refs,
-                         const DevTexture* __restrict__ textures,
-                         unsigned long long* __restrict__ stats,
-                         unsigned long long* __restrict__ slabs, uint32_t part_refs,
-                         int total_tiles) {
-    __shared__ unsigned long long key[TW * TH];
-    __shared__ uint4 lrec[kRasterChunk * 5];
-    __shared__ uint32_t lslot[kRasterChunk];
-    __shared__ uint32_t qbuf[4][3][128];
-    __shared__ unsigned long long red[4][2];
+void k_raster_persistent(
+    const DevFrame* __restrict__ frames, const int* __restrict__ tile_first, int nframes,
+    int total_tiles, uint32_t* __restrict__ tile_counts,
+    const uint32_t* __restrict__ tile_offsets, const uint32_t* __restrict__ tile_slab,
+    const uint32_t* __restrict__ refs, const DevTexture* __restrict__ textures,
+    unsigned long long* __restrict__ stats, const DevBatchCounters* __restrict__ counters,
+    const uint32_t* __restrict__ split_first, const uint32_t* __restrict__ split_tile,
+    unsigned long long* __restrict__ slabs, uint32_t* __restrict__ slab_done, uint32_t max_slabs,
+    uint32_t part_refs, int extra) {
+    __shared__ RasterLds<TW, TH> L;
     const int lane = threadIdx.x & 63, wave = sgpr(threadIdx.x >> 6);
-    for (int g = (int)blockIdx.x; g < total_tiles; g += (int)gridDim.x) {
-        raster_tile<TW, TH>(g, frames, tile_first, nframes, tile_counts, tile_offsets, tile_slab, refs,
-                            textures, stats, slabs, part_refs, key, lrec, lslot, qbuf, red, lane,
+    const SplitLists s = split_lists(counters, split_first, max_slabs, part_refs, (uint32_t)extra);
+    for (int j = (int)blockIdx.x; j < extra + total_tiles; j += (int)gridDim.x) {
+        raster_part<TW, TH>(frames, tile_first, nframes, tile_counts, tile_offsets, tile_slab,
+                            refs, textures, stats, split_first, split_tile, slabs, slab_done,
+                            part_refs, j < extra ? 0 : j - extra, j < extra ? j : -1, s, L, lane,
                             wave);
-        // red and the LDS tile state are rewritten by the next tile.
+        // The LDS state is rewritten by the next tile.
         __syncthreads();
     }
 }
@@ -2669,42 +2684,40 @@ void launch_put(void* dst, const void* src, size_t bytes, hipStream_t s) {
 }
 
 template <int TW, int TH>
-static void raster_t(const LaunchParams& p, hipStream_t s, bool parts) {
-    if (parts) {
-        // Workgroups of the parts kernel: enough to fill every CU at the
-        // raster's occupancy, but no more than the batch has tiles (a single
-        // frame rarely splits many); with no work items they return at once,
-        // and any number of them covers the items.
-        const uint32_t grid = std::min<uint32_t>(256u * (uint32_t)raster_waves(TW * TH),
-                                                 std::max<uint32_t>(256u, (uint32_t)p.total_tiles));
-        if (p.max_slabs)
-            hipLaunchKernelGGL((k_raster_parts<TW, TH>), dim3(grid), dim3(256), 0, s, p.frames,
-                               p.tile_first, p.nframes, p.tile_counts, p.tile_offsets, p.refs,
-                               p.stats, p.counters, p.split_first, p.split_tile, p.max_slabs,
-                               p.slabs, p.part_refs);
-        return;
-    }
+static void raster_t(const LaunchParams& p, hipStream_t s) {
+    // Workgroups for split tiles' parts: four times what fills every CU at the
+    // raster's occupancy, so that the parts of a dense batch end close together
+    // (8 dense requests, 7,560 tiles: 628 us with one time, 481 with two, 423 with
+    // four, 425 with eight); fewer for a small batch (one frame: 256, 1,024 and
+    // 2,048 alike), and one time for a batch whose tiles alone fill the chip over
+    // and over (64 mixed frames: one, two, four and eight times alike; they return
+    // at once where nothing is split, 2,048 in 1 of 300 us, 8,192 in 4).
+    const int fill = 256 * raster_waves(TW * TH);
+    const int most = p.total_tiles > 8 * fill ? fill : 4 * fill;
+    const int extra =
+        p.max_slabs ? (std::min(most, std::max(1024, p.total_tiles)) + 7) / 8 * 8 : 0;
     if (p.raster_persistent) {
-        const uint32_t grid =
-            std::min<uint32_t>((uint32_t)p.total_tiles, 256u * (uint32_t)raster_waves(TW * TH));
-        hipLaunchKernelGGL((k_raster_persistent<TW, TH>), dim3(grid), dim3(256), 0, s, p.frames,
-                           p.tile_first, p.nframes, p.tile_counts, p.tile_offsets, p.tile_slab, p.refs,
-                           p.textures, p.stats, p.slabs, p.part_refs, p.total_tiles);
+        hipLaunchKernelGGL((k_raster_persistent<TW, TH>), dim3(std::min(p.total_tiles, fill)),
+                           dim3(256), 0, s, p.frames, p.tile_first, p.nframes,
+                           p.total_tiles, p.tile_counts, p.tile_offsets, p.tile_slab, p.refs,
+                           p.textures, p.stats, p.counters, p.split_first, p.split_tile, p.slabs,
+                           p.slab_done, p.max_slabs, p.part_refs, extra);
         return;
     }
     constexpr int kRound = 8 * kTileRun;
-    const uint32_t grid = (uint32_t)((p.total_tiles + kRound - 1) / kRound * kRound);
-    hipLaunchKernelGGL((k_raster<TW, TH>), dim3(grid), dim3(256), 0, s, p.frames, p.tile_first, p.nframes,
-                       p.tile_counts, p.tile_offsets, p.tile_slab, p.refs, p.textures, p.stats,
-                       p.slabs, p.part_refs, p.total_tiles);
+    const int tiles = (p.total_tiles + kRound - 1) / kRound * kRound;
+    hipLaunchKernelGGL((k_raster<TW, TH>), dim3(tiles + extra), dim3(256), 0, s, p.frames, p.tile_first, p.nframes,
+                           p.total_tiles, p.tile_counts, p.tile_offsets, p.tile_slab, p.refs,
+                           p.textures, p.stats, p.counters, p.split_first, p.split_tile, p.slabs,
+                           p.slab_done, p.max_slabs, p.part_refs, extra);
 }
 
-static bool raster_dispatch(const LaunchParams& p, hipStream_t s, bool parts) {
+bool launch_raster(const LaunchParams& p, hipStream_t s) {
     if (p.total_tiles == 0) return true;
-#define GR_RASTER_CASE(W, H)                          \
-    if (p.tw_log2 == W && p.th_log2 == H) {           \
-        raster_t<(1 << W), (1 << H)>(p, s, parts);    \
-        return true;                                  \
+#define GR_RASTER_CASE(W, H)                \
+    if (p.tw_log2 == W && p.th_log2 == H) { \
+        raster_t<(1 << W), (1 << H)>(p, s); \
+        return true;                        \
     }
     GR_RASTER_CASE(3, 3) GR_RASTER_CASE(3, 4) GR_RASTER_CASE(3, 5) GR_RASTER_CASE(3, 6)
     GR_RASTER_CASE(4, 3) GR_RASTER_CASE(4, 4) GR_RASTER_CASE(4, 5) GR_RASTER_CASE(4, 6)
@@ -2713,8 +2726,5 @@ static bool raster_dispatch(const LaunchParams& p, hipStream_t s, bool parts) {
 #undef GR_RASTER_CASE
     return false;
 }
-
-bool launch_raster_parts(const LaunchParams& p, hipStream_t s) { return raster_dispatch(p, s, true); }
-bool launch_raster(const LaunchParams& p, hipStream_t s) { return raster_dispatch(p, s, false); }
 
 }  // namespace gr

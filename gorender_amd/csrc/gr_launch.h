@@ -24,11 +24,13 @@ struct LaunchParams {
     uint32_t* tile_offsets;  // [total_tiles]
     uint32_t* tile_cursor;   // [total_tiles]
     uint32_t* tile_slab;     // [total_tiles]: slab of a split tile or kNoSlab
-    uint32_t* split_first;   // [max_slabs + 1]: first work item of each slab's tile
+    uint32_t* split_first;   // [max_slabs + 1]: first of the split tiles' entries that
+                             // are of each slab's tile
     uint32_t* split_tile;    // [max_slabs]: the slab's tile
     unsigned long long* slabs;  // [max_slabs][tile pixels] keys; zero between draws
+    uint32_t* slab_done;     // [max_slabs]: parts merged into each slab; zero between draws
     uint32_t max_slabs;
-    uint32_t part_refs;      // tile-list entries per raster part
+    uint32_t part_refs;      // least tile-list entries per raster part
     uint32_t split_refs;     // lists longer than this count as split (gr_stats.tiles_split)
     uint32_t* frame_overflow;// [nframes]
     FaceBlock* blocks;       // [face_blocks]
@@ -72,7 +74,6 @@ void launch_decorate(const LaunchParams& p, hipStream_t s);
 void launch_fog(void* rgba, const void* depth, uint64_t n, float fog_start, float fog_end,
                 uint32_t color, hipStream_t s);
 void launch_bin_fill(const LaunchParams& p, hipStream_t s);
-bool launch_raster_parts(const LaunchParams& p, hipStream_t s);
 bool launch_raster(const LaunchParams& p, hipStream_t s);
 void launch_fill32(uint32_t* p, uint32_t v, size_t n, hipStream_t s);
 // Adds an order-independent digest of `words` 32-bit words at p to *out.
