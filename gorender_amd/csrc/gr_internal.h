@@ -42,7 +42,10 @@ gr_status static_scratch_init(int device);
 void* static_scratch(int device, size_t* bytes);
 // One frame drawn with every per-draw buffer carved from [base, base + bytes +
 // kNoAllocTail): no allocation of any kind on the way.
-constexpr size_t kNoAllocTail = 64u << 10;
+// The tail: face blocks' state, then the split tiles' slabs, counters and ranges.
+constexpr size_t kNoAllocBlocks = 64u << 10;
+constexpr size_t kNoAllocSlabs = 16u << 20;
+constexpr size_t kNoAllocTail = kNoAllocBlocks + kNoAllocSlabs + (1u << 20);
 gr_status enqueue_noalloc(gr_context* c, const gr_frame* frame, const gr_object* objs, int32_t no,
                           void* d_rgba, void* d_depth, void* base, size_t bytes);
 

@@ -2663,23 +2663,50 @@ void launch_checksum(const void* p, size_t words, unsigned long long* out, hipSt
                        words, out);
 }
 
-// Writes c.n words (at most kPutWords) carried by the kernel's arguments to
-// dst: host data reaches device memory without a host buffer that must outlive
-// the call, and without an allocation.
-__global__ __launch_bounds__(256) void k_put(uint32_t* __restrict__ dst, PutChunk c) {
-    for (uint32_t i = threadIdx.x; i < c.n; i += 256) dst[i] = c.w[i];
+// Writes the words carried by the kernel's arguments to their two places and
+// clears the zero ranges: host data reaches device memory without a host buffer
+// that must outlive the call, and without an allocation.
+__global__ __launch_bounds__(256) void k_put(PutChunk c) {
+    const uint32_t t = blockIdx.x * 256u + threadIdx.x, step = gridDim.x * 256u;
+    for (uint32_t i = t; i < c.n[0] + c.n[1]; i += step)
+        (i < c.n[0] ? c.dst[0][i] : c.dst[1][i - c.n[0]]) = c.w[i];
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+        for (size_t i = t; i < c.zero_n[k]; i += step) c.zero[k][i] = make_uint4(0u, 0u, 0u, 0u);
 }
 
-void launch_put(void* dst, const void* src, size_t bytes, hipStream_t s) {
-    const size_t words = (bytes + 3) / 4;
-    for (size_t w0 = 0; w0 < words; w0 += kPutWords) {
+void launch_put(const PutSpan put[2], const ZeroSpan zero[3], hipStream_t s) {
+    // The first launch clears; as many follow as the words need.
+    size_t done[2] = {0, 0};
+    size_t most = 0;
+    for (int k = 0; k < 3; k++) most = std::max(most, zero[k].bytes / 16);
+    for (bool first = true;; first = false) {
         PutChunk c;
-        c.n = (uint32_t)std::min<size_t>(kPutWords, words - w0);
-        c.pad = 0;
-        const size_t b0 = w0 * 4, nb = std::min<size_t>((size_t)c.n * 4, bytes - b0);
-        std::memset(c.w, 0, sizeof c.w);
-        std::memcpy(c.w, (const char*)src + b0, nb);
-        hipLaunchKernelGGL(k_put, dim3(1), dim3(256), 0, s, (uint32_t*)dst + w0, c);
+        std::memset(&c, 0, sizeof c);
+        size_t room = kPutWords, at = 0;
+        for (int k = 0; k < 2; k++) {
+            const size_t words = (put[k].bytes + 3) / 4;
+            const size_t n = std::min(room, words - done[k]);
+            const size_t b0 = done[k] * 4;
+            c.dst[k] = (uint32_t*)put[k].dst + done[k];
+            c.n[k] = (uint32_t)n;
+            if (n)
+                std::memcpy(c.w + at, (const char*)put[k].src + b0,
+                            std::min(n * 4, put[k].bytes - b0));
+            done[k] += n;
+            room -= n;
+            at += n;
+        }
+        if (!first && at == 0) return;
+        size_t blocks = 1;
+        if (first) {
+            for (int k = 0; k < 3; k++) {
+                c.zero[k] = (uint4*)zero[k].p;
+                c.zero_n[k] = zero[k].bytes / 16;
+            }
+            blocks = std::min<size_t>(std::max<size_t>(1, (most + 255) / 256), 1024);
+        }
+        hipLaunchKernelGGL(k_put, dim3((unsigned)blocks), dim3(256), 0, s, c);
     }
 }
 

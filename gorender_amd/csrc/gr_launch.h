@@ -53,11 +53,25 @@ struct LaunchParams {
     int face_grid;
 };
 
-// Host words carried to device memory by one k_put launch (its argument).
-constexpr int kPutWords = 496;
+// Host words carried to device memory by one k_put launch (its argument, within
+// 4 KiB), and ranges it clears (16-byte pieces).
+constexpr int kPutWords = 960;
 struct PutChunk {
-    uint32_t n, pad;
+    uint32_t* dst[2];
+    uint32_t n[2];
+    uint4* zero[3];
+    size_t zero_n[3];
     uint32_t w[kPutWords];
+};
+static_assert(sizeof(PutChunk) <= 4096, "a kernel's arguments");
+struct PutSpan {
+    void* dst;  // 4-byte aligned
+    const void* src;
+    size_t bytes;
+};
+struct ZeroSpan {
+    void* p;       // 16-byte aligned
+    size_t bytes;  // a multiple of 16
 };
 
 // Prefix tables of the XCD-aware order for per-frame unit counts `n`.
@@ -78,7 +92,8 @@ bool launch_raster(const LaunchParams& p, hipStream_t s);
 void launch_fill32(uint32_t* p, uint32_t v, size_t n, hipStream_t s);
 // Adds an order-independent digest of `words` 32-bit words at p to *out.
 void launch_checksum(const void* p, size_t words, unsigned long long* out, hipStream_t s);
-// Copies `bytes` host bytes to dst (4-byte aligned) through kernel arguments.
-void launch_put(void* dst, const void* src, size_t bytes, hipStream_t s);
+// Copies host bytes to device memory through kernel arguments, after clearing the
+// zero ranges (which hold none of them) in the same launch where one is enough.
+void launch_put(const PutSpan put[2], const ZeroSpan zero[3], hipStream_t s);
 
 }  // namespace gr

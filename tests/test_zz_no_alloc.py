@@ -76,6 +76,25 @@ def test_noalloc_frame_past_per_block_records(ctx):
     _same(scene, got, want)
 
 
+@pytest.mark.parametrize("size,tile", [((160, 128), 32), ((512, 512), 8), ((520, 512), 8),
+                                       ((64, 64), 64)])
+def test_noalloc_long_lists(ctx, size, tile):
+    # Lists of hundreds of entries: split in frames of up to 4,096 tiles (whole
+    # and of broken parts), whole in larger ones; the same frame twice, so the
+    # second draw starts from what the first one left.
+    scene = C.sphere(w=size[0], h=size[1], eye=(0, 0, 1.3), nlat=90, nlon=144)
+    old = ctx.config()
+    ctx.set_config(tile_w=tile, tile_h=tile, tile_split=1 << 20)
+    try:
+        want = _draw(ctx, scene, noalloc=False)
+        for _ in range(2):
+            got = _draw(ctx, scene, noalloc=True)
+            _same(scene, got, want)
+        assert_same(scene, (got[0], got[1], got[2]), refcpu.draw(scene))
+    finally:
+        ctx.set_config(tile_w=old.tile_w, tile_h=old.tile_h, tile_split=old.tile_split)
+
+
 def test_noalloc_reports_capacity(ctx):
     # Sixteen copies of a 480-face sphere filling a 4096 x 4096 frame in 8 x 8
     # tiles: millions of tile-list entries, more than the array holds. The
