@@ -287,6 +287,24 @@ def test_split_sizes(ctx, split, eye, grid):
         dp.free()
 
 
+@pytest.mark.parametrize("far", [60000.0, 65531.0, 65532.0, 65540.0])
+def test_overlays_far_vertices(ctx, far):
+    """Unclipped edges and vertex dots up to and past the coordinates that take
+    32-bit steps, on every side of the frame."""
+    w, h = 64, 48
+    px = np.array([[10, 5], [far, 9], [30, 40], [20, 20], [-far + 60, 11], [33, 2],
+                   [7, 7], [9, far], [50, 30], [40, 12], [22, -far + 70], [3, 44]], np.float64)
+    v = np.ones((12, 4), np.float32)
+    v[:, 0], v[:, 1] = (px[:, 0] - w / 2) / (w / 2), (px[:, 1] - h / 2) / (h / 2)
+    v[:, 2] = 0.5
+    flags = _lib.GR_SHOW_FACES | _lib.GR_SHOW_EDGES | _lib.GR_SHOW_VERTICES
+    f = np.arange(12, dtype=np.int32).reshape(4, 3)
+    eye = np.eye(4, dtype=np.float32)
+    scene = S.SceneData(S.FrameData(w, h, flags=flags), [S.MeshData(v, f)], [],
+                        [S.ObjectData(0, eye, eye)], name=f"far-{far}")
+    assert_same(scene, ctx.draw(scene), refcpu.draw(scene))
+
+
 def test_frames_sharing_objects(ctx):
     """Frames of a batch that name the same range of its object array."""
     import scene_cases as C
