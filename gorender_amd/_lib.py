@@ -173,6 +173,7 @@ SIGNATURES = {
     "gr_png_decode": (c_int32, [ctypes.c_char_p, POINTER(c_int32), POINTER(c_int32),
                                 POINTER(POINTER(ctypes.c_uint8))]),
     "gr_host_free": (None, [c_void_p]),
+    "gr_host_copy": (c_int32, [c_void_p, c_void_p, ctypes.c_size_t]),
     "gr_texture_load": (c_int32, [c_void_p, ctypes.c_char_p, POINTER(c_int32)]),
     "gr_check_exact_division": (c_int32, [c_void_p, ctypes.c_uint64, ctypes.c_uint64,
                                           POINTER(ctypes.c_uint64), POINTER(ctypes.c_float)]),

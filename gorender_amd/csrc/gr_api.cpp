@@ -1819,8 +1819,8 @@ gr_status gr_draw(gr_context* c, const gr_frame* frame, const gr_object* objs, i
                 continue;
             }
             if (st) return st;
-            if (rgba) std::memcpy(rgba, staged, npx * 4);
-            if (depth) std::memcpy(depth, staged + npx * 4, npx * 4);
+            if (rgba) gr_internal::host_copy(rgba, staged, npx * 4);
+            if (depth) gr_internal::host_copy(depth, staged + npx * 4, npx * 4);
             if (stats) {
                 std::vector<unsigned long long> sv;
                 if ((st = read_stats(c, sv))) return st;

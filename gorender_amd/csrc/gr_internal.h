@@ -33,6 +33,8 @@ void grow_refs_to(gr_context* c, unsigned long long needed);
 // and message a batch holding it would fail with.
 gr_status check_request(gr_context* c, const gr_frame* frame, const gr_object* objects,
                         int32_t num_objects);
+// Copy of host memory, shared by several threads when it is large (gr_copy.cpp).
+void host_copy(void* dst, const void* src, size_t n);
 // Keep every batch on pipe 0 (the serving loop overlaps its own readback).
 void set_one_pipe(gr_context* c, bool on);
 

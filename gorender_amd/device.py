@@ -6,6 +6,8 @@ scenes synchronously into numpy buffers or asynchronously into device memory.
 from __future__ import annotations
 
 import ctypes
+import sys
+import threading
 from typing import Dict, List, Optional, Sequence, Tuple
 
 import numpy as np
@@ -35,6 +37,61 @@ def frame_struct(fr: FrameData) -> _lib.gr_frame:
     return f
 
 
+class ResultArrays:
+    """Memory of the arrays that a context's frames are delivered in.
+
+    A fresh array of a frame's size costs more in page faults than the copy into
+    it, so memory whose last array is gone is used again: a block is free when
+    nothing but this pool refers to it (an array made of it, and every view of
+    that, keeps it as its base). Blocks number at most LIMIT bytes and are given
+    back when the context is closed."""
+
+    LIMIT = 256 << 20
+    LEAST = 256 << 10
+
+    def __init__(self):
+        self._lock = threading.Lock()
+        self._blocks: Dict[int, List[np.ndarray]] = {}
+        self._bytes = 0
+
+    def empty(self, dtype, shape) -> np.ndarray:
+        n = int(np.dtype(dtype).itemsize * np.prod(shape, dtype=np.int64))
+        if n < self.LEAST:
+            return np.empty(shape, dtype)
+        with self._lock:
+            for b in self._blocks.get(n, ()):
+                if sys.getrefcount(b) == 3:  # the list's, the loop's and the call's
+                    return b.view(dtype).reshape(shape)
+            if self._bytes + n > self.LIMIT:
+                self._drop_free(n)
+            if self._bytes + n > self.LIMIT:
+                return np.empty(shape, dtype)
+            b = np.empty(n, np.uint8)
+            self._blocks.setdefault(n, []).append(b)
+            self._bytes += n
+            return b.view(dtype).reshape(shape)
+
+    def copy_out(self, ptr, dtype, shape) -> np.ndarray:
+        """An array holding what the C pointer names (gr_host_copy)."""
+        out = self.empty(dtype, shape)
+        _lib.check(_lib.load().gr_host_copy(out.ctypes.data, ctypes.cast(ptr, ctypes.c_void_p),
+                                            out.nbytes))
+        return out
+
+    def _drop_free(self, keep: int) -> None:
+        """Forgets the free blocks of sizes other than `keep`."""
+        for n, blocks in self._blocks.items():
+            if n != keep:
+                used = [b for b in blocks if sys.getrefcount(b) > 3]
+                self._bytes -= n * (len(blocks) - len(used))
+                blocks[:] = used
+
+    def clear(self) -> None:
+        with self._lock:
+            self._blocks.clear()
+            self._bytes = 0
+
+
 class Context:
     """A gorender_hip context on one GPU."""
 
@@ -45,11 +102,13 @@ class Context:
         self.handle = h
         self._mesh_cache: Dict[int, int] = {}
         self._tex_cache: Dict[int, int] = {}
+        self.arrays = ResultArrays()
 
     def close(self) -> None:
         if self.handle:
             self.lib.gr_destroy(self.handle)
             self.handle = None
+            self.arrays.clear()
 
     def __enter__(self):
         return self
@@ -147,8 +206,8 @@ class Context:
             mesh_handles, _ = self.upload_scene(s)
         fr = frame_struct(s.frame)
         objs = self.objects_struct(s, mesh_handles)
-        rgba = np.empty((s.frame.height, s.frame.width, 4), np.uint8)
-        depth = np.empty((s.frame.height, s.frame.width), np.float32)
+        rgba = self.arrays.empty(np.uint8, (s.frame.height, s.frame.width, 4))
+        depth = self.arrays.empty(np.float32, (s.frame.height, s.frame.width))
         st = _lib.gr_stats()
         _lib.check(self.lib.gr_draw(self.handle, ctypes.byref(fr), objs, len(s.objects),
                                     _ptr(rgba), _ptr(depth), ctypes.byref(st)))
@@ -186,8 +245,8 @@ class Context:
         st = _lib.gr_stats()
         _lib.check(self.lib.gr_present_wait(self.handle, ctypes.byref(rp), ctypes.byref(dp),
                                             ctypes.byref(st)))
-        rgba = np.ctypeslib.as_array(rp, (height, width, 4)).copy()
-        depth = np.ctypeslib.as_array(dp, (height, width)).copy() if dp else None
+        rgba = self.arrays.copy_out(rp, np.uint8, (height, width, 4))
+        depth = self.arrays.copy_out(dp, np.float32, (height, width)) if dp else None
         return rgba, depth, st.as_dict()
 
     def prepare_batch(self, scenes: Sequence[SceneData], mesh_handles: Sequence[Sequence[int]],

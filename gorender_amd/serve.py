@@ -92,11 +92,9 @@ class Server:
         h, w = r.height, r.width
         rgba = depth = None
         if copy:
-            rgba = np.ctypeslib.as_array(ctypes.cast(r.rgba, ctypes.POINTER(ctypes.c_uint8)),
-                                         shape=(h, w, 4)).copy()
+            rgba = self.ctx.arrays.copy_out(r.rgba, np.uint8, (h, w, 4))
             if r.depth:
-                depth = np.ctypeslib.as_array(
-                    ctypes.cast(r.depth, ctypes.POINTER(ctypes.c_float)), shape=(h, w)).copy()
+                depth = self.ctx.arrays.copy_out(r.depth, np.float32, (h, w))
         out = ServeResult(rgba, depth, r.stats.as_dict(), r.submit_ns, r.start_ns, r.done_ns,
                           r.batch_size)
         self.release(ticket)

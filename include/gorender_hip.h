@@ -436,6 +436,10 @@ gr_status gr_server_replay(gr_server *server, const gr_frame *frames, const gr_o
                            int32_t num_distinct, const double *arrival_s, int32_t n,
                            int64_t *latency_ns, int32_t *batch_size);
 
+/* Copies host memory (a presented or served frame out of its pinned buffer); a
+ * large copy is shared by several threads of the library. */
+gr_status gr_host_copy(void *dst, const void *src, size_t bytes);
+
 /* ---- measurement ---- */
 /* When enabled, each kernel launch is bracketed by HIP events on the context
  * stream and its duration accumulated per kernel name. */

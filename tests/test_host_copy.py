@@ -1,0 +1,79 @@
+"""gr_host_copy and the arrays that frames are delivered in (no GPU needed)."""
+import threading
+
+import numpy as np
+import pytest
+
+from gorender_amd import _lib
+from gorender_amd.device import ResultArrays
+
+PIECE = 128 << 10
+SHARED = 512 << 10
+
+
+@pytest.mark.parametrize("n", [0, 1, PIECE, SHARED - 1, SHARED, SHARED + 1, 8 * PIECE + 3,
+                               (9 << 20) + 5])
+def test_host_copy(n):
+    """Below and above the shared size, of whole and of broken pieces; nothing
+    past the end is touched."""
+    src = np.random.default_rng(n).integers(0, 256, n + 1, dtype=np.uint8)
+    dst = np.zeros(n + 64, np.uint8)
+    _lib.check(_lib.load().gr_host_copy(dst.ctypes.data, src.ctypes.data, n))
+    assert np.array_equal(dst[:n], src[:n]) and not dst[n:].any()
+
+
+def test_host_copy_refuses_null():
+    with pytest.raises(_lib.GorenderError) as e:
+        _lib.check(_lib.load().gr_host_copy(None, None, 1))
+    assert e.value.status == _lib.GR_ERR_INVALID_ARGUMENT
+
+
+def test_host_copy_from_several_threads():
+    """Copies at once from four threads, most of which find the helpers taken."""
+    lib = _lib.load()
+    bad = []
+
+    def work(seed):
+        rng = np.random.default_rng(seed)
+        for k in range(40):
+            src = rng.integers(0, 256, SHARED + 1000 * k + seed, dtype=np.uint8)
+            dst = np.zeros_like(src)
+            _lib.check(lib.gr_host_copy(dst.ctypes.data, src.ctypes.data, src.nbytes))
+            if not np.array_equal(src, dst):
+                bad.append((seed, k))
+
+    threads = [threading.Thread(target=work, args=(s,)) for s in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+
+
+def test_result_arrays_reuse_only_what_is_free():
+    pool = ResultArrays()
+    a = pool.empty(np.float32, (512, 512))
+    at = a.ctypes.data
+    b = pool.empty(np.uint8, (512, 512, 4))
+    assert b.ctypes.data != at
+    view = a[100:]
+    del a
+    c = pool.empty(np.float32, (512, 512))
+    assert c.ctypes.data not in (at, b.ctypes.data)  # a view is still in use
+    del view
+    d = pool.empty(np.float32, (1024, 256))
+    assert d.ctypes.data == at and d.dtype == np.float32 and d.shape == (1024, 256)
+
+
+def test_result_arrays_are_bounded():
+    pool = ResultArrays()
+    pool.LIMIT = 4 << 20
+    held = [pool.empty(np.uint8, (1 << 20,)) for _ in range(6)]
+    assert pool._bytes == 4 << 20
+    assert len({h.ctypes.data for h in held}) == 6
+    del held
+    other = pool.empty(np.uint8, (3 << 20,))  # free blocks of another size make room
+    assert pool._bytes == 3 << 20 and other.nbytes == 3 << 20
+    assert pool.empty(np.uint8, (10,)).base is None  # small arrays are their own
+    pool.clear()
+    other[:] = 1
