@@ -1,4 +1,6 @@
 """gr_host_copy and the arrays that frames are delivered in (no GPU needed)."""
+import os
+import signal
 import threading
 
 import numpy as np
@@ -77,3 +79,18 @@ def test_result_arrays_are_bounded():
     assert pool.empty(np.uint8, (10,)).base is None  # small arrays are their own
     pool.clear()
     other[:] = 1
+
+
+def test_host_copy_in_a_forked_child():
+    """The helper threads stay in the process that started them."""
+    lib = _lib.load()
+    src = np.random.default_rng(3).integers(0, 256, 8 << 20, dtype=np.uint8)
+    dst = np.zeros_like(src)
+    _lib.check(lib.gr_host_copy(dst.ctypes.data, src.ctypes.data, src.nbytes))
+    pid = os.fork()
+    if pid == 0:
+        signal.alarm(20)
+        dst[:] = 0
+        ok = lib.gr_host_copy(dst.ctypes.data, src.ctypes.data, src.nbytes) == 0
+        os._exit(0 if ok and np.array_equal(src, dst) else 1)
+    assert os.waitpid(pid, 0)[1] == 0
