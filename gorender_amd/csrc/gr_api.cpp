@@ -466,7 +466,7 @@ gr_status make_plan(gr_context* c, const gr_batch_frame* bf, int nf, const gr_ob
         d.face_color = pack_rgba(fr.face_color);
         d.clear_color = pack_rgba(fr.clear_color);
         d.dot_color = pack_rgba(fr.dot_color);
-        d.dot_step = fr.dot_step;
+        d.dot_inv = fr.dot_step >= 1 ? 0xFFFFFFFFu / (uint32_t)fr.dot_step : 0u;
         // The grid is a product: x bounds from tile % n, y bounds from tile / n.
         const int ng = fr.ref_tiles == 16 ? 4 : 1;
         for (int g = 0; g < 4; g++) {

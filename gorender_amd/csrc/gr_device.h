@@ -99,7 +99,7 @@ struct DevFrame {
     float light[3];
     float ambient, diffuse, znear, zfar;
     uint32_t face_color, clear_color, dot_color;
-    int32_t dot_step;
+    uint32_t dot_inv;  // floor((2^32 - 1) / step) of the dot grid, 0 for none
     // Reference TPF grid (renderer.go:50-76): first and last x of its columns, y of
     // its rows; NaN past a 1x1 grid's first.
     float ref_cols[4][2], ref_rows[4][2];

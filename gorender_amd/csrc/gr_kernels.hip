@@ -73,6 +73,10 @@ __device__ __forceinline__ int64_t wmul(int64_t a, int64_t b) {
     return (int64_t)((uint64_t)a * (uint64_t)b);
 }
 
+// Lanes of the wave for which p holds, as the compare's own mask (__ballot makes an
+// integer of p and compares that: two more vector instructions).
+__device__ __forceinline__ uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+
 // Load and store of one value through a global-address-space pointer: the
 // pointers of DevFrame and DevMesh are generic, and a generic (flat) access
 // also counts against the LDS wait counter, so a later LDS wait would wait for
@@ -258,12 +262,12 @@ __device__ __forceinline__ int wave_last_le(const T* key, int n, T b) {
     while (len > 64) {
         const int step = (len + 63) >> 6;
         const bool le = lane * step < len && gld(&key[lo + lane * step]) <= b;
-        const int k = __popcll(__ballot(le)) - 1;
+        const int k = __popcll(ballot(le)) - 1;
         lo += k * step;
         len = min(step, len - k * step);
     }
     const bool le = lane < len && gld(&key[lo + lane]) <= b;
-    return lo + __popcll(__ballot(le)) - 1;
+    return lo + __popcll(ballot(le)) - 1;
 }
 
 // Workgroup h -> (frame, unit within the frame) in the XCD-aware order: the
@@ -290,7 +294,7 @@ __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v)
 // case (the raster's covered-fragment count is wave-uniform except on the
 // int64 path): the full reduction runs only when another lane holds a count.
 __device__ __forceinline__ unsigned long long wave_total(unsigned long long v, int lane) {
-    if (__ballot(v != 0ull && lane != 0) == 0ull)
+    if (ballot(v != 0ull && lane != 0) == 0ull)
         return __builtin_amdgcn_readfirstlane((unsigned)v) |
                ((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(v >> 32)) << 32);
     return wave_sum_u64(v);
@@ -394,7 +398,7 @@ __device__ int wave_clip(CV* buf0, CV* buf1, const CV& a, const CV& b, const CV&
         const bool ib = act && inside(P, N, B);
         const bool one = ia || ib;     // at least one output vertex
         const bool two = ia && !ib;    // [X, A]
-        const uint64_t b1 = __ballot(one), b2 = __ballot(two);
+        const uint64_t b1 = ballot(one), b2 = ballot(two);
         const uint64_t lt = lanemask_lt(lane);
         const int pos = __popcll(b1 & lt) + __popcll(b2 & lt);
         const int m = __popcll(b1) + __popcll(b2);
@@ -926,8 +930,10 @@ __device__ __forceinline__ uint32_t block_rec(uint32_t gb, uint32_t ovf, uint32_
 // past its own range).
 __device__ __forceinline__ uint32_t rec_index(const DevFrame& fr, uint32_t slot) {
     const uint32_t blk = slot / (uint32_t)kSlotsPerWg, off = slot % (uint32_t)kSlotsPerWg;
+    // blk is below 2^32 / kSlotsPerWg: a 24-bit product.
     return off < (uint32_t)kRecsPerBlock
-               ? ((uint32_t)fr.face_block_begin + blk) * (uint32_t)kRecsPerBlock + off
+               ? __umul24(blk, (uint32_t)kRecsPerBlock) +
+                     (uint32_t)fr.face_block_begin * (uint32_t)kRecsPerBlock + off
                : gld(&fr.blocks[blk].ovf) + (off - (uint32_t)kRecsPerBlock);
 }
 
@@ -1109,7 +1115,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
         if (w > 0 && n <= kLaneTiles)
             for (int ty = t.ty0; ty <= t.ty1; ty++)
                 for (int tx = t.tx0; tx <= t.tx1; tx++) add((uint32_t)(ty * fr.tiles_x + tx));
-        for (uint64_t big = __ballot(w > 0 && n > kLaneTiles); big; big &= big - 1) {
+        for (uint64_t big = ballot(w > 0 && n > kLaneTiles); big; big &= big - 1) {
             const int L = __builtin_ctzll(big);
             wave_rect(__builtin_amdgcn_readlane(t.tx0, L), __builtin_amdgcn_readlane(t.ty0, L),
                       __builtin_amdgcn_readlane(t.tx1, L), __builtin_amdgcn_readlane(t.ty1, L),
@@ -1169,11 +1175,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
                 p = __builtin_ctz(~all_in | 0x40u);
                 survivor = !(p < 6 && !(((m0 | m1 | m2) >> p) & 1u));
             }
-            const uint64_t sm = __ballot(survivor);
+            const uint64_t sm = ballot(survivor);
             if (survivor)
                 W.sface[nsurv + __popcll(sm & lanemask_lt(lane))] = (uint32_t)fo | ((uint32_t)p << 8);
             nsurv += __popcll(sm);
-            nrec += (uint32_t)__popcll(sm) + (kMaxFan - 1) * (uint32_t)__popcll(__ballot(survivor && p < 6));
+            nrec += (uint32_t)__popcll(sm) + (kMaxFan - 1) * (uint32_t)__popcll(ballot(survivor && p < 6));
         }
     }
     wave_sync();
@@ -1302,7 +1308,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
         // once. The prefix of the fan sizes (0, 1, 2 or kMaxFan) in face order
         // is counted from three ballots.
         if (mode == 2) n = kMaxFan;
-        const uint64_t b1 = __ballot(n == 1), b2 = __ballot(n == 2), b7 = __ballot(n == kMaxFan);
+        const uint64_t b1 = ballot(n == 1), b2 = ballot(n == 2), b7 = ballot(n == kMaxFan);
         const uint64_t lt = lanemask_lt(lane);
         // The lane's slots start at offset off of the block's.
         uint32_t total;
@@ -1322,7 +1328,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
                                            box));
             count(box);
             emit = mode == 3 && nq == 4;
-            if (t == 1 || !__ballot(emit)) break;
+            if (t == 1 || !ballot(emit)) break;
             if (emit) {
                 q[1] = q[2];
                 q[2] = q[3];
@@ -1335,7 +1341,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
         // (clipping.go:44-62) or an empty record.
         CV* buf0 = W.poly[0];
         CV* buf1 = W.poly[1];
-        for (uint64_t gen = __ballot(mode == 2); gen;) {
+        for (uint64_t gen = ballot(mode == 2); gen;) {
             int nst = 0;
             for (; gen && nst < kStage; gen &= gen - 1, nst++) {
                 const int L = __builtin_ctzll(gen);
@@ -1640,7 +1646,7 @@ __global__ __launch_bounds__(kScanThreads) void k_bin_scan(
         else
             v = i < ntiles ? gld(&cnt[i]) : 0u;
         const bool split = !over && v > part_refs;
-        const uint64_t sm = __ballot(split);
+        const uint64_t sm = ballot(split);
         const unsigned long long x = wave_scan_u64(v);
         const uint32_t sv = split ? v : 0u;
         const uint32_t xi = sm ? wave_scan_u32(sv) : 0u;
@@ -1676,7 +1682,7 @@ __global__ __launch_bounds__(kScanThreads) void k_bin_scan(
                 if (slab < max_slabs) split_tile[slab] = tile;
                 tile_slab[tile] = slab < max_slabs ? slab : kNoSlab;
             }
-            const uint64_t cm = __ballot(split && slab < max_slabs && v > split_refs);
+            const uint64_t cm = ballot(split && slab < max_slabs && v > split_refs);
             if (cm && lane == 0)
                 atomicAdd(&stats[f * kNumStats + kStatSplit], (unsigned long long)__popcll(cm));
         }
@@ -1764,7 +1770,7 @@ __global__ __launch_bounds__(kFillThreads) void k_bin_fill(const DevFrame* __res
                     if (m > 0 && m <= kLaneTiles)
                         for (int ty = y0; ty <= y1; ty++)
                             for (int tx = x0; tx <= x1; tx++) fn((ty - wy) * ww + tx - wx, i);
-                    for (uint64_t big = __ballot(m > kLaneTiles); big; big &= big - 1) {
+                    for (uint64_t big = ballot(m > kLaneTiles); big; big &= big - 1) {
                         const int L = __builtin_ctzll(big);
                         const uint32_t bi = (uint32_t)__builtin_amdgcn_readlane((int)i, L);
                         wave_rect(__builtin_amdgcn_readlane(x0, L) - wx,
@@ -1891,12 +1897,50 @@ __device__ __forceinline__ uint32_t sample(const DevTexture& t, float u, float v
     }
 }
 
+// |v| % m for |v| < 2^20, 0 < m < 2^31 and rm = RN(1 / m) or a neighbour, with v's
+// sign: go_int_rem of such a v. The quotient's error is below 2^20 * 3 * 2^-24, so
+// its floor is one off at most, and one of the two additions sets that right.
+__device__ __forceinline__ int32_t rem_small(float v, uint32_t m, float rm) {
+    const float a = __builtin_fabsf(v);
+    // A quotient above 0 has m <= 2^20: a 24-bit product.
+    uint32_t r = (uint32_t)a - (uint32_t)__umul24((uint32_t)(a * rm), m);
+    r = min(r, r + m);
+    r = min(r, r - m);
+    return v < 0.f ? -(int32_t)r : (int32_t)r;
+}
+
+// sample() for a texture the wave shares, with its descriptor in scalar registers.
+__device__ __forceinline__ uint32_t sample_shared(const DevTexture& t, float u, float v) {
+    typedef const __attribute__((address_space(1))) char* gbytes;
+    const float fx = (1 - u) * t.scale * t.wf, fy = v * t.scale * t.hf;
+    if (t.type == 2) {
+        // Sides are powers of two, at most 2^28 texels.
+        const uint32_t x = (uint32_t)go_int_lo(fx) & (uint32_t)(t.w - 1);
+        const uint32_t y = (uint32_t)go_int_lo(fy) & (uint32_t)(t.h - 1);
+        const uint32_t at = ((y << __builtin_ctz((uint32_t)t.w)) + x) << 2;
+        return *(const __attribute__((address_space(1))) uint32_t*)((gbytes)t.texels + at);
+    }
+    if (t.type == 1 &&
+        ballot(!(__builtin_fabsf(fx) < 1048576.f && __builtin_fabsf(fy) < 1048576.f)) == 0ull) {
+        const int32_t x = rem_small(fx, (uint32_t)t.w, __builtin_amdgcn_rcpf(t.wf));
+        const int32_t y = rem_small(fy, (uint32_t)t.h, __builtin_amdgcn_rcpf(t.hf));
+        const uint32_t at = (uint32_t)max(y * t.w + x, 0) << 2;
+        return *(const __attribute__((address_space(1))) uint32_t*)((gbytes)t.texels + at);
+    }
+    return sample(t, u, v);
+}
+
 // rasterizer.go:81-88
 __device__ __forceinline__ uint32_t color_intensity(uint32_t c, float k) {
-    uint32_t r = go_uint8((float)(c & 0xFFu) * k);
-    uint32_t g = go_uint8((float)((c >> 8) & 0xFFu) * k);
-    uint32_t b = go_uint8((float)((c >> 16) & 0xFFu) * k);
-    return r | (g << 8) | (b << 16) | (c & 0xFF000000u);
+    const float r = (float)(c & 0xFFu) * k, g = (float)((c >> 8) & 0xFFu) * k,
+                b = (float)((c >> 16) & 0xFFu) * k;
+    if (ballot(!(__builtin_fabsf(k) < 8388608.f)) == 0ull) {
+        // Every product of the wave is within int32: the low bytes of the
+        // conversions, put together by byte selects.
+        const uint32_t rg = __builtin_amdgcn_perm((uint32_t)(int32_t)g, (uint32_t)(int32_t)r, 0x0C0C0400u);
+        return rg | __builtin_amdgcn_perm(c, (uint32_t)(int32_t)b, 0x07000C0Cu);
+    }
+    return go_uint8(r) | (go_uint8(g) << 8) | (go_uint8(b) << 16) | (c & 0xFF000000u);
 }
 
 // The raster stage reads a staged RasterRec as five 16-byte pieces: divisors,
@@ -1930,7 +1974,7 @@ __device__ __forceinline__ void frag_depth(const uint32_t (*q)[128], uint32_t he
                                       __uint_as_float(rc.z), __uint_as_float(rc.w));
         // Almost every triangle has reciprocals: when all of the wave's do, the
         // branch is taken once for the wave instead of per lane.
-        const Bary b = __ballot(rf.x == 0.f) == 0ull ? bary_rcp((float)f12, (float)f20, df, rf)
+        const Bary b = ballot(rf.x == 0.f) == 0ull ? bary_rcp((float)f12, (float)f20, df, rf)
                                                       : bary((float)f12, (float)f20, df, rf);
         if (b.zrec >= -1.0f) atomicMax(&key[px_idx], depth_key(b.zrec, lslot[i] + 1u));
     }
@@ -2088,7 +2132,7 @@ __device__ __forceinline__ unsigned long long raster_list(
             // they go to the wave's ring by ballot, and every 64 queued
             // fragments get their exact depth.
             auto step = [&](int all, int g1, int g2, uint32_t pk) {
-                const uint64_t mask = __ballot(all < 0);
+                const uint64_t mask = ballot(all < 0);
                 if (mask) {
                     if (all < 0) {
                         const uint32_t k =
@@ -2141,34 +2185,44 @@ __device__ __forceinline__ unsigned long long raster_list(
 // Deferred shading of the winning fragment of each pixel of the tile, one
 // write per pixel. Returns the wave's count of shaded pixels.
 //
-// Background colours are read as values and the dot test is evaluated
-// without short-circuit branches: hipcc 7.2 (clang 22) turned the
-// short-circuit form into a select of field addresses that dropped the
-// y % step condition when the loop runs once per thread.
+// k_raster is bound by the issue of vector instructions where frames are many (93%
+// of its cycles for 32 frames of 1280x720), so a pixel's are kept few: one
+// reciprocal for u and v, indices of a shared texture by shift or by a reciprocal
+// of its side, colour bytes put together by byte selects, 32-bit offsets, and the
+// dot grid by one product. 32 frames of 200,000 triangles: k_raster 301 -> 294 us;
+// 64 mixed frames: 516 -> 505.
 template <int TW, int TH>
 __device__ __forceinline__ unsigned long long shade_tile(const DevFrame& fr, int X0, int Y0,
                                                          const unsigned long long* key,
                                                          const DevTexture* __restrict__ textures) {
     constexpr int NPX = TW * TH;
+    static_assert(256 % TW == 0, "a thread keeps its column");
     const uint32_t dot_color = fr.dot_color, clear_color = fr.clear_color;
-    const int step = fr.dot_step;
-    const int step1 = step >= 1 ? step : 1;
-    unsigned long long shaded = 0;  // wave-uniform
-    for (int i = threadIdx.x; i < NPX; i += 256) {
-        const int x = X0 + (i % TW), y = Y0 + (i / TW);
+    const int x = X0 + (int)(threadIdx.x % TW);
+    int y = Y0 + (int)(threadIdx.x / TW);
+    // DotGrid (rasterizer.go:46-52): x, y in {step, 2*step, ...}, the multiples of
+    // step but 0. n is one iff n * (dot_inv + 1) mod 2^32 <= dot_inv, dot_inv =
+    // floor((2^32 - 1) / step), for the n < 2^14 of a frame (with n = k * step + r
+    // and step * (dot_inv + 1) = 2^32 + e, 0 <= e < step, the product is
+    // k * e + r * (dot_inv + 1), and k * e <= n < dot_inv; a step above n has
+    // k = 0); dot_inv 0, of no grid, takes 0 alone.
+    const uint32_t dot_inv = fr.dot_inv;
+    const bool dot_x = x != 0 && (uint32_t)x * (dot_inv + 1u) <= dot_inv;
+    uint32_t dot_y = (uint32_t)y * (dot_inv + 1u);
+    uint32_t at = ((uint32_t)y * (uint32_t)fr.W + (uint32_t)x) << 2;  // below 2^30
+    typedef __attribute__((address_space(1))) char* gbytes;
+    uint32_t shaded = 0;  // wave-uniform
+    for (int i = threadIdx.x; i < NPX; i += 256, y += 256 / TW, dot_y += (256 / TW) * (dot_inv + 1u),
+             at += (uint32_t)fr.W * (uint32_t)(256 / TW * 4)) {
         const bool inframe = x < fr.W && y < fr.H;
         const unsigned long long k = key[i];
         const uint32_t seq = (uint32_t)k;
-        shaded += (unsigned long long)__popcll(__ballot(inframe && seq != 0u));
+        shaded += (uint32_t)__popcll(ballot(inframe && seq != 0u));
         if (!inframe) continue;
         uint32_t color;
         float depth;
         if (seq == 0u) {
-            // DotGrid (rasterizer.go:46-52): x, y in {step, 2*step, ...}
-            const uint32_t dot = (uint32_t)(step >= 1) & (uint32_t)(x >= step) &
-                                 (uint32_t)(y >= step) & (uint32_t)(x % step1 == 0) &
-                                 (uint32_t)(y % step1 == 0);
-            color = dot ? dot_color : clear_color;
+            color = dot_x && y != 0 && dot_y <= dot_inv ? dot_color : clear_color;
             depth = -1.0f;
         } else {
             const uint32_t ri = rec_index(fr, seq - 1u);
@@ -2188,9 +2242,11 @@ __device__ __forceinline__ unsigned long long shade_tile(const DevFrame& fr, int
             const float zkey = __uint_as_float((ord & 0x80000000u) ? (ord & 0x7FFFFFFFu) : ~ord);
             // rsf is 0 or kShadeWide (IEEE division) unless the raster record
             // holds reciprocals.
-            const bool common = zkey != 0.0f && s.rsf != 0u && s.rsf != kShadeWide;
+            const bool common = __builtin_fabsf(zkey) >= 0x1p-41f && __builtin_fabsf(zkey) <= 0x1p42f &&
+                                s.rsf != 0u && s.rsf != kShadeWide;
+            const bool fast = ballot(!common) == 0ull;
             Bary b;
-            if (__ballot(!common) == 0ull) {
+            if (fast) {
                 // Every pixel of the wave: int32 edge values, reciprocals, and
                 // zRec from the key (one branch for the wave, not per lane).
                 const float rsf = __uint_as_float(s.rsf);
@@ -2223,12 +2279,12 @@ __device__ __forceinline__ unsigned long long shade_tile(const DevFrame& fr, int
                 }
             }
             // rasterizer.go:158-170
-            float u = (b.alpha * s.uz[0] + b.beta * s.uz[1] + b.gamma * s.uz[2]) / b.zrec;
-            float v = (b.alpha * s.vz[0] + b.beta * s.vz[1] + b.gamma * s.vz[2]) / b.zrec;
-            float inten = b.alpha * s.in[0] + b.beta * s.in[1] + b.gamma * s.in[2];
+            const float un = b.alpha * s.uz[0] + b.beta * s.uz[1] + b.gamma * s.uz[2];
+            const float vn = b.alpha * s.vz[0] + b.beta * s.vz[1] + b.gamma * s.vz[2];
+            const float inten = b.alpha * s.in[0] + b.beta * s.in[1] + b.gamma * s.in[2];
             uint32_t c;
             const int tex0 = sgpr(s.tex);
-            if (__ballot(s.tex != tex0) == 0ull) {
+            if (ballot(s.tex != tex0) == 0ull) {
                 // One texture (or none) for the wave's pixels: its descriptor
                 // is read once, with scalar loads.
                 if (tex0 < 0) {
@@ -2242,26 +2298,45 @@ __device__ __forceinline__ unsigned long long shade_tile(const DevFrame& fr, int
                     for (int k = 0; k < 10; k++) w[k] = src[k];
                     DevTexture t;
                     __builtin_memcpy(&t, w, sizeof(DevTexture));
-                    c = sample(t, u, v);
+                    float u, v;
+                    if (fast && __builtin_fabsf(t.scale) >= 0x1p-40f && __builtin_fabsf(t.scale) <= 0x1p10f) {
+                        // Both quotients from one reciprocal: what the compiler
+                        // makes of a division (reciprocal, one Newton step, two
+                        // residual corrections, all fused) without its scaling
+                        // and its special cases, which do nothing for z in
+                        // [2^-41, 2^42] and |numerator| in [2^-80, 2^86]. Below,
+                        // |u| < 2^-38: 1 - u is 1, and v * scale * h is under 1
+                        // either way. Above, a quotient is the same one, or at
+                        // least 2^127, infinite or a NaN, and so past int64 once
+                        // scaled, in both ways.
+                        const float y0 = __builtin_amdgcn_rcpf(b.zrec);
+                        const float y1 = __builtin_fmaf(__builtin_fmaf(-b.zrec, y0, 1.0f), y0, y0);
+                        u = div_rcp(un, b.zrec, y1);
+                        v = div_rcp(vn, b.zrec, y1);
+                    } else {
+                        u = un / b.zrec;
+                        v = vn / b.zrec;
+                    }
+                    c = sample_shared(t, u, v);
                 }
             } else {
-                c = s.tex < 0 ? fr.face_color : sample(textures[s.tex], u, v);
+                c = s.tex < 0 ? fr.face_color : sample(textures[s.tex], un / b.zrec, vn / b.zrec);
             }
             color = color_intensity(c, inten);
             depth = b.zrec;
         }
-        const size_t idx = (size_t)y * fr.W + x;
         if (fr.okey) {
             // Overlay keys are zero between draws: each pixel's is read once.
-            const uint32_t ok = gld(&fr.okey[idx]);
+            uint32_t* const o = fr.okey + (at >> 2);
+            const uint32_t ok = gld(o);
             if (ok) {
-                gst(&fr.okey[idx], 0u);
+                gst(o, 0u);
                 if ((ok >> 1) >= seq)
                     color = (ok & 1u) ? kVertexColor : ((fr.flags & kShowFaces) ? kEdgeColor : kWhite);
             }
         }
-        gst(&((uint32_t*)fr.rgba)[idx], color);
-        gst(&fr.depth[idx], depth);
+        *(__attribute__((address_space(1))) uint32_t*)((gbytes)fr.rgba + at) = color;
+        *(__attribute__((address_space(1))) float*)((gbytes)fr.depth + at) = depth;
     }
     return shaded;
 }

@@ -422,3 +422,25 @@ def test_overflow_records(ctx):
     finally:
         ctx.set_config(refs_capacity=old.refs_capacity)
     assert_same(scene, got, want)
+
+
+@pytest.mark.parametrize("side,kind,scale,stretch,step", [
+    ((64, 16), 2, 1.0, 1.0, 1), ((16, 64), 2, 3.5, 40.0, 7), ((1, 1), 2, 1.0, 5.0, 333),
+    ((100, 37), 1, 1.0, 1.0, 10), ((100, 37), 1, 2.5, -9.0, 2), ((1, 3), 1, 1.0, 2000.0, 64),
+    ((17, 17), 1, 1.0, 3e5, 3), ((17, 17), 1, 1024.0, 1.0, 2**31 - 1), ((17, 17), 1, 1025.0, 1.0, 0),
+    ((64, 64), 2, 1e-13, 1e20, -5), ((17, 17), 1, 0.0, 1e30, 65), ((17, 17), 1, -2.0, 1e-30, 64),
+    ((64, 64), 2, 1.0, 1e30, 63), ((17, 17), 1, 1.0, float("inf"), 16), ((64, 64), 2, 1.0, 0.0, 32)])
+def test_shading_forms(ctx, side, kind, scale, stretch, step):
+    """Texture sides, scales and coordinates on both sides of the shortened
+    quotient, remainder and index, and steps of the dot grid."""
+    import scene_cases as C
+    scene = C.sphere(w=200, h=130, eye=(0, 0, 1.6), nlat=14, nlon=22)
+    w, h = side
+    rgba = np.random.default_rng(5).integers(0, 256, (h, w, 4), dtype=np.uint8)
+    scene.textures[:] = [S.TextureData(kind, w, h, scale, rgba=rgba)] * len(scene.textures)
+    mesh = scene.meshes[0]
+    with np.errstate(invalid="ignore"):
+        mesh.uvs = (np.asarray(mesh.uvs) * np.float32(stretch)).astype(np.float32)
+    scene.frame.dot_step = step
+    with np.errstate(invalid="ignore"):
+        assert_same(scene, ctx.draw(scene), refcpu.draw(scene))
