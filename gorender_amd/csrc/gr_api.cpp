@@ -401,7 +401,7 @@ gr_status check_frame(gr_context* c, const gr_frame& fr, const gr_object* objs, 
 // place of buffer pointers), the header layout and the sizes of the per-batch
 // buffers. Objects must be laid out frame by frame.
 struct Plan {
-    int nf = 0, nobj = 0, fblocks = 0, tiles = 0;
+    int nf = 0, nobj = 0, fblocks = 0, dense_blocks = 0, tiles = 0;
     int twl = 0, thl = 0;
     size_t okey_words = 0;
     bool decorate = false;  // a frame asks for tile borders or the crosshair
@@ -514,6 +514,7 @@ gr_status make_plan(gr_context* c, const gr_batch_frame* bf, int nf, const gr_ob
             o.face_block = P.fblocks;
             o.seq_block = seq;
             P.fblocks += o.face_blocks;
+            if (o.dense) P.dense_blocks += o.face_blocks;
             seq += o.face_blocks;
         }
         d.face_blocks = P.fblocks - d.face_block_begin;
@@ -646,6 +647,10 @@ gr::LaunchParams launch_params(const Plan& P, const Bufs& B) {
     p.slab_done = B.slab_done;
     p.max_slabs = B.max_slabs;
     p.part_refs = B.part_refs;
+    // Half of the faces in dense meshes, in a launch whose tiles fill the chip (the
+    // lists of a smaller one are cut into parts of 64, which end no sooner: 1,000,000
+    // faces in one 1080p frame, k_raster 36.5 -> 38.2 us).
+    p.dense = P.tiles > kFineTiles && 2ll * P.dense_blocks >= P.fblocks;
     p.split_refs = B.split_refs;
     p.frame_overflow = (uint32_t*)(bb + P.off_over);
     p.blocks = B.blocks;

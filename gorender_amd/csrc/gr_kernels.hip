@@ -1987,14 +1987,21 @@ __device__ __forceinline__ void frag_depth(const uint32_t (*q)[128], uint32_t he
 // the per-wave fragment rings and the stats reduction.
 constexpr int kRasterChunk = 64;
 constexpr int kRasterLdsFixed = kRasterChunk * (80 + 4) + 4 * 3 * 128 * 4 + 4 * 2 * 8 + 16;
+constexpr int kStartWords = kRasterChunk + 2;  // of a dense workgroup, 8 bytes each
 
 // Waves per SIMD the tile's LDS allows (one wave per SIMD per workgroup), at
 // most 8: the register budget follows from it (512 / waves VGPRs).
-constexpr int raster_waves(int npx) {
-    return (160 * 1024) / (npx * 8 + kRasterLdsFixed) >= 8
-               ? 8
-               : (160 * 1024) / (npx * 8 + kRasterLdsFixed);
+constexpr int raster_waves(int npx, bool dense = false) {
+    const int lds = npx * 8 + kRasterLdsFixed + (dense ? kStartWords * 8 : 0);
+    return (160 * 1024) / lds >= 8 ? 8 : (160 * 1024) / lds;
 }
+
+// Boxes walked by their pixels in dense lists, and how many of a chunk's 64 make
+// it one. 8 requests of 500,000 faces, k_raster: 369 us with (64, 24), 382 (64, 40),
+// 389 (32, 24), 406 (32, 40), 425 (16, 40), 436 with each box walked on its own.
+constexpr uint32_t kSmallBox = 64;
+constexpr int kSmallBoxes = 24;
+static_assert(kRasterChunk * kSmallBox <= 64 * kRasterChunk, "a start word per 64 candidates");
 
 // Walk form of a record for one tile (piece 2 of the staged record): the box
 // clamped to the tile as one word (x0 - X0 | y0 - Y0 << 6 | x1 - x0 << 12 |
@@ -2029,11 +2036,21 @@ __device__ __forceinline__ uint4 walk_form(const uint4& w2, const uint4& w3, con
 // Resolves n tile-list entries (slots) into the tile's depth keys: the
 // visibility part of rasterizer.go:139-156 for every listed triangle. Returns
 // this lane's share of the covered-fragment count (summed over the wave).
-template <int TW, int TH>
+//
+// Each record's box is walked by a wave, 64 pixels a step: right where boxes are
+// large. Dense lists hold boxes of a few pixels, which leave most lanes idle
+// (some 30 vector instructions for 1 to 5 pixels). DENSE puts the pixels of a
+// chunk's small boxes end to end and tests 64 of them a step, whichever records
+// they are of: 8 requests of 500,000 faces, k_raster 430 -> 360 us. Its registers
+// and set-up cost sparse lists 4% (32 frames of 200,000 triangles 295 -> 307 us,
+// 1,000,000 faces of instances in one frame 36.5 -> 38.2), so it is a variant.
+// Lanes by record, or four lanes a record, were slower: the largest box of the
+// wave sets the steps.
+template <int TW, int TH, bool DENSE>
 __device__ __forceinline__ unsigned long long raster_list(
     const DevFrame& fr, int X0, int Y0, const uint32_t* __restrict__ list, uint32_t cnt,
-    unsigned long long* key, uint4* lrec, uint32_t* lslot, uint32_t (*q)[128], int lane,
-    int wave) {
+    unsigned long long* key, uint4* lrec, uint32_t* lslot, uint32_t (*q)[128],
+    unsigned long long* starts, int lane, int wave) {
     constexpr int CHUNK = kRasterChunk;  // triangles staged in LDS at a time
     static_assert(TW * TH <= 4096 && CHUNK <= (1 << 20),
                   "fragment codes hold the pixel index in 12 bits");
@@ -2050,6 +2067,7 @@ __device__ __forceinline__ unsigned long long raster_list(
         // than once per record in every wave's scalar unit).
         __syncthreads();
         if (threadIdx.x < n) lslot[threadIdx.x] = list[base + threadIdx.x];
+        if (DENSE && wave == 3) starts[lane] = 0ull;
         __syncthreads();
         {
             const uint32_t t = threadIdx.x & 63u;
@@ -2061,17 +2079,108 @@ __device__ __forceinline__ unsigned long long raster_list(
                     const uint4 w2 = gload(src + 2), w3 = gload(src + 3), w4 = gload(src + 4);
                     lrec[t * 5 + 2] = walk_form<TW, TH>(w2, w3, w4, X0, Y0);
                     lrec[t * 5 + 3] = make_uint4(w2.w, w3.z, w4.y, w3.x);  // A01 A12 A20 B01
-                    lrec[t * 5 + 4] = make_uint4(w3.w, w4.z, 0u, 0u);      // B12 B20
+                    if (DENSE) {
+                        *reinterpret_cast<uint2*>(&lrec[t * 5 + 4]) = make_uint2(w3.w, w4.z);
+                    } else {
+                        lrec[t * 5 + 4] = make_uint4(w3.w, w4.z, 0u, 0u);  // B12 B20
+                    }
+                }
+            }
+            if (DENSE && wave == 0) {
+                // Small boxes: their first candidates, and a bit at each in
+                // starts; a box walked on its own has one candidate, of width 0.
+                const uint32_t info = t < n ? lrec[t * 5 + 2].x : 0u;
+                const uint32_t bw = ((info >> 12) & 63u) + 1u;
+                const uint32_t area = bw * ((info >> 18) & 127u);
+                uint64_t small = ballot(area != 0u && area <= kSmallBox && !(info & kWalkWide));
+                uint32_t end = 0u;
+                if (__popcll(small) >= kSmallBoxes) {
+                    const bool sm = (small >> lane) & 1u;
+                    const uint32_t cand = t < n ? (sm ? area : 1u) : 0u;
+                    end = wave_scan_u32(cand);
+                    if (t < n) {
+                        const uint32_t at = end - cand;
+                        const uint32_t px = ((info >> 6) & 63u) * (uint32_t)TW + (info & 63u);
+                        // First candidate | first pixel << 16, 2^16 / width (from
+                        // above, exact for 64 pixels) | width << 20.
+                        *(reinterpret_cast<uint2*>(&lrec[t * 5 + 4]) + 1) = make_uint2(
+                            at | px << 16,
+                            ((uint32_t)(65536.f * __builtin_amdgcn_rcpf((float)bw)) + 1u) |
+                                (sm ? bw << 20 : 0u));
+                        atomicOr(reinterpret_cast<uint32_t*>(starts) + (at >> 5), 1u << (at & 31u));
+                    }
+                } else {
+                    small = 0ull;
+                }
+                const uint64_t own = ballot(area != 0u) & ~small;
+                if (lane == 63) {
+                    starts[kRasterChunk] = own;
+                    starts[kRasterChunk + 1] = end;
                 }
             }
         }
         __syncthreads();
+        // Lanes with all < 0 hold an inside fragment (every edge value < 0,
+        // rasterizer.go:147, and the pixel inside the box); they go to the wave's
+        // LDS ring by ballot, and every 64 queued fragments get their exact depth
+        // on a full wave.
+        uint32_t qhead = 0, qtail = 0;  // wave-uniform ring positions
+        auto step = [&](int all, int g1, int g2, uint32_t pk) {
+            const uint64_t mask = ballot(all < 0);
+            if (mask) {
+                if (all < 0) {
+                    const uint32_t k =
+                        __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)mask, qtail)) &
+                        127u;
+                    q[0][k] = pk;
+                    q[1][k] = (uint32_t)g1;
+                    q[2][k] = (uint32_t)g2;
+                }
+                const uint32_t m = (uint32_t)__popcll(mask);
+                qtail += m;
+                covered_wave += m;
+                if (qtail - qhead >= 64u) {
+                    frag_depth<TW>(q, qhead, 64u, lrec, lslot, key, lane);
+                    qhead += 64u;
+                }
+            }
+        };
+        uint64_t own = 0;  // DENSE: the wave's records still to be walked
+        if (DENSE) {
+            const uint32_t total = (uint32_t)sgpr((int)(uint32_t)starts[kRasterChunk + 1]);
+            const uint32_t first = (uint32_t)lane < n ? lrec[lane * 5 + 4].z & 0xFFFFu : ~0u;
+            for (uint32_t b = (uint32_t)wave * 64u; b < total; b += 256u) {
+                // A candidate's record: the last with a start at or before it.
+                const unsigned long long sv = starts[b >> 6];
+                const uint64_t m = ((uint64_t)(uint32_t)sgpr((int)(sv >> 32)) << 32 |
+                                    (uint32_t)sgpr((int)(uint32_t)sv)) >> 1;
+                const uint32_t r0 = (uint32_t)__popcll(ballot(first <= b)) - 1u;
+                const uint32_t i = __builtin_amdgcn_mbcnt_hi(
+                    (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, r0));
+                const uint4 w2 = lrec[i * 5 + 2], w3 = lrec[i * 5 + 3], w4 = lrec[i * 5 + 4];
+                const uint32_t c = b + (uint32_t)lane, p = c - (w4.z & 0xFFFFu);
+                const uint32_t y = __umul24(p, w4.w & 0xFFFFFu) >> 16;
+                const uint32_t x = p - __umul24(y, w4.w >> 20);
+                const int g0 = (int)edge24((int)w3.x, (int)x, (int)w3.w, (int)y, w2.y);
+                const int g1 = (int)edge24((int)w3.y, (int)x, (int)w4.x, (int)y, w2.z);
+                const int g2 = (int)edge24((int)w3.z, (int)x, (int)w4.y, (int)y, w2.w);
+                const int in = c < total && (w4.w >> 20) != 0u ? -1 : 0;
+                step(g0 & g1 & g2 & in, g1, g2, (i << 12) + (w4.z >> 16) + y * (uint32_t)TW + x);
+            }
+            const unsigned long long ov = starts[kRasterChunk];
+            own = ((uint64_t)(uint32_t)sgpr((int)(ov >> 32)) << 32 |
+                   (uint32_t)sgpr((int)(uint32_t)ov)) &
+                  (0x1111111111111111ull << wave);
+        }
         // Per wave, one triangle at a time: lanes cover an lpr x (64/lpr) pixel
         // block of its clamped box, stepping the int32 edge values by additions
-        // (rasterizer.go:139-183 walks them the same way); inside fragments go
-        // to an LDS ring by ballot and their exact depth runs on full waves.
-        uint32_t qhead = 0, qtail = 0;  // wave-uniform ring positions
-        for (uint32_t i = wave; i < n; i += 4) {
+        // (rasterizer.go:139-183 walks them the same way).
+        for (uint32_t i = wave; DENSE ? own != 0 : i < n; i += 4) {
+            if (DENSE) {
+                i = (uint32_t)__builtin_ctzll(own);
+                own &= own - 1;
+            }
             // The walk form of the record (see walk_form): the box word moves
             // to a scalar register, the coefficients stay in vector registers
             // (the same value in every lane).
@@ -2127,32 +2236,6 @@ __device__ __forceinline__ unsigned long long raster_list(
             // (y * TW + x, below 4096 for every tile size), exact in every lane
             // that enqueues (its pixel lies inside the tile).
             const uint32_t prow = (i << 12) + (uint32_t)(oy * TW + ox) + (uint32_t)(ly * TW + lx);
-            // One walk step: lanes with all < 0 hold an inside fragment (every
-            // edge value < 0, rasterizer.go:147, and the pixel inside the box);
-            // they go to the wave's ring by ballot, and every 64 queued
-            // fragments get their exact depth.
-            auto step = [&](int all, int g1, int g2, uint32_t pk) {
-                const uint64_t mask = ballot(all < 0);
-                if (mask) {
-                    if (all < 0) {
-                        const uint32_t k =
-                            __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
-                                                      __builtin_amdgcn_mbcnt_lo(
-                                                          (uint32_t)mask, qtail)) &
-                            127u;
-                        q[0][k] = pk;
-                        q[1][k] = (uint32_t)g1;
-                        q[2][k] = (uint32_t)g2;
-                    }
-                    const uint32_t m = (uint32_t)__popcll(mask);
-                    qtail += m;
-                    covered_wave += m;
-                    if (qtail - qhead >= 64u) {
-                        frag_depth<TW>(q, qhead, 64u, lrec, lslot, key, lane);
-                        qhead += 64u;
-                    }
-                }
-            };
             // The box is at most TW <= 64 pixels wide, so one column block of
             // lanes covers it: a flat loop over row blocks. The lane's column
             // is inside the box iff gx < 0; only the last block can hold rows
@@ -2342,7 +2425,7 @@ __device__ __forceinline__ unsigned long long shade_tile(const DevFrame& fr, int
 }
 
 // LDS of one raster workgroup.
-template <int TW, int TH>
+template <int TW, int TH, bool DENSE>
 struct RasterLds {
     unsigned long long key[TW * TH];
     uint4 lrec[kRasterChunk * 5];  // the staged raster records
@@ -2350,6 +2433,9 @@ struct RasterLds {
     uint32_t qbuf[4][3][128];      // per-wave ring: pixel, f12, f20
     unsigned long long red[4][2];  // per wave: covered fragments, shaded pixels
     uint32_t last;                 // the workgroup shades a split tile
+    // Per 64 candidates of a dense chunk, which start a record; then the records
+    // walked on their own, and the number of candidates.
+    unsigned long long starts[DENSE ? kStartWords : 1];
 };
 
 // Entries of the batch's split tiles (k_bin_scan) and the size of their parts:
@@ -2381,7 +2467,7 @@ __device__ __forceinline__ SplitLists split_lists(const DevBatchCounters* counte
 // sequence) resolve does not depend on order); the workgroup that merges last takes
 // them back, leaves the slab and its counter cleared for the next draw, and shades.
 // No part waits for another. Every thread of the workgroup calls it.
-template <int TW, int TH>
+template <int TW, int TH, bool DENSE>
 __device__ __forceinline__ void raster_part(
     const DevFrame* __restrict__ frames, const int* __restrict__ tile_first, int nframes,
     uint32_t* __restrict__ tile_counts, const uint32_t* __restrict__ tile_offsets,
@@ -2389,7 +2475,7 @@ __device__ __forceinline__ void raster_part(
     const DevTexture* __restrict__ textures, unsigned long long* __restrict__ stats,
     const uint32_t* __restrict__ split_first, const uint32_t* __restrict__ split_tile,
     unsigned long long* __restrict__ slabs, uint32_t* __restrict__ slab_done, uint32_t part_refs,
-    int g, int item, const SplitLists& s, RasterLds<TW, TH>& L, int lane, int wave) {
+    int g, int item, const SplitLists& s, RasterLds<TW, TH, DENSE>& L, int lane, int wave) {
     constexpr int NPX = TW * TH;
     uint32_t slab_i = kNoSlab, first = 0u, pos = 0u;
     if (item >= 0) {
@@ -2421,8 +2507,8 @@ __device__ __forceinline__ void raster_part(
     for (int i = threadIdx.x; i < NPX; i += 256) L.key[i] = kBackgroundKey;
     // raster_list's first barrier orders the initialisation before its use.
     const unsigned long long covered =
-        raster_list<TW, TH>(fr, X0, Y0, refs + tile_offsets[g] + beg, n, L.key, L.lrec, L.lslot,
-                            L.qbuf[wave], lane, wave);
+        raster_list<TW, TH, DENSE>(fr, X0, Y0, refs + tile_offsets[g] + beg, n, L.key, L.lrec, L.lslot,
+                            L.qbuf[wave], L.starts, lane, wave);
     __syncthreads();
     bool shade = true;
     if (parts > 1u) {
@@ -2491,8 +2577,8 @@ __device__ __forceinline__ int xcd_tile(int h) {
 // what it keeps in scalar registers across items spills (k_raster 295 -> 325 us for
 // 32 frames of 200,000 triangles). Parts in a kernel of their own ahead of the tiles'
 // took 13 us more for a single frame and 75 of 533 us for 8 dense requests.
-template <int TW, int TH>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_waves(TW * TH))))
+template <int TW, int TH, bool DENSE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(raster_waves(TW * TH, DENSE))))
 void k_raster(
     const DevFrame* __restrict__ frames, const int* __restrict__ tile_first, int nframes,
     int total_tiles, uint32_t* __restrict__ tile_counts,
@@ -2502,13 +2588,13 @@ void k_raster(
     const uint32_t* __restrict__ split_first, const uint32_t* __restrict__ split_tile,
     unsigned long long* __restrict__ slabs, uint32_t* __restrict__ slab_done, uint32_t max_slabs,
     uint32_t part_refs, int extra) {
-    __shared__ RasterLds<TW, TH> L;
+    __shared__ RasterLds<TW, TH, DENSE> L;
     const int lane = threadIdx.x & 63, wave = sgpr(threadIdx.x >> 6);
     const SplitLists s = split_lists(counters, split_first, max_slabs, part_refs, (uint32_t)extra);
     const int it = (int)blockIdx.x < extra ? (int)blockIdx.x : -1;
     const int g = it < 0 ? xcd_tile((int)blockIdx.x - extra) : 0;
     if (g >= total_tiles) return;
-    raster_part<TW, TH>(frames, tile_first, nframes, tile_counts, tile_offsets, tile_slab, refs,
+    raster_part<TW, TH, DENSE>(frames, tile_first, nframes, tile_counts, tile_offsets, tile_slab, refs,
                         textures, stats, split_first, split_tile, slabs, slab_done, part_refs, g,
                         it, s, L, lane, wave);
 }
@@ -2526,11 +2612,11 @@ void k_raster_persistent(
     const uint32_t* __restrict__ split_first, const uint32_t* __restrict__ split_tile,
     unsigned long long* __restrict__ slabs, uint32_t* __restrict__ slab_done, uint32_t max_slabs,
     uint32_t part_refs, int extra) {
-    __shared__ RasterLds<TW, TH> L;
+    __shared__ RasterLds<TW, TH, false> L;
     const int lane = threadIdx.x & 63, wave = sgpr(threadIdx.x >> 6);
     const SplitLists s = split_lists(counters, split_first, max_slabs, part_refs, (uint32_t)extra);
     for (int j = (int)blockIdx.x; j < extra + total_tiles; j += (int)gridDim.x) {
-        raster_part<TW, TH>(frames, tile_first, nframes, tile_counts, tile_offsets, tile_slab,
+        raster_part<TW, TH, false>(frames, tile_first, nframes, tile_counts, tile_offsets, tile_slab,
                             refs, textures, stats, split_first, split_tile, slabs, slab_done,
                             part_refs, j < extra ? 0 : j - extra, j < extra ? j : -1, s, L, lane,
                             wave);
@@ -2846,10 +2932,11 @@ static void raster_t(const LaunchParams& p, hipStream_t s) {
     }
     constexpr int kRound = 8 * kTileRun;
     const int tiles = (p.total_tiles + kRound - 1) / kRound * kRound;
-    hipLaunchKernelGGL((k_raster<TW, TH>), dim3(tiles + extra), dim3(256), 0, s, p.frames, p.tile_first, p.nframes,
-                           p.total_tiles, p.tile_counts, p.tile_offsets, p.tile_slab, p.refs,
-                           p.textures, p.stats, p.counters, p.split_first, p.split_tile, p.slabs,
-                           p.slab_done, p.max_slabs, p.part_refs, extra);
+    hipLaunchKernelGGL((p.dense ? k_raster<TW, TH, true> : k_raster<TW, TH, false>),
+                       dim3(tiles + extra), dim3(256), 0, s, p.frames, p.tile_first, p.nframes,
+                       p.total_tiles, p.tile_counts, p.tile_offsets, p.tile_slab, p.refs, p.textures,
+                       p.stats, p.counters, p.split_first, p.split_tile, p.slabs, p.slab_done,
+                       p.max_slabs, p.part_refs, extra);
 }
 
 bool launch_raster(const LaunchParams& p, hipStream_t s) {

@@ -31,6 +31,7 @@ struct LaunchParams {
     uint32_t* slab_done;     // [max_slabs]: parts merged into each slab; zero between draws
     uint32_t max_slabs;
     uint32_t part_refs;      // least tile-list entries per raster part
+    bool dense;              // lists of many small boxes (k_raster's DENSE)
     uint32_t split_refs;     // lists longer than this count as split (gr_stats.tiles_split)
     uint32_t* frame_overflow;// [nframes]
     FaceBlock* blocks;       // [face_blocks]

@@ -444,3 +444,32 @@ def test_shading_forms(ctx, side, kind, scale, stretch, step):
     scene.frame.dot_step = step
     with np.errstate(invalid="ignore"):
         assert_same(scene, ctx.draw(scene), refcpu.draw(scene))
+
+
+@pytest.mark.parametrize("grid,eye,tile", [
+    ((100, 160), 4.5, (32, 32)), ((100, 160), 2.2, (8, 64)), ((100, 160), 3.0, (64, 64)),
+    ((200, 320), 9.0, (16, 16)), ((200, 320), 5.0, (64, 8))])
+def test_dense_batches(ctx, grid, eye, tile):
+    """Batches that take the dense raster, at several tile shapes: chunks of
+    small boxes, of mixed ones, and of boxes cut by their tile."""
+    import scene_cases as C
+    scene = C.sphere(w=331, h=245, eye=(0.02, 0.01, eye), nlat=grid[0], nlon=grid[1])
+    want = refcpu.draw(scene)
+    tiles = -(-331 // tile[0]) * -(-245 // tile[1])
+    old = ctx.config()
+    try:
+        ctx.set_config(tile_w=tile[0], tile_h=tile[1], refs_capacity=1 << 23)
+        handles = ctx.upload_scene(scene)[0]
+        n = 4096 // tiles + 1
+        outs = [ctx.frame_buffers(331, 245) for _ in range(n)]
+        ctx.draw_batch([scene] * n, [handles] * n, [(o[0].ptr, o[1].ptr) for o in outs])
+        ctx.synchronize()
+        stats = ctx.last_stats()
+        for k, (rg, dp) in enumerate(outs):
+            assert np.array_equal(rg.to_numpy(np.uint8, (245, 331, 4)), want[0]), k
+            assert np.array_equal(dp.to_numpy(np.uint32, (245, 331)), want[1].view(np.uint32)), k
+            assert stats[k]["fragments_covered"] == want[2]["fragments_covered"]
+            rg.free()
+            dp.free()
+    finally:
+        ctx.set_config(tile_w=old.tile_w, tile_h=old.tile_h, refs_capacity=old.refs_capacity)
