@@ -7,10 +7,12 @@
 //               = 256 faces = 1792 slots in draw order. The workgroup then
 //               counts its tile references in LDS and adds them to the global
 //               tile counts.
-//   k_bin_scan  one workgroup per frame: tile counts -> tile-list offsets.
+//   k_bin_scan  one workgroup per frame: tile counts -> tile-list offsets, and
+//               the slabs of tiles whose lists are split.
 //   k_bin_fill  per face workgroup: scatter slots into tile lists, with one
 //               global atomic per distinct tile per workgroup.
-//   k_raster    one workgroup per screen tile: triangles staged in LDS,
+//   k_raster    one workgroup per screen tile or part of a split tile's list:
+//               triangles staged in LDS,
 //               visibility with a 64-bit (depth, draw-sequence) max key in LDS,
 //               one deferred shading pass and a single write of colour + depth.
 //
@@ -2268,8 +2270,9 @@ __device__ __forceinline__ unsigned long long raster_list(
 // Deferred shading of the winning fragment of each pixel of the tile, one
 // write per pixel. Returns the wave's count of shaded pixels.
 //
-// k_raster is bound by the issue of vector instructions where frames are many (93%
-// of its cycles for 32 frames of 1280x720), so a pixel's are kept few: one
+// Where frames are many k_raster is bound by its instructions (512 frames of
+// 1280x720: vector issue in 74% of its cycles, pairs counted once, at 7.5 of 8
+// waves), so a pixel's are kept few: one
 // reciprocal for u and v, indices of a shared texture by shift or by a reciprocal
 // of its side, colour bytes put together by byte selects, 32-bit offsets, and the
 // dot grid by one product. 32 frames of 200,000 triangles: k_raster 301 -> 294 us;
@@ -2913,8 +2916,8 @@ template <int TW, int TH>
 static void raster_t(const LaunchParams& p, hipStream_t s) {
     // Workgroups for split tiles' parts: four times what fills every CU at the
     // raster's occupancy, so that the parts of a dense batch end close together
-    // (8 dense requests, 7,560 tiles: 628 us with one time, 481 with two, 423 with
-    // four, 425 with eight); fewer for a small batch (one frame: 256, 1,024 and
+    // (8 dense requests, 7,560 tiles, before the dense form: 628 us with one time,
+    // 481 with two, 423 with four, 425 with eight); fewer for a small batch (one frame: 256, 1,024 and
     // 2,048 alike), and one time for a batch whose tiles alone fill the chip over
     // and over (64 mixed frames: one, two, four and eight times alike; they return
     // at once where nothing is split, 2,048 in 1 of 300 us, 8,192 in 4).

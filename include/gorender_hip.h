@@ -149,7 +149,8 @@ typedef struct {
     int64_t faces_front;       /* faces passing the backface test */
     int64_t clip_overflow;     /* faces dropped by GR_ERR_CLIP_OVERFLOW */
     int64_t refs;              /* tile-list entries used */
-    int64_t tiles_split;       /* tiles whose list several raster workgroups shared */
+    int64_t tiles_split;       /* tiles whose list is longer than tile_split (several
+                                  raster workgroups share it) */
 } gr_stats;
 
 /* One frame of an asynchronous batch: outputs are device pointers. */
@@ -168,7 +169,8 @@ typedef struct {
     int32_t raster_waves;         /* waves per raster workgroup: 4 */
     int32_t tile_split;           /* tile-list entries per raster workgroup, 64..2^24: a
                                      longer list is split into parts that several
-                                     workgroups resolve (same result, more parallelism) */
+                                     workgroups resolve (same result, more parallelism);
+                                     launches of at most 4096 tiles split from 64 on */
     int32_t pipelines;            /* 1 or 2 (default): with 2, consecutive asynchronous draws
                                      alternate between two sets of buffers and streams, so a
                                      draw's geometry stages overlap the previous draw's raster;
