@@ -2394,7 +2394,9 @@ __device__ __forceinline__ unsigned long long shade_tile(const DevFrame& fr, int
                         // |u| < 2^-38: 1 - u is 1, and v * scale * h is under 1
                         // either way. Above, a quotient is the same one, or at
                         // least 2^127, infinite or a NaN, and so past int64 once
-                        // scaled, in both ways.
+                        // scaled, in both ways. (Checked on the device: 128
+                        // numerators for each of the 2^23 significands of z,
+                        // the ranges' ends included, all the same bits.)
                         const float y0 = __builtin_amdgcn_rcpf(b.zrec);
                         const float y1 = __builtin_fmaf(__builtin_fmaf(-b.zrec, y0, 1.0f), y0, y0);
                         u = div_rcp(un, b.zrec, y1);
