@@ -6,8 +6,9 @@ scenes synchronously into numpy buffers or asynchronously into device memory.
 from __future__ import annotations
 
 import ctypes
-import sys
+import math
 import threading
+from collections import deque
 from typing import Dict, List, Optional, Sequence, Tuple
 
 import numpy as np
@@ -37,39 +38,60 @@ def frame_struct(fr: FrameData) -> _lib.gr_frame:
     return f
 
 
+class _Lease:
+    """Memory of a ResultArrays on loan to one array: the array and every view of
+    it hold the lease, which hands the memory back when the last of them is gone."""
+
+    __slots__ = ("__array_interface__", "_memory", "_returned")
+
+    def __init__(self, memory: np.ndarray, returned: deque, dtype: np.dtype, shape):
+        self.__array_interface__ = {"version": 3, "typestr": dtype.str, "shape": shape,
+                                    "data": (memory.ctypes.data, False)}
+        self._memory = memory
+        self._returned = returned
+
+    def __del__(self):
+        # Any thread may be here, at any point of its work: one atomic append.
+        self._returned.append(self._memory)
+
+
 class ResultArrays:
     """Memory of the arrays that a context's frames are delivered in.
 
     A fresh array of a frame's size costs more in page faults than the copy into
-    it, so memory whose last array is gone is used again: a block is free when
-    nothing but this pool refers to it (an array made of it, and every view of
-    that, keeps it as its base). Blocks number at most LIMIT bytes and are given
-    back when the context is closed."""
+    it, so memory whose last array is gone is used again (a caller that keeps its
+    frames, or more of them than LIMIT, gets fresh memory for each, as without).
+    The arrays do not own their memory: ndarray.resize in place needs a copy.
+    Blocks number at most LIMIT bytes and are given back when the context is
+    closed."""
 
     LIMIT = 256 << 20
     LEAST = 256 << 10
 
     def __init__(self):
         self._lock = threading.Lock()
-        self._blocks: Dict[int, List[np.ndarray]] = {}
-        self._bytes = 0
+        self.clear()
 
     def empty(self, dtype, shape) -> np.ndarray:
-        n = int(np.dtype(dtype).itemsize * np.prod(shape, dtype=np.int64))
+        dtype = np.dtype(dtype)
+        n = dtype.itemsize * math.prod(shape)
         if n < self.LEAST:
             return np.empty(shape, dtype)
         with self._lock:
-            for b in self._blocks.get(n, ()):
-                if sys.getrefcount(b) == 3:  # the list's, the loop's and the call's
-                    return b.view(dtype).reshape(shape)
-            if self._bytes + n > self.LIMIT:
-                self._drop_free(n)
-            if self._bytes + n > self.LIMIT:
-                return np.empty(shape, dtype)
-            b = np.empty(n, np.uint8)
-            self._blocks.setdefault(n, []).append(b)
-            self._bytes += n
-            return b.view(dtype).reshape(shape)
+            while self._returned:
+                b = self._returned.popleft()
+                self._free.setdefault(b.nbytes, []).append(b)
+            if self._free.get(n):
+                b = self._free[n].pop()
+            else:
+                if self._bytes + n > self.LIMIT:
+                    self._bytes -= sum(k * len(v) for k, v in self._free.items())
+                    self._free.clear()
+                if self._bytes + n > self.LIMIT:
+                    return np.empty(shape, dtype)
+                b = np.empty(n, np.uint8)
+                self._bytes += n
+            return np.asarray(_Lease(b, self._returned, dtype, shape))
 
     def copy_out(self, ptr, dtype, shape) -> np.ndarray:
         """An array holding what the C pointer names (gr_host_copy)."""
@@ -78,18 +100,12 @@ class ResultArrays:
                                             out.nbytes))
         return out
 
-    def _drop_free(self, keep: int) -> None:
-        """Forgets the free blocks of sizes other than `keep`."""
-        for n, blocks in self._blocks.items():
-            if n != keep:
-                used = [b for b in blocks if sys.getrefcount(b) > 3]
-                self._bytes -= n * (len(blocks) - len(used))
-                blocks[:] = used
-
     def clear(self) -> None:
+        """Gives the free blocks back; those on loan go with their last array."""
         with self._lock:
-            self._blocks.clear()
-            self._bytes = 0
+            self._free: Dict[int, List[np.ndarray]] = {}
+            self._returned: deque = deque()  # by leases of this pool since it was cleared
+            self._bytes = 0  # of the blocks, on loan or free
 
 
 class Context:

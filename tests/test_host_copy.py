@@ -1,6 +1,7 @@
 """gr_host_copy and the arrays that frames are delivered in (no GPU needed)."""
 import os
 import signal
+import sys
 import threading
 
 import numpy as np
@@ -79,6 +80,59 @@ def test_result_arrays_are_bounded():
     assert pool.empty(np.uint8, (10,)).base is None  # small arrays are their own
     pool.clear()
     other[:] = 1
+
+
+def test_result_arrays_do_not_rest_on_reference_counts(monkeypatch):
+    """What an interpreter counts for a local or an argument is its own business:
+    memory is on loan as long as an array or a view of it lives."""
+    pool = ResultArrays()
+    monkeypatch.setattr(sys, "getrefcount", lambda o: 3)
+    held = [pool.empty(np.uint8, (512, 512, 4))[1:] for _ in range(4)]
+    assert len({h.ctypes.data for h in held}) == 4
+    for k, h in enumerate(held):
+        h[:] = k
+    assert [int(h.max()) for h in held] == [0, 1, 2, 3]
+
+
+def test_result_arrays_from_several_threads():
+    """Arrays taken, filled and dropped by four threads at once, a few kept across
+    turns: none is handed out twice, and the blocks stay few."""
+    pool = ResultArrays()
+    bad = []
+
+    def work(seed):
+        kept = []
+        for k in range(300):
+            a = pool.empty(np.uint32, (256, 256 + 64 * (k % 3)))
+            a[:] = seed * 1000 + k
+            kept.append((seed * 1000 + k, a[5:]))
+            if len(kept) == 4:
+                v, a = kept.pop(k % 4)
+                if not (a == v).all():
+                    bad.append((seed, k))
+
+    threads = [threading.Thread(target=work, args=(s,)) for s in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+    pool.empty(np.uint8, (1 << 18,))
+    assert pool._bytes <= 3 * 4 * 5 * (256 * 384 * 4)
+
+
+def test_result_arrays_on_loan_outlive_a_cleared_pool():
+    pool = ResultArrays()
+    a = pool.empty(np.uint8, (1 << 20,))
+    a[:] = 7
+    pool.clear()
+    b = pool.empty(np.uint8, (1 << 20,))
+    b[:] = 9
+    assert (a == 7).all()
+    del a  # its memory goes: it is not the cleared pool's any more
+    c = pool.empty(np.uint8, (1 << 20,))
+    assert pool._bytes == 2 << 20
+    assert c.ctypes.data != b.ctypes.data
 
 
 def test_host_copy_in_a_forked_child():
