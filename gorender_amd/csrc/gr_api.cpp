@@ -1156,6 +1156,13 @@ namespace gr_internal {
 
 gr_status fail(gr_status s, const std::string& msg) { return ::fail(s, msg); }
 
+hipError_t pinned_alloc(void** p, size_t bytes) {
+    const hipError_t e = hipHostMalloc(p, bytes, hipHostMallocDefault);
+    if (e == hipSuccess)
+        for (size_t b = 0; b < bytes; b += 4096) ((volatile char*)*p)[b] = 0;
+    return e;
+}
+
 gr_status enqueue_batch(gr_context* c, const gr_batch_frame* frames, int32_t nf,
                         const gr_object* objs, int32_t no) {
     try {
@@ -1799,7 +1806,7 @@ gr_status gr_draw(gr_context* c, const gr_frame* frame, const gr_object* objs, i
             if (c->h_frame) GR_HIP(hipHostFree(c->h_frame));
             c->h_frame = nullptr;
             c->h_frame_cap = 0;
-            GR_HIP(hipHostMalloc(&c->h_frame, npx * 8, hipHostMallocDefault));
+            GR_HIP(gr_internal::pinned_alloc(&c->h_frame, npx * 8));
             c->h_frame_cap = npx * 8;
         }
         char* const staged = (char*)c->h_frame;
@@ -1860,7 +1867,7 @@ gr_status gr_present_draw(gr_context* c, const gr_frame* frame, const gr_object*
             if (ps.host) GR_HIP(hipHostFree(ps.host));
             ps.host = nullptr;
             ps.host_cap = 0;
-            GR_HIP(hipHostMalloc(&ps.host, hb, hipHostMallocDefault));
+            GR_HIP(gr_internal::pinned_alloc(&ps.host, hb));
             ps.host_cap = hb;
         }
         if (!ps.h_meta) GR_HIP(hipHostMalloc(&ps.h_meta, gr::kNumStats * 8 + 16, hipHostMallocDefault));

@@ -123,7 +123,7 @@ gr_status gr_server::take_target(size_t bytes, size_t host_bytes, Target* t) {
     if (h != free_host.end()) {
         t->host = h->second;
         free_host.erase(h);
-    } else if (hipHostMalloc(&t->host, host_bytes, hipHostMallocDefault) != hipSuccess) {
+    } else if (gr_internal::pinned_alloc(&t->host, host_bytes) != hipSuccess) {
         free_dev.emplace(bytes, t->dev);
         t->dev = t->host = nullptr;
         return fail(GR_ERR_OUT_OF_MEMORY, "pinned host target");

@@ -57,3 +57,34 @@ def test_present_overflow_redraws(ctx):
             _check(scene, ctx.present_wait(320, 240), want)
     finally:
         ctx.set_config(tile_w=old.tile_w, tile_h=old.tile_h, refs_capacity=old.refs_capacity)
+
+
+def test_first_copy_of_a_frame_takes_no_page_faults():
+    """The pinned pages of a fresh context's frames are mapped before the threads
+    that share a copy read them (each of the threads would take the fault of the
+    same large page): a first copy into memory already written faults nowhere."""
+    import ctypes
+    import resource
+
+    from gorender_amd.device import Context
+    w, h = 1920, 1080
+    scene = C.sphere(w=w, h=h)
+    dst = np.ones((h, w, 4), np.uint8)
+    with Context(0) as c:
+        src = np.ones(1 << 20, np.uint8)  # the copy's threads run already
+        _lib.check(c.lib.gr_host_copy(dst.ctypes.data, src.ctypes.data, src.nbytes))
+        handles = c.upload_scene(scene)[0]
+        for _ in range(2):
+            c.present_draw(scene, handles, with_depth=False)
+        for _ in range(2):
+            rp, dp = ctypes.POINTER(ctypes.c_uint8)(), ctypes.POINTER(ctypes.c_float)()
+            st = _lib.gr_stats()
+            _lib.check(c.lib.gr_present_wait(c.handle, ctypes.byref(rp), ctypes.byref(dp),
+                                             ctypes.byref(st)))
+            before = resource.getrusage(resource.RUSAGE_SELF).ru_minflt
+            _lib.check(c.lib.gr_host_copy(dst.ctypes.data, ctypes.cast(rp, ctypes.c_void_p),
+                                          dst.nbytes))
+            faults = resource.getrusage(resource.RUSAGE_SELF).ru_minflt - before
+            # Pages of at most 2 MB: four or more faults for 8.3 MB not yet mapped.
+            assert faults < 2, faults
+    assert np.array_equal(dst, refcpu.draw(scene)[0])
