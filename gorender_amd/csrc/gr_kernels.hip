@@ -1716,6 +1716,7 @@ __global__ __launch_bounds__(kFillThreads) void k_bin_fill(const DevFrame* __res
     constexpr uint32_t kFillKeep = 256;
     __shared__ uint2 lrange[kFillKeep];  // tx0 | tx1 << 16, ty0 | ty1 << 16
     uint32_t ux = 0u, uy = 0u;  // union: last + 1 | (0xFFFF - first) << 16
+    uint32_t nrefs = 0u;        // references
     for (uint32_t i = threadIdx.x; i < cnt; i += kFillThreads) {
         const uint32_t ri = block_rec(b, ovf, i);
         const TileRect t = rec_tiles(&fr.rrec[ri], twl, thl);
@@ -1725,6 +1726,7 @@ __global__ __launch_bounds__(kFillThreads) void k_bin_fill(const DevFrame* __res
         if (t.tx0 > t.tx1) continue;
         ux = max_u16x2(ux, (uint32_t)(t.tx1 + 1) | (uint32_t)(0xFFFF - t.tx0) << 16);
         uy = max_u16x2(uy, (uint32_t)(t.ty1 + 1) | (uint32_t)(0xFFFF - t.ty0) << 16);
+        nrefs += (uint32_t)((t.tx1 - t.tx0 + 1) * (t.ty1 - t.ty0 + 1));
     }
     // fn(t, i) for the tile range of every record i, 64 records at a time by all
     // lanes of the wave (empty past the last record).
@@ -1752,40 +1754,67 @@ __global__ __launch_bounds__(kFillThreads) void k_bin_fill(const DevFrame* __res
     const int rx0 = 0xFFFF - (int)(ux >> 16), rx1 = (int)(ux & 0xFFFFu) - 1;
     const int ry0 = 0xFFFF - (int)(uy >> 16), ry1 = (int)(uy & 0xFFFFu) - 1;
     if (rx1 < 0) return;
-    // The union in windows of at most kLdsTiles tiles (one, but for triangles
-    // that span most of a large frame).
+    // fn(tx, ty, i) for every reference of record i to a tile of [x0, x1] x [y0, y1]:
+    // each box by its record's lane, or the boxes of many tiles one after the other
+    // by the whole wave where that takes fewer steps (a step here is one box, plus
+    // one per 64 tiles). One lane walking the 2,040 tiles of a full-screen triangle
+    // kept its workgroup 300 us after all others were done; but where most lanes
+    // have such a box, the lanes are the faster side: 2,000 triangles of some 190
+    // tiles at 1280x720 90 us, 209 with every box over 16 tiles placed by the wave.
+    auto each_ref = [&](int x0, int y0, int x1, int y1, auto&& fn) {
+        each_range([&](const TileRect& t, uint32_t i) {
+            const int bx0 = max(t.tx0, x0), bx1 = min(t.tx1, x1);
+            const int by0 = max(t.ty0, y0), by1 = min(t.ty1, y1);
+            const int m = max(bx1 - bx0 + 1, 0) * max(by1 - by0 + 1, 0);
+            constexpr int kLaneTiles = 16;
+            uint64_t big = ballot(m > kLaneTiles);
+            if (big) {
+                const uint32_t most = wave_reduce((uint32_t)m, 0u, [](uint32_t a, uint32_t b) {
+                    return a > b ? a : b;
+                });
+                if ((uint32_t)__popcll(big) * (3u + (most >> 6)) >= most) big = 0ull;
+            }
+            if (m > 0 && (m <= kLaneTiles || !big))
+                for (int ty = by0; ty <= by1; ty++)
+                    for (int tx = bx0; tx <= bx1; tx++) fn(tx, ty, i);
+            for (; big; big &= big - 1) {
+                const int L = __builtin_ctzll(big);
+                const uint32_t bi = (uint32_t)__builtin_amdgcn_readlane((int)i, L);
+                wave_rect(__builtin_amdgcn_readlane(bx0, L), __builtin_amdgcn_readlane(by0, L),
+                          __builtin_amdgcn_readlane(bx1, L), __builtin_amdgcn_readlane(by1, L),
+                          (int)threadIdx.x, [&](int tx, int ty) { fn(tx, ty, bi); });
+            }
+        });
+    };
+    // The union in windows of at most kLdsTiles tiles.
     const int ww = min(rx1 - rx0 + 1, kLdsTiles), wh = min(ry1 - ry0 + 1, kLdsTiles / ww);
+    const uint32_t windows = (uint32_t)((rx1 - rx0) / ww + 1) * (uint32_t)((ry1 - ry0) / wh + 1);
+    nrefs = wave_sum_u32(nrefs);
+    // Triangles scattered over a large frame: one global atomic per reference, where
+    // that is less than what the further windows cost (each clears and scans its
+    // counters and goes through all records twice, some 8 us). The line falls with
+    // the blocks of the frame, whose atomics queue up at the same cache lines. us by
+    // windows | by references, 32x32 tiles but where stated: 20,000 triangles of 8
+    // pixels at 3840x2160 90 | 14, at 7680x4320 238 | 14, of 60 pixels 154 | 49 and
+    // 437 | 49; 200,000 of 30 pixels at 1920x1080 78 | 176, at 2560x1440 83 | 111, at
+    // 3840x2160 137 | 60; 2,000 of 150 pixels at 1920x1080 87 | 121, at 2560x1440
+    // 180 | 149; 20,000 of 60 pixels at 1280x720 in 8x8 tiles 498 | 351.
+    const uint32_t sparse = max(64u, min(8192u, 300000u / (uint32_t)max(fr.face_blocks, 1)));
+    if (nrefs < sparse * (windows - 1u)) {
+        each_ref(rx0, ry0, rx1, ry1, [&](int tx, int ty, uint32_t i) {
+            refs[atomicAdd(&tile_cursor[fr.tile_begin + ty * fr.tiles_x + tx], 1u)] = slot0 + i;
+        });
+        return;
+    }
     for (int wy = ry0; wy <= ry1; wy += wh)
         for (int wx = rx0; wx <= rx1; wx += ww) {
             const int xe = min(wx + ww - 1, rx1), ye = min(wy + wh - 1, ry1);
             const int n = ww * (ye - wy + 1);
-            // fn(window tile, i) for every reference of record i to a tile of
-            // the window: a few tiles by the record's lane, more by the whole
-            // wave (one lane walking the 2,040 tiles of a full-screen triangle
-            // kept its workgroup 300 us after all others were done).
-            auto each_ref = [&](auto&& fn) {
-                each_range([&](const TileRect& t, uint32_t i) {
-                    const int x0 = max(t.tx0, wx), x1 = min(t.tx1, xe);
-                    const int y0 = max(t.ty0, wy), y1 = min(t.ty1, ye);
-                    const int w = max(x1 - x0 + 1, 0), m = w * max(y1 - y0 + 1, 0);
-                    constexpr int kLaneTiles = 16;
-                    if (m > 0 && m <= kLaneTiles)
-                        for (int ty = y0; ty <= y1; ty++)
-                            for (int tx = x0; tx <= x1; tx++) fn((ty - wy) * ww + tx - wx, i);
-                    for (uint64_t big = ballot(m > kLaneTiles); big; big &= big - 1) {
-                        const int L = __builtin_ctzll(big);
-                        const uint32_t bi = (uint32_t)__builtin_amdgcn_readlane((int)i, L);
-                        wave_rect(__builtin_amdgcn_readlane(x0, L) - wx,
-                                  __builtin_amdgcn_readlane(y0, L) - wy,
-                                  __builtin_amdgcn_readlane(x1, L) - wx,
-                                  __builtin_amdgcn_readlane(y1, L) - wy, (int)threadIdx.x,
-                                  [&](int tx, int ty) { fn(ty * ww + tx, bi); });
-                    }
-                });
-            };
             for (int k = threadIdx.x; k < n; k += kFillThreads) lcnt[k] = 0u;
             __syncthreads();
-            each_ref([&](int t, uint32_t) { atomicAdd(&lcnt[t], 1u); });
+            each_ref(wx, wy, xe, ye, [&](int tx, int ty, uint32_t) {
+                atomicAdd(&lcnt[(ty - wy) * ww + tx - wx], 1u);
+            });
             __syncthreads();
             // One global reservation per touched tile; lcnt becomes the write
             // cursor.
@@ -1796,7 +1825,9 @@ __global__ __launch_bounds__(kFillThreads) void k_bin_fill(const DevFrame* __res
                         &tile_cursor[fr.tile_begin + (wy + k / ww) * fr.tiles_x + wx + k % ww], v);
             }
             __syncthreads();
-            each_ref([&](int t, uint32_t i) { refs[atomicAdd(&lcnt[t], 1u)] = slot0 + i; });
+            each_ref(wx, wy, xe, ye, [&](int tx, int ty, uint32_t i) {
+                refs[atomicAdd(&lcnt[(ty - wy) * ww + tx - wx], 1u)] = slot0 + i;
+            });
             __syncthreads();
         }
 }

@@ -473,3 +473,61 @@ def test_dense_batches(ctx, grid, eye, tile):
             dp.free()
     finally:
         ctx.set_config(tile_w=old.tile_w, tile_h=old.tile_h, refs_capacity=old.refs_capacity)
+
+
+def _soup(n, w, h, px, seed=1):
+    """n triangles of about px pixels at random places, drawn in no order of place."""
+    rng = np.random.default_rng(seed)
+    c = rng.uniform([2, 2], [w - 2, h - 2], (n, 1, 2))
+    a = rng.uniform(0, 2 * np.pi, (n, 1)) + np.array([0, 2 * np.pi / 3, 4 * np.pi / 3])
+    p = np.clip(c + px * np.stack([np.cos(a), np.sin(a)], -1), 0, [w - 1, h - 1]).reshape(-1, 2)
+    v = np.ones((3 * n, 4), np.float32)
+    v[:, 0], v[:, 1] = (p[:, 0] - w / 2) / (w / 2), (p[:, 1] - h / 2) / (h / 2)
+    v[:, 2] = 0.5 + 0.4 * np.sin(np.arange(3 * n))
+    # Both windings: about half of the faces cover pixels whichever side counts.
+    f = np.arange(3 * n, dtype=np.int32).reshape(n, 3)
+    f[::2] = f[::2, ::-1]
+    eye = np.eye(4, dtype=np.float32)
+    return S.SceneData(S.FrameData(w, h, flags=_lib.GR_SHOW_FACES), [S.MeshData(v, f)], [],
+                       [S.ObjectData(0, eye, eye)], name=f"soup-{n}-{px}")
+
+
+@pytest.mark.parametrize("size", [(256, 256), (520, 257), (1041, 1033)])
+@pytest.mark.parametrize("n,px", [(40, 3), (300, 14), (300, 15), (700, 40), (1300, 200), (9000, 6)])
+def test_binning_scattered_triangles(ctx, size, n, px):
+    """Face blocks whose triangles lie all over the frame, in one binning window
+    (1,024 tiles), a few and many: placed by references or through the windows,
+    boxes on either side of what a lane places by itself, few and many of them."""
+    scene = _soup(n, *size, px)
+    old = ctx.config()
+    ctx.set_config(tile_w=8, tile_h=8, refs_capacity=1 << 22)
+    try:
+        assert_same(scene, ctx.draw(scene), refcpu.draw(scene))
+    finally:
+        ctx.set_config(tile_w=old.tile_w, tile_h=old.tile_h, refs_capacity=old.refs_capacity)
+
+
+def test_binning_cost_follows_the_references(ctx):
+    """Small triangles all over a frame of 129,600 tiles: placing their few thousand
+    references takes less than the raster of the frame (it took five times as long
+    when every block went through all windows of the frame)."""
+    scene = _soup(20000, 3840, 2160, 8)
+    old = ctx.config()
+    ctx.set_config(tile_w=8, tile_h=8, pipelines=1)
+    try:
+        handles = ctx.upload_scene(scene)[0]
+        rg, dp = ctx.frame_buffers(3840, 2160)
+        best = {}
+        ctx.set_kernel_timing(True)
+        for _ in range(6):
+            ctx.reset_kernel_times()
+            ctx.draw_device(scene, handles, rg.ptr, dp.ptr)
+            ctx.synchronize()
+            for k, (ms, _) in ctx.kernel_times().items():
+                best[k] = min(best.get(k, 1e9), ms)
+        assert best["k_bin_fill"] < best["k_raster"], best
+        rg.free()
+        dp.free()
+    finally:
+        ctx.set_kernel_timing(False)
+        ctx.set_config(tile_w=old.tile_w, tile_h=old.tile_h, pipelines=old.pipelines)
