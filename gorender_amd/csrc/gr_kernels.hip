@@ -2511,10 +2511,17 @@ __device__ __forceinline__ void raster_part(
     const DevTexture* __restrict__ textures, unsigned long long* __restrict__ stats,
     const uint32_t* __restrict__ split_first, const uint32_t* __restrict__ split_tile,
     unsigned long long* __restrict__ slabs, uint32_t* __restrict__ slab_done, uint32_t part_refs,
-    int g, int item, const SplitLists& s, RasterLds<TW, TH, DENSE>& L, int lane, int wave) {
+    const DevBatchCounters* __restrict__ counters, uint32_t max_slabs, uint32_t extra, int g,
+    int item, RasterLds<TW, TH, DENSE>& L, int lane, int wave) {
     constexpr int NPX = TW * TH;
+    // Only parts of split tiles look at the split lists: in every workgroup, their
+    // counter ahead of everything else and the values held past it took frames of
+    // 129,600 empty 8x8 tiles from 89 to 126 us and 8,160 tiles of large triangles
+    // from 194 to 226.
+    SplitLists s{0u, 0u, 1u};
     uint32_t slab_i = kNoSlab, first = 0u, pos = 0u;
     if (item >= 0) {
+        s = split_lists(counters, split_first, max_slabs, part_refs, extra);
         const unsigned long long at = (unsigned long long)item * s.part;
         if (at >= s.entries) return;
         pos = (uint32_t)at;
@@ -2523,10 +2530,19 @@ __device__ __forceinline__ void raster_part(
         if (pos == first) return;  // the tile's own workgroup starts there
         g = sgpr((int)split_tile[slab_i]);
     }
-    const uint32_t cnt = (uint32_t)sgpr((int)tile_counts[g]);
+    const uint32_t cnt_v = tile_counts[g], off = tile_offsets[g];
+    const int fi = wave_last_le(tile_first, nframes, g);
+    const DevFrame& fr = frames[fi];
+    const int t = g - fr.tile_begin;
+    const int X0 = (t % fr.tiles_x) * TW, Y0 = (t / fr.tiles_x) * TH;
+    for (int i = threadIdx.x; i < NPX; i += 256) L.key[i] = kBackgroundKey;
+    const uint32_t cnt = (uint32_t)sgpr((int)cnt_v);
     if (item < 0 && cnt > part_refs) {
         slab_i = (uint32_t)sgpr((int)tile_slab[g]);
-        if (slab_i != kNoSlab) pos = first = (uint32_t)sgpr((int)split_first[slab_i]);
+        if (slab_i != kNoSlab) {
+            s = split_lists(counters, split_first, max_slabs, part_refs, extra);
+            pos = first = (uint32_t)sgpr((int)split_first[slab_i]);
+        }
     }
     // Parts of the tile, and this one's entries [beg, beg + n).
     uint32_t beg = 0u, n = cnt, parts = 1u;
@@ -2535,15 +2551,10 @@ __device__ __forceinline__ void raster_part(
         beg = pos - first;
         n = min(cnt - beg, s.part - pos % s.part);
     }
-    const int fi = wave_last_le(tile_first, nframes, g);
-    const DevFrame& fr = frames[fi];
-    const int t = g - fr.tile_begin;
-    const int X0 = (t % fr.tiles_x) * TW, Y0 = (t / fr.tiles_x) * TH;
 
-    for (int i = threadIdx.x; i < NPX; i += 256) L.key[i] = kBackgroundKey;
     // raster_list's first barrier orders the initialisation before its use.
     const unsigned long long covered =
-        raster_list<TW, TH, DENSE>(fr, X0, Y0, refs + tile_offsets[g] + beg, n, L.key, L.lrec, L.lslot,
+        raster_list<TW, TH, DENSE>(fr, X0, Y0, refs + off + beg, n, L.key, L.lrec, L.lslot,
                             L.qbuf[wave], L.starts, lane, wave);
     __syncthreads();
     bool shade = true;
@@ -2626,13 +2637,12 @@ void k_raster(
     uint32_t part_refs, int extra) {
     __shared__ RasterLds<TW, TH, DENSE> L;
     const int lane = threadIdx.x & 63, wave = sgpr(threadIdx.x >> 6);
-    const SplitLists s = split_lists(counters, split_first, max_slabs, part_refs, (uint32_t)extra);
     const int it = (int)blockIdx.x < extra ? (int)blockIdx.x : -1;
     const int g = it < 0 ? xcd_tile((int)blockIdx.x - extra) : 0;
     if (g >= total_tiles) return;
     raster_part<TW, TH, DENSE>(frames, tile_first, nframes, tile_counts, tile_offsets, tile_slab, refs,
-                        textures, stats, split_first, split_tile, slabs, slab_done, part_refs, g,
-                        it, s, L, lane, wave);
+                        textures, stats, split_first, split_tile, slabs, slab_done, part_refs,
+                        counters, max_slabs, (uint32_t)extra, g, it, L, lane, wave);
 }
 
 // Persistent form: a fixed grid (every CU at the raster's occupancy) in which
@@ -2650,12 +2660,11 @@ void k_raster_persistent(
     uint32_t part_refs, int extra) {
     __shared__ RasterLds<TW, TH, false> L;
     const int lane = threadIdx.x & 63, wave = sgpr(threadIdx.x >> 6);
-    const SplitLists s = split_lists(counters, split_first, max_slabs, part_refs, (uint32_t)extra);
     for (int j = (int)blockIdx.x; j < extra + total_tiles; j += (int)gridDim.x) {
         raster_part<TW, TH, false>(frames, tile_first, nframes, tile_counts, tile_offsets, tile_slab,
                             refs, textures, stats, split_first, split_tile, slabs, slab_done,
-                            part_refs, j < extra ? 0 : j - extra, j < extra ? j : -1, s, L, lane,
-                            wave);
+                            part_refs, counters, max_slabs, (uint32_t)extra,
+                            j < extra ? 0 : j - extra, j < extra ? j : -1, L, lane, wave);
         // The LDS state is rewritten by the next tile.
         __syncthreads();
     }
