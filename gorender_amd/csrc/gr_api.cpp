@@ -583,8 +583,9 @@ struct Bufs {
 
 // Entries per raster part. A launch of at most kFineTiles tiles leaves the chip's
 // 2,048 raster workgroups part idle and lasts as long as its longest list: lists
-// are split from kFinePart entries on (one staged chunk) while every tile can have
-// a slab. Larger launches split at the configured tile_split. (us of parts and
+// above a share of the launch's (k_bin_scan) are split into parts of kFinePart
+// entries or more (one staged chunk) while every tile can have a slab. Larger
+// launches split at the configured tile_split. (us of parts and
 // raster with parts of 512 | 192 | 128 | 64 entries: 64 instances of 1M triangles
 // 109 | 82 | 68 | 53, a frame of 5,000 28 | 28 | 31 | 30; frames of 200,000
 // triangles in flight 66 -> 44 us each with 64.)

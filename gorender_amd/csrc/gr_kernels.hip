@@ -1538,11 +1538,18 @@ __global__ __launch_bounds__(256) void k_fog(uint32_t* __restrict__ rgba,
 // release in every face workgroup, which on a multi-XCD part writes back and
 // invalidates L2 each time.
 //
-// A tile whose list holds more than part_refs entries may be split over several
-// raster workgroups: it takes a slab (depth keys of its pixels), and its entries a
-// range [split_first[slab], + count) of the split tiles' entries put end to end
-// (split_tile[slab] = the tile). One counter hands out both, so the ranges ascend
-// with the slabs. With no slab left the tile stays whole (slower, same result).
+// A tile whose list is longer than part_refs and than one share of the launch's
+// entries over the raster workgroups that the chip holds (or than split_refs,
+// whatever the share) is split over several raster workgroups: it takes a slab
+// (depth keys of its pixels), and its entries a range [split_first[slab], + count)
+// of the split tiles' entries put end to end (split_tile[slab] = the tile). One
+// counter hands out both, so the ranges ascend with the slabs. With no slab left
+// the tile stays whole (slower, same result).
+//
+// Lists up to a share end with the others anyway, and their parts cost a merge: 200,000
+// small triangles all over 2560x1440, k_raster 67 us with every list over 64 split, 46
+// so (20,000 of 60 pixels at 3840x2160 in 64x64 tiles 141 | 118). With two shares
+// instead of one, 500,000 faces in the middle of 1920x1080 take 114 us for 91.
 constexpr int kScanThreads = 1024;
 __global__ __launch_bounds__(kScanThreads) void k_bin_scan(
     const DevFrame* __restrict__ frames, int nframes, uint32_t* __restrict__ tile_counts,
@@ -1552,11 +1559,12 @@ __global__ __launch_bounds__(kScanThreads) void k_bin_scan(
     unsigned long long refs_capacity, uint32_t* __restrict__ tile_slab,
     uint32_t* __restrict__ split_first, uint32_t* __restrict__ split_tile, uint32_t max_slabs,
     uint32_t part_refs, uint32_t split_refs, uint32_t* __restrict__ rec_pool,
-    const FaceBlock* __restrict__ blocks) {
+    const FaceBlock* __restrict__ blocks, int total_tiles, float inv_held) {
     constexpr int NW = kScanThreads / 64;
     __shared__ unsigned long long wsum[NW], wsplit[NW];
     __shared__ uint32_t wstat[NW][4];
     __shared__ unsigned long long base_s, split_s;
+    __shared__ uint32_t longest_s;  // the longest list left whole
     const int f = blockIdx.x;
     const DevFrame& fr = frames[f];
     const int ntiles = fr.tiles_x * fr.tiles_y;
@@ -1571,6 +1579,19 @@ __global__ __launch_bounds__(kScanThreads) void k_bin_scan(
     for (int k = 0; k < kKeep; k++) {
         const int i = (int)threadIdx.x + k * kScanThreads;
         v0[k] = i < ntiles ? gld(&cnt[i]) : 0u;
+    }
+    // The launch's references, where parts are smaller than split_refs (launches of
+    // few tiles). A frame that overflowed may be clearing its own counts: its batch
+    // is drawn again.
+    const bool shared = nframes > 1 && part_refs < split_refs;  // at most kAllTiles tiles
+    constexpr int kAllTiles = 4 * kScanThreads;
+    uint4 all4 = make_uint4(0u, 0u, 0u, 0u);
+    uint32_t all1 = 0u;
+    if (shared) {
+        const int quads = min(total_tiles, kAllTiles) >> 2, i = 4 * quads + (int)threadIdx.x;
+        if ((int)threadIdx.x < quads)
+            all4 = gload(reinterpret_cast<const uint4*>(tile_counts) + threadIdx.x);
+        if (threadIdx.x < 3 && i < min(total_tiles, kAllTiles)) all1 = gld(&tile_counts[i]);
     }
 
     // k_face is done with the record pools: their total to the batch counters,
@@ -1619,11 +1640,22 @@ __global__ __launch_bounds__(kScanThreads) void k_bin_scan(
     for (int i = (int)threadIdx.x + kKeep * kScanThreads; i < ntiles; i += kScanThreads)
         local += gld(&cnt[i]);
     local = wave_sum_u64(local);
-    if (lane == 0) wsum[wave] = local;
+    unsigned long long all = local;
+    if (shared)
+        all = wave_sum_u64((unsigned long long)all4.x + all4.y + all4.z + all4.w + all1);
+    if (lane == 0) {
+        wsum[wave] = local;
+        wsplit[wave] = all;
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
         unsigned long long tot = 0;
-        for (int w = 0; w < NW; w++) tot += wsum[w];
+        all = 0;
+        for (int w = 0; w < NW; w++) {
+            tot += wsum[w];
+            all += wsplit[w];
+        }
+        longest_s = min(split_refs, max(part_refs, (uint32_t)((float)all * inv_held)));
         // One frame starts at 0, without waiting for the counter.
         unsigned long long base = 0;
         if (nframes > 1) base = atomicAdd(&counters->refs_used, tot);
@@ -1637,6 +1669,7 @@ __global__ __launch_bounds__(kScanThreads) void k_bin_scan(
     }
     __syncthreads();
     const bool over = frame_overflow[f] != 0u;
+    const uint32_t longest = longest_s;
     unsigned long long run = base_s;
     for (int c = 0; c < ntiles; c += kScanThreads) {
         const int i = c + (int)threadIdx.x;
@@ -1647,7 +1680,8 @@ __global__ __launch_bounds__(kScanThreads) void k_bin_scan(
             v = v0[1];
         else
             v = i < ntiles ? gld(&cnt[i]) : 0u;
-        const bool split = !over && v > part_refs;
+        const bool split = !over && v > longest;
+        if (v > part_refs && !split) tile_slab[fr.tile_begin + i] = kNoSlab;
         const uint64_t sm = ballot(split);
         const unsigned long long x = wave_scan_u64(v);
         const uint32_t sv = split ? v : 0u;
@@ -2760,7 +2794,8 @@ void launch_bin_scan(const LaunchParams& p, hipStream_t s) {
     hipLaunchKernelGGL(k_bin_scan, dim3(p.nframes), dim3(kScanThreads), 0, s, p.frames, p.nframes,
                        p.tile_counts, p.tile_offsets, p.tile_cursor, p.frame_overflow, p.stats,
                        p.counters, p.ctrl, p.refs_capacity, p.tile_slab, p.split_first,
-                       p.split_tile, p.max_slabs, p.part_refs, p.split_refs, p.rec_pool, p.blocks);
+                       p.split_tile, p.max_slabs, p.part_refs, p.split_refs, p.rec_pool, p.blocks,
+                       p.total_tiles, 1.0f / (256 * raster_waves(1 << (p.tw_log2 + p.th_log2))));
 }
 
 void launch_bin_fill(const LaunchParams& p, hipStream_t s) {

@@ -170,7 +170,9 @@ typedef struct {
     int32_t tile_split;           /* tile-list entries per raster workgroup, 64..2^24: a
                                      longer list is split into parts that several
                                      workgroups resolve (same result, more parallelism);
-                                     launches of at most 4096 tiles split from 64 on */
+                                     launches of at most 4096 tiles, with at most 64 MiB
+                                     of depth keys, also split lists of more than 64
+                                     that are longer than the others */
     int32_t pipelines;            /* 1 or 2 (default): with 2, consecutive asynchronous draws
                                      alternate between two sets of buffers and streams, so a
                                      draw's geometry stages overlap the previous draw's raster;

@@ -531,3 +531,34 @@ def test_binning_cost_follows_the_references(ctx):
     finally:
         ctx.set_kernel_timing(False)
         ctx.set_config(tile_w=old.tile_w, tile_h=old.tile_h, pipelines=old.pipelines)
+
+
+@pytest.mark.parametrize("n,px,tile", [(6000, 40, 8), (2500, 90, 16), (9000, 12, 8), (3000, 60, 64)])
+def test_split_shares(ctx, n, px, tile):
+    """Lists of over 64 entries in every tile, about as long as a share of the
+    launch's entries (some are left whole), alone and beside frames that leave one
+    frame's lists above the share of the batch or put them below it."""
+    scene = _soup(n, 512, 512, px)
+    light = _soup(200, 512, 512, 20, seed=3)
+    heavy = _soup(9000, 256, 256, 60, seed=4)
+    want = [refcpu.draw(s) for s in (scene, light, heavy)]
+    old = ctx.config()
+    ctx.set_config(tile_w=tile, tile_h=tile, refs_capacity=1 << 23)
+    try:
+        handles = [ctx.upload_scene(s)[0] for s in (scene, light, heavy)]
+        assert_same(scene, ctx.draw(scene, handles[0]), want[0])
+        for batch in ([0, 1], [0, 2], [1, 2, 0]) if tile > 8 else ([1], [2]):
+            frames = [(scene, light, heavy)[k] for k in batch]
+            outs = [ctx.frame_buffers(s.frame.width, s.frame.height) for s in frames]
+            ctx.draw_batch(frames, [handles[k] for k in batch], [(o[0].ptr, o[1].ptr) for o in outs])
+            ctx.synchronize()
+            stats = ctx.last_stats()
+            for j, k in enumerate(batch):
+                h, w = frames[j].frame.height, frames[j].frame.width
+                got = (outs[j][0].to_numpy(np.uint8, (h, w, 4)),
+                       outs[j][1].to_numpy(np.float32, (h, w)), stats[j])
+                assert_same(frames[j], got, want[k])
+                for b in outs[j]:
+                    b.free()
+    finally:
+        ctx.set_config(tile_w=old.tile_w, tile_h=old.tile_h, refs_capacity=old.refs_capacity)
