@@ -402,6 +402,7 @@ gr_status check_frame(gr_context* c, const gr_frame& fr, const gr_object* objs, 
 // buffers. Objects must be laid out frame by frame.
 struct Plan {
     int nf = 0, nobj = 0, fblocks = 0, dense_blocks = 0, tiles = 0;
+    int frame_tiles = 0;  // of the frame with the most
     int twl = 0, thl = 0;
     size_t okey_words = 0;
     bool decorate = false;  // a frame asks for tile borders or the crosshair
@@ -485,6 +486,7 @@ gr_status make_plan(gr_context* c, const gr_batch_frame* bf, int nf, const gr_ob
         d.tiles_y = (fr.height + TH - 1) / TH;
         d.tile_begin = P.tiles;
         P.tiles += d.tiles_x * d.tiles_y;
+        P.frame_tiles = std::max(P.frame_tiles, d.tiles_x * d.tiles_y);
         d.face_block_begin = P.fblocks;
         d.rgba = (uint8_t*)bf[f].d_rgba;
         d.depth = (float*)bf[f].d_depth;
@@ -636,6 +638,7 @@ gr::LaunchParams launch_params(const Plan& P, const Bufs& B) {
     p.textures = B.textures;
     p.face_blocks = P.fblocks;
     p.total_tiles = P.tiles;
+    p.frame_tiles = P.frame_tiles;
     p.tw_log2 = P.twl;
     p.th_log2 = P.thl;
     p.tile_counts = B.tile_counts;

@@ -2737,7 +2737,7 @@ void launch_face_normals(const float* pos, const int32_t* vi, int F, float* fn, 
     hipLaunchKernelGGL(k_face_normals, dim3((F + 255) / 256), dim3(256), 0, s, pos, vi, F, fn);
 }
 
-constexpr int kWideFaceBlocks = 4096;
+constexpr int kWideFaceBlocks = 4096, kWideFaceBlocksPast = 384;
 void launch_face(const LaunchParams& p, hipStream_t s) {
     if (p.face_blocks == 0) return;
     // Four waves a block for launches that leave the chip part idle, one past
@@ -2745,13 +2745,18 @@ void launch_face(const LaunchParams& p, hipStream_t s) {
     // on each of 1,024 SIMDs). us with one | four waves: 2 blocks 27.5 | 19.6,
     // 20 18.8 | 12.1, 157 29.5 | 18.8, 782 33.7 | 30.6, 4,000 57 | 50, 20,000
     // 254 | 262, 25,000 119 | 266, 38,000 279 | 458.
+    // In frames past the tile table (kTableTiles) a dense mesh is bound by the
+    // atomics of its tiles, which more waves at once only queue up longer (a sphere
+    // in the middle of 2560x1440: 200 blocks 42 | 41, 391 73 | 79, 586 100 | 125,
+    // 1,953 357 | 471); where it is not, four waves gain a few us, and a frame
+    // among others nothing, from 200 blocks on.
     auto launch = [&](auto kernel, int threads) {
         hipLaunchKernelGGL(kernel, dim3(p.face_grid), dim3(threads), 0, s, p.objs, p.frames,
                            p.tile_counts, p.blocks, p.tw_log2, p.th_log2, p.xcd_face,
                            p.obj_first, p.nframes, p.rec_pool, p.rec_pools, p.pool_recs,
                            p.ovf_begin, p.ctrl, p.frame_overflow);
     };
-    if (p.face_blocks <= kWideFaceBlocks)
+    if (p.face_blocks <= (p.frame_tiles <= kTableTiles ? kWideFaceBlocks : kWideFaceBlocksPast))
         launch(k_face<4>, 256);
     else
         launch(k_face<1>, 64);

@@ -562,3 +562,20 @@ def test_split_shares(ctx, n, px, tile):
                     b.free()
     finally:
         ctx.set_config(tile_w=old.tile_w, tile_h=old.tile_h, refs_capacity=old.refs_capacity)
+
+
+@pytest.mark.parametrize("size", [(512, 256), (520, 256)])
+@pytest.mark.parametrize("grid", [(190, 258), (191, 259)])
+def test_face_stage_forms_by_tiles(ctx, size, grid):
+    """383 and 387 face blocks, either side of the four-wave form's limit in frames
+    of more than 2,048 tiles, in a frame of 2,048 and in one of more."""
+    import scene_cases as C
+    scene = C.sphere(w=size[0], h=size[1], eye=(0, 0, 2.6), nlat=grid[0], nlon=grid[1])
+    blocks = -(-len(scene.meshes[0].vertex_indices) // 256)
+    assert (blocks <= 384) == (grid[0] == 190)
+    old = ctx.config()
+    ctx.set_config(tile_w=8, tile_h=8)
+    try:
+        assert_same(scene, ctx.draw(scene), refcpu.draw(scene))
+    finally:
+        ctx.set_config(tile_w=old.tile_w, tile_h=old.tile_h)
