@@ -593,9 +593,9 @@ struct Bufs {
 // triangles in flight 66 -> 44 us each with 64.)
 constexpr int kFineTiles = 4096;
 constexpr uint32_t kFinePart = 64;
-uint32_t part_size(const Plan& P, uint32_t tile_split, size_t slab_bytes,
+uint32_t part_size(int64_t tiles, uint32_t tile_split, size_t slab_bytes,
                    unsigned long long slab_budget) {
-    const bool fine = P.tiles <= kFineTiles && (unsigned long long)P.tiles * slab_bytes <= slab_budget;
+    const bool fine = tiles <= kFineTiles && (unsigned long long)tiles * slab_bytes <= slab_budget;
     return fine ? std::min(kFinePart, tile_split) : tile_split;
 }
 
@@ -742,7 +742,7 @@ gr_status size_bufs(gr_context* c, const Plan& P, Pipe& Q, unsigned long long re
     if ((st = ensure_zeroed(c, Q.tile_counts, (size_t)P.tiles * 4, s))) return st;
     if ((st = ensure(c, Q.tiles, 3 * (size_t)P.tiles * sizeof(uint32_t)))) return st;
     const size_t slab_bytes = (size_t)TW * TH * 8;
-    const uint32_t part_refs = part_size(P, tile_split, slab_bytes, kSlabBudget);
+    const uint32_t part_refs = part_size(P.tiles, tile_split, slab_bytes, kSlabBudget);
     const uint32_t max_slabs = slab_limit(P, refs_cap, part_refs, slab_bytes);
     if ((st = ensure(c, Q.splits, (2 * (size_t)max_slabs + 1) * sizeof(uint32_t)))) return st;
     if ((st = ensure_zeroed(c, Q.slabs, (size_t)max_slabs * (slab_bytes + 4), s))) return st;
@@ -1141,6 +1141,78 @@ gr_status graph_launch(gr_batch_graph* g) {
     return GR_OK;
 }
 
+// The autotuner's measurement of one configuration.
+struct TuneRun {
+    int split = 0;
+    double ms = 0.0;             // a launch
+    unsigned long long sum = 0;  // digest of every frame's colour and depth
+    unsigned long long refs = 0;
+    int64_t refs_capacity = 0;
+};
+
+// Longest list that a batch of `refs` entries leaves whole under `split` (k_bin_scan):
+// where two splits have the same one, they are the same program.
+uint32_t longest_whole(const gr_batch_frame* frames, int nf, int tw, int th, int split,
+                       unsigned long long refs) {
+    int64_t tiles = 0;
+    for (int f = 0; f < nf; f++)
+        tiles += (int64_t)((frames[f].frame.width + tw - 1) / tw) *
+                 ((frames[f].frame.height + th - 1) / th);
+    const uint32_t part = part_size(tiles, (uint32_t)split, (size_t)tw * th * 8, kSlabBudget);
+    if (part >= (uint32_t)split) return (uint32_t)split;
+    const float share = (float)refs / (float)gr::raster_workgroups(tw * th);
+    return std::min((uint32_t)split, std::max(part, (uint32_t)share));
+}
+
+// Times the context's present configuration, and gives it the tile-list capacity
+// that the batch needs plus a quarter.
+gr_status tune_run(gr_context* c, const gr_batch_frame* frames, int32_t nf, const gr_object* objs,
+                   int32_t no, int32_t reps, hipEvent_t ea, hipEvent_t eb,
+                   unsigned long long* d_sum, TuneRun* run) {
+    gr_status st;
+    // Untimed launch: grows the tile lists while they overflow, then sizes them to
+    // the batch's references plus a quarter.
+    unsigned long long needed = 0;
+    for (int attempt = 0;; attempt++) {
+        if ((st = enqueue(c, frames, nf, objs, no))) return st;
+        st = sync_and_check(c, &needed);
+        if (st != GR_ERR_CAPACITY) break;
+        if (attempt == 3) return fail(GR_ERR_CAPACITY, "tile-list capacity could not be satisfied");
+        grow_refs(c, needed);
+    }
+    if (st) return st;
+    std::vector<unsigned long long> sv;
+    if ((st = read_stats(c, sv))) return st;
+    run->refs = 0;
+    for (int f = 0; f < nf; f++) run->refs += sv[(size_t)f * gr::kNumStats + gr::kStatRefs];
+    // The capacity also holds the triangle records the face blocks claimed.
+    gr::DevBatchCounters bc;
+    GR_HIP(hipMemcpy(&bc, c->last_counters, sizeof bc, hipMemcpyDeviceToHost));
+    c->cfg.refs_capacity =
+        std::max<int64_t>(1 << 16, (int64_t)grown(std::max(run->refs, bc.recs_used)));
+    run->refs_capacity = c->cfg.refs_capacity;
+    GR_HIP(hipEventRecord(ea, c->stream));
+    for (int r = 0; r < reps; r++)
+        if ((st = enqueue(c, frames, nf, objs, no))) return st;
+    GR_HIP(hipEventRecord(eb, c->stream));
+    if ((st = sync_and_check(c, &needed))) return st;
+    float ms = 0.f;
+    GR_HIP(hipEventElapsedTime(&ms, ea, eb));
+    run->ms = (double)ms / reps;
+    // Digest of every frame's colour and depth.
+    gr::launch_fill32((uint32_t*)d_sum, 0u, 2, c->stream);
+    for (int f = 0; f < nf; f++) {
+        const size_t px = (size_t)frames[f].frame.width * frames[f].frame.height;
+        gr::launch_checksum(frames[f].d_rgba, px, d_sum, c->stream);
+        gr::launch_checksum(frames[f].d_depth, px, d_sum, c->stream);
+    }
+    GR_HIP(hipGetLastError());
+    GR_HIP(hipMemcpyAsync(c->h_ctrl, d_sum, 8, hipMemcpyDeviceToHost, c->stream));
+    GR_HIP(hipStreamSynchronize(c->stream));
+    std::memcpy(&run->sum, c->h_ctrl, 8);
+    return GR_OK;
+}
+
 void graph_free(gr_batch_graph* g) {
     graph_drop_exec(g);
     free_pipe_bufs(g->buf);
@@ -1286,7 +1358,7 @@ gr_status enqueue_noalloc(gr_context* c, const gr_frame* frame, const gr_object*
         // Split tiles (never counted in the statistics: the configured size does
         // not apply here).
         const size_t slab_bytes = (size_t)TW * TH * 8;
-        B.part_refs = part_size(P, 0xFFFFFFFFu, slab_bytes, kNoAllocSlabs);
+        B.part_refs = part_size(P.tiles, 0xFFFFFFFFu, slab_bytes, kNoAllocSlabs);
         B.split_refs = 0xFFFFFFFFu;
         if (B.part_refs != 0xFFFFFFFFu) {
             B.max_slabs = (uint32_t)P.tiles;
@@ -2221,72 +2293,43 @@ gr_status gr_autotune(gr_context* c, const gr_batch_frame* frames, int32_t nf,
         static const int kTiles[4] = {8, 16, 32, 64};
         static const int kSplits[4] = {256, 512, 1024, 4096};
         bool have_best = false, have_sum = false;
-        double best_ms = 0.0;
+        TuneRun fastest;
         unsigned long long first_sum = 0;
         gr_config best_cfg = saved;
         int32_t nres = 0;
         for (int tw : kTiles)
-            for (int th : kTiles)
+            for (int th : kTiles) {
+                std::vector<TuneRun> runs;  // of this tile shape
                 for (int split : kSplits) {
                     c->cfg = saved;
                     c->cfg.tile_w = tw;
                     c->cfg.tile_h = th;
                     c->cfg.tile_split = split;
-                    // Untimed launch: grows the tile lists while they overflow,
-                    // then sizes them to the batch's references plus a quarter.
-                    unsigned long long needed = 0;
-                    for (int attempt = 0;; attempt++) {
-                        if ((st = enqueue(c, frames, nf, objs, no))) return st;
-                        st = sync_and_check(c, &needed);
-                        if (st != GR_ERR_CAPACITY) break;
-                        if (attempt == 3)
-                            return fail(GR_ERR_CAPACITY, "tile-list capacity could not be satisfied");
-                        grow_refs(c, needed);
-                    }
-                    if (st) return st;
-                    std::vector<unsigned long long> sv;
-                    if ((st = read_stats(c, sv))) return st;
-                    unsigned long long refs = 0;
-                    for (int f = 0; f < nf; f++) refs += sv[(size_t)f * gr::kNumStats + gr::kStatRefs];
-                    // The capacity also holds the triangle records the face blocks claimed.
-                    gr::DevBatchCounters bc;
-                    GR_HIP(hipMemcpy(&bc, c->last_counters, sizeof bc, hipMemcpyDeviceToHost));
-                    refs = std::max(refs, bc.recs_used);
-                    c->cfg.refs_capacity = std::max<int64_t>(1 << 16, (int64_t)grown(refs));
-                    GR_HIP(hipEventRecord(ea, c->stream));
-                    for (int r = 0; r < reps; r++)
-                        if ((st = enqueue(c, frames, nf, objs, no))) return st;
-                    GR_HIP(hipEventRecord(eb, c->stream));
-                    if ((st = sync_and_check(c, &needed))) return st;
-                    float ms = 0.f;
-                    GR_HIP(hipEventElapsedTime(&ms, ea, eb));
-                    // Digest of every frame's colour and depth.
-                    gr::launch_fill32((uint32_t*)d_sum, 0u, 2, c->stream);
-                    for (int f = 0; f < nf; f++) {
-                        const size_t px = (size_t)frames[f].frame.width * frames[f].frame.height;
-                        gr::launch_checksum(frames[f].d_rgba, px, d_sum, c->stream);
-                        gr::launch_checksum(frames[f].d_depth, px, d_sum, c->stream);
-                    }
-                    GR_HIP(hipGetLastError());
-                    unsigned long long sum = 0;
-                    GR_HIP(hipMemcpyAsync(c->h_ctrl, d_sum, 8, hipMemcpyDeviceToHost, c->stream));
-                    GR_HIP(hipStreamSynchronize(c->stream));
-                    std::memcpy(&sum, c->h_ctrl, 8);
-                    const double per = (double)ms / reps;
+                    TuneRun run;
+                    for (const TuneRun& r : runs)
+                        if (longest_whole(frames, nf, tw, th, r.split, r.refs) ==
+                            longest_whole(frames, nf, tw, th, split, r.refs))
+                            run = r;  // the same program: timed once
+                    if (run.split == 0 &&
+                        (st = tune_run(c, frames, nf, objs, no, reps, ea, eb, d_sum, &run)))
+                        return st;
+                    run.split = split;
+                    c->cfg.refs_capacity = run.refs_capacity;
+                    runs.push_back(run);
                     if (results && nres < max_results) {
                         gr_tune_result& tr = results[nres];
                         tr.tile_w = tw;
                         tr.tile_h = th;
                         tr.tile_split = split;
                         tr.raster_waves = c->cfg.raster_waves;
-                        tr.ms_per_launch = per;
-                        tr.checksum = sum;
+                        tr.ms_per_launch = run.ms;
+                        tr.checksum = run.sum;
                         nres++;
                     }
                     if (!have_sum) {
-                        first_sum = sum;
+                        first_sum = run.sum;
                         have_sum = true;
-                    } else if (sum != first_sum) {
+                    } else if (run.sum != first_sum) {
                         c->cfg = saved;
                         if (num_results) *num_results = nres;
                         return fail(GR_ERR_DEVICE, "autotune: the image depends on the "
@@ -2295,12 +2338,18 @@ gr_status gr_autotune(gr_context* c, const gr_batch_frame* frames, int32_t nf,
                                                        std::to_string(th) + ", split " +
                                                        std::to_string(split) + ")");
                     }
-                    if (!have_best || per < best_ms) {
+                    if (!have_best || run.ms < fastest.ms) {
                         have_best = true;
-                        best_ms = per;
+                        fastest = run;
                         best_cfg = c->cfg;
                     }
                 }
+            }
+        // A tile_split that changes nothing for this batch stays as it was.
+        if (longest_whole(frames, nf, best_cfg.tile_w, best_cfg.tile_h, saved.tile_split,
+                          fastest.refs) ==
+            longest_whole(frames, nf, best_cfg.tile_w, best_cfg.tile_h, fastest.split, fastest.refs))
+            best_cfg.tile_split = saved.tile_split;
         best_cfg.pipelines = saved.pipelines;
         c->cfg = best_cfg;
         if (best) *best = best_cfg;

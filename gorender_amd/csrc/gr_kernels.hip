@@ -2737,6 +2737,8 @@ void launch_face_normals(const float* pos, const int32_t* vi, int F, float* fn, 
     hipLaunchKernelGGL(k_face_normals, dim3((F + 255) / 256), dim3(256), 0, s, pos, vi, F, fn);
 }
 
+int raster_workgroups(int npx) { return 256 * raster_waves(npx); }
+
 constexpr int kWideFaceBlocks = 4096, kWideFaceBlocksPast = 384;
 void launch_face(const LaunchParams& p, hipStream_t s) {
     if (p.face_blocks == 0) return;
@@ -2800,7 +2802,7 @@ void launch_bin_scan(const LaunchParams& p, hipStream_t s) {
                        p.tile_counts, p.tile_offsets, p.tile_cursor, p.frame_overflow, p.stats,
                        p.counters, p.ctrl, p.refs_capacity, p.tile_slab, p.split_first,
                        p.split_tile, p.max_slabs, p.part_refs, p.split_refs, p.rec_pool, p.blocks,
-                       p.total_tiles, 1.0f / (256 * raster_waves(1 << (p.tw_log2 + p.th_log2))));
+                       p.total_tiles, 1.0f / raster_workgroups(1 << (p.tw_log2 + p.th_log2)));
 }
 
 void launch_bin_fill(const LaunchParams& p, hipStream_t s) {
@@ -3003,7 +3005,7 @@ static void raster_t(const LaunchParams& p, hipStream_t s) {
     // 2,048 alike), and one time for a batch whose tiles alone fill the chip over
     // and over (64 mixed frames: one, two, four and eight times alike; they return
     // at once where nothing is split, 2,048 in 1 of 300 us, 8,192 in 4).
-    const int fill = 256 * raster_waves(TW * TH);
+    const int fill = raster_workgroups(TW * TH);
     const int most = p.total_tiles > 8 * fill ? fill : 4 * fill;
     const int extra =
         p.max_slabs ? (std::min(most, std::max(1024, p.total_tiles)) + 7) / 8 * 8 : 0;

@@ -91,6 +91,8 @@ void launch_fog(void* rgba, const void* depth, uint64_t n, float fog_start, floa
                 uint32_t color, hipStream_t s);
 void launch_bin_fill(const LaunchParams& p, hipStream_t s);
 bool launch_raster(const LaunchParams& p, hipStream_t s);
+// k_raster workgroups that the chip holds at a time, for tiles of npx pixels.
+int raster_workgroups(int npx);
 void launch_fill32(uint32_t* p, uint32_t v, size_t n, hipStream_t s);
 // Adds an order-independent digest of `words` 32-bit words at p to *out.
 void launch_checksum(const void* p, size_t words, unsigned long long* out, hipStream_t s);

@@ -286,7 +286,9 @@ void gr_batch_graph_destroy(gr_batch_graph *graph);
  * the context's config: raster tiles {8,16,32,64} x {8,16,32,64}, tile_split
  * {256, 512, 1024, 4096}, with the tile-list capacity sized to what the batch
  * needs plus a quarter. Each candidate is timed over `reps` launches (HIP
- * events, one pipe) after one untimed launch, and its frames' colour and depth
+ * events, one pipe) after one untimed launch (once for settings of tile_split
+ * that make no difference to the batch: they share the result, and tile_split stays
+ * as it was if it is one of them), and its frames' colour and depth
  * are checksummed on the device: the image may not depend on the
  * configuration, so a candidate whose checksum differs from the first's fails
  * the call (GR_ERR_DEVICE). results (may be NULL) receives up to max_results

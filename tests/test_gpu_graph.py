@@ -185,3 +185,26 @@ def test_autotune_keeps_the_image(ctx):
         ctx.set_config(tile_w=old.tile_w, tile_h=old.tile_h, tile_split=old.tile_split,
                        refs_capacity=old.refs_capacity)
         _free(outs)
+
+
+def test_autotune_times_the_same_program_once(ctx):
+    """Short lists in few tiles: no tile_split makes a difference, so each tile shape
+    is timed once for all of them and the context keeps the tile_split it had."""
+    scenes = [sphere(w=200, h=120, eye=(0, 0, 1.4)), sphere(w=160, h=96, eye=(0, 0, 3.0))]
+    handles = [ctx.upload_scene(s)[0] for s in scenes]
+    outs, ptrs = _outputs(ctx, scenes)
+    old = ctx.config()
+    try:
+        prepared = ctx.prepare_batch(scenes, handles, ptrs)
+        for split in (1024, 777):
+            ctx.set_config(tile_split=split)
+            best, tried = ctx.autotune(prepared, reps=2)
+            assert len(tried) == 64
+            for k in range(0, 64, 4):
+                assert [t["tile_split"] for t in tried[k:k + 4]] == [256, 512, 1024, 4096]
+                assert len({t["ms_per_launch"] for t in tried[k:k + 4]}) == 1
+            assert best["tile_split"] == ctx.config().tile_split == split
+    finally:
+        ctx.set_config(tile_w=old.tile_w, tile_h=old.tile_h, tile_split=old.tile_split,
+                       refs_capacity=old.refs_capacity)
+        _free(outs)
