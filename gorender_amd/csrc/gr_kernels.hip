@@ -147,13 +147,22 @@ __device__ __forceinline__ bool rcp_range(float d) {
 // RN(q + r*y) = RN(a/d) (Markstein, IBM J. Res. Dev. 34(1), 1990; the
 // Handbook of Floating-Point Arithmetic states it for any precision p).
 // Domain: d with rcp_range(d), a == +0 or 2^-70 <= |a| <= 2^70 (a == -0
-// would come back as +0 for d > 0).
+// would come back as +0 for d > 0). For another y see rcp_step.
 __device__ __forceinline__ float div_rcp(float a, float d, float y) {
     float q = a * y;
     float r = __builtin_fmaf(-d, q, a);
     q = __builtin_fmaf(r, y, q);
     r = __builtin_fmaf(-d, q, a);
     return __builtin_fmaf(r, y, q);
+}
+
+// A reciprocal of d for several quotients by the same divisor: the hardware's, and
+// one Newton step. It need not be the correctly rounded one, which div_rcp's theorem
+// asks for; that div_rcp(a, d, rcp_step(d)) is RN(a / d) all the same, for |d| in
+// [2^-41, 2^42] and |a| in [2^-80, 2^86], is what gr_check_exact_division tests.
+__device__ __forceinline__ float rcp_step(float d) {
+    const float y = __builtin_amdgcn_rcpf(d);
+    return __builtin_fmaf(__builtin_fmaf(-d, y, 1.0f), y, y);
 }
 
 // ---------------------------------------------------------------------------
@@ -2451,21 +2460,15 @@ __device__ __forceinline__ unsigned long long shade_tile(const DevFrame& fr, int
                     __builtin_memcpy(&t, w, sizeof(DevTexture));
                     float u, v;
                     if (fast && __builtin_fabsf(t.scale) >= 0x1p-40f && __builtin_fabsf(t.scale) <= 0x1p10f) {
-                        // Both quotients from one reciprocal: what the compiler
-                        // makes of a division (reciprocal, one Newton step, two
-                        // residual corrections, all fused) without its scaling
-                        // and its special cases, which do nothing for z in
-                        // [2^-41, 2^42] and |numerator| in [2^-80, 2^86]. Below,
+                        // Both quotients from one reciprocal (rcp_step), for
+                        // |numerator| in [2^-80, 2^86] the exact ones. Below,
                         // |u| < 2^-38: 1 - u is 1, and v * scale * h is under 1
                         // either way. Above, a quotient is the same one, or at
                         // least 2^127, infinite or a NaN, and so past int64 once
-                        // scaled, in both ways. (Checked on the device: 128
-                        // numerators for each of the 2^23 significands of z,
-                        // the ranges' ends included, all the same bits.)
-                        const float y0 = __builtin_amdgcn_rcpf(b.zrec);
-                        const float y1 = __builtin_fmaf(__builtin_fmaf(-b.zrec, y0, 1.0f), y0, y0);
-                        u = div_rcp(un, b.zrec, y1);
-                        v = div_rcp(vn, b.zrec, y1);
+                        // scaled, in both ways.
+                        const float y = rcp_step(b.zrec);
+                        u = div_rcp(un, b.zrec, y);
+                        v = div_rcp(vn, b.zrec, y);
                     } else {
                         u = un / b.zrec;
                         v = vn / b.zrec;
@@ -2816,7 +2819,9 @@ void launch_bin_fill(const LaunchParams& p, hipStream_t s) {
 // + i) in four families over the documented domain (|d| in [2^-40, 2^41),
 // |a| in [2^-70, 2^70] or +0): random floats; quotients next to a rounding
 // midpoint; divisors with extreme mantissas (all ones, powers of two); integer
-// numerators over integer divisors as the raster stage divides them.
+// numerators over integer divisors as the raster stage divides them. Each pair is
+// then taken once more for the quotients of a shared reciprocal (rcp_step), with
+// exponents over its own domain, the ends included.
 __device__ __forceinline__ uint64_t splitmix64(uint64_t x) {
     x += 0x9E3779B97F4A7C15ull;
     x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
@@ -2831,7 +2836,6 @@ __device__ __forceinline__ float make_float(uint32_t sign, int exp, uint32_t man
 __global__ __launch_bounds__(256) void k_check_div(uint64_t n, uint64_t seed,
                                                    unsigned long long* mismatches,
                                                    float* first_bad) {
-    unsigned long long bad = 0;
     for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n;
          i += (uint64_t)gridDim.x * 256) {
         const uint64_t r0 = splitmix64(seed + 2 * i), r1 = splitmix64(seed + 2 * i + 1);
@@ -2861,20 +2865,32 @@ __global__ __launch_bounds__(256) void k_check_div(uint64_t n, uint64_t seed,
             a = (float)(int32_t)(((r1 >> 16) & 0x7FFFFFFFu) | 1u) * ((r1 >> 63) ? -1.0f : 1.0f);
             if (((r1 >> 8) & 3) == 0) a = (float)(int32_t)((r1 >> 20) & 0xFFF) + 1.0f;
         }
-        const float y = 1.0f / d;
-        const float want = a / d;
-        const float got = div_rcp(a, d, y);
-        if (__float_as_uint(want) != __float_as_uint(got)) {
-            if (atomicAdd(mismatches, 1ull) == 0ull) {
-                first_bad[0] = a;
-                first_bad[1] = d;
+        auto check = [&](float num, float div, float y) {
+            const float want = num / div;
+            const float got = div_rcp(num, div, y);
+            if (__float_as_uint(want) != __float_as_uint(got) &&
+                atomicAdd(mismatches, 1ull) == 0ull) {
+                first_bad[0] = num;
+                first_bad[1] = div;
                 first_bad[2] = want;
                 first_bad[3] = got;
             }
-            bad++;
+        };
+        check(a, d, 1.0f / d);
+        // z of the pair's significand in [2^-41, 2^42]; a of its own in [2^-80, 2^86]
+        // (the next to a midpoint: the product with z of a float plus half an ulp).
+        const uint64_t r2 = splitmix64(r0 ^ r1);
+        const int ez = (int)(r2 % 84) - 41, ea = (int)((r2 >> 8) % 167) - 80;
+        const float z = make_float((uint32_t)(r2 >> 63), ez, ez == 42 ? 0u : __float_as_uint(d));
+        float num = make_float((uint32_t)(r2 >> 62) & 1u, ea, ea == 86 ? 0u : __float_as_uint(a));
+        if (fam == 1) {
+            const int em = (int)((r2 >> 16) % 101) - 50;
+            num = (float)((double)z * ((double)make_float(0, em, (uint32_t)(r2 >> 24)) +
+                                       ldexp(1.0, em - 24)));
+            if (__builtin_fabsf(num) < 0x1p-80f || __builtin_fabsf(num) > 0x1p86f) num = 1.0f;
         }
+        check(num, z, rcp_step(z));
     }
-    (void)bad;
 }
 
 void launch_check_div(uint64_t n, uint64_t seed, unsigned long long* mismatches, float* first_bad,

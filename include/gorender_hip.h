@@ -458,9 +458,11 @@ void gr_reset_kernel_times(gr_context *ctx);
 /* ---- self-check (no reference counterpart) ----
  * The raster stage divides by per-triangle divisors through their correctly
  * rounded reciprocals and two residual corrections, which equals IEEE float32
- * division on the divisor/numerator ranges it admits. This runs `count` pairs
- * drawn from `seed` over those ranges on the device, compares both quotients
- * bit for bit, and returns the mismatch count; first_mismatch (4 floats, may
+ * division on the divisor/numerator ranges it admits; the shading pass divides two
+ * numerators by one depth through a reciprocal that need not be correctly rounded,
+ * over ranges of its own. This runs `count` pairs drawn from `seed` over each of
+ * those ranges on the device, compares the quotients bit for bit, and returns the
+ * mismatch count; first_mismatch (4 floats, may
  * be NULL) receives numerator, divisor, IEEE quotient, tested quotient. */
 gr_status gr_check_exact_division(gr_context *ctx, uint64_t count, uint64_t seed,
                                   uint64_t *mismatches, float *first_mismatch);

@@ -23,3 +23,18 @@ def test_exact_division_matches_ieee(ctx, seed):
     _lib.check(ctx.lib.gr_check_exact_division(ctx.handle, n, seed, ctypes.byref(bad), first))
     assert bad.value == 0, (f"{bad.value} of {n} quotients differ; first: a={first[0]!r} "
                             f"d={first[1]!r} ieee={first[2]!r} got={first[3]!r}")
+
+
+@pytest.mark.parametrize("count", [1, 255, 257, 1 << 28])
+def test_shared_reciprocal_matches_ieee(ctx, count):
+    """The same call takes the shading pass's quotients by a shared reciprocal (the
+    hardware's and one Newton step) over the depths and numerators of that pass: few
+    pairs (one workgroup, a broken one), and a quarter of a billion, a quarter of
+    them next to a rounding midpoint."""
+    bad = ctypes.c_uint64(1)
+    first = (ctypes.c_float * 4)()
+    from gorender_amd import _lib
+    _lib.check(ctx.lib.gr_check_exact_division(ctx.handle, count, 0xD1F5 + count,
+                                               ctypes.byref(bad), first))
+    assert bad.value == 0, (f"{bad.value} quotients differ; first: a={first[0]!r} "
+                            f"d={first[1]!r} ieee={first[2]!r} got={first[3]!r}")
