@@ -26,7 +26,8 @@ constexpr int kHelpers = 3;
 // The helper threads of the process. They live until it ends: the pool is never
 // destroyed, and a thread that waits holds nothing. The caller copies too and
 // takes every piece no helper has taken, so a copy never depends on them (a forked
-// child, which has none, copies alone).
+// child, which has none, copies alone). The library is linked never to be unloaded,
+// since they wait in its code.
 class CopyPool {
 public:
     void copy(char* dst, const char* src, size_t n) {

@@ -1,6 +1,7 @@
 """gr_host_copy and the arrays that frames are delivered in (no GPU needed)."""
 import os
 import signal
+import subprocess
 import sys
 import threading
 
@@ -148,3 +149,22 @@ def test_host_copy_in_a_forked_child():
         ok = lib.gr_host_copy(dst.ctypes.data, src.ctypes.data, src.nbytes) == 0
         os._exit(0 if ok and np.array_equal(src, dst) else 1)
     assert os.waitpid(pid, 0)[1] == 0
+
+
+def test_library_stays_while_its_threads_wait():
+    """Closing the library leaves its code mapped: helper threads wait in it."""
+    code = (
+        "import _ctypes, ctypes, sys\n"
+        "lib = ctypes.CDLL(sys.argv[1])\n"
+        "a, b = ctypes.create_string_buffer(b'x' * (8 << 20)), ctypes.create_string_buffer(8 << 20)\n"
+        "n = ctypes.c_size_t(8 << 20)\n"
+        "assert lib.gr_host_copy(b, a, n) == 0 and b.raw[: 8 << 20] == a.raw[: 8 << 20]\n"
+        "_ctypes.dlclose(lib._handle)\n"
+        "assert sys.argv[1] in open('/proc/self/maps').read(), 'unmapped'\n"
+        "again = ctypes.CDLL(sys.argv[1])\n"
+        "ctypes.memset(b, 0, 8 << 20)\n"
+        "assert again.gr_host_copy(b, a, n) == 0 and b.raw[: 8 << 20] == a.raw[: 8 << 20]\n")
+    path = os.path.realpath(_lib.ALT_LIB_PATH or _lib.LIB_PATH)
+    r = subprocess.run([sys.executable, "-c", code, path], capture_output=True, text=True,
+                       timeout=120)
+    assert r.returncode == 0, r.stderr[-2000:]
