@@ -14,8 +14,8 @@
 #include <thread>
 
 #include "gorender_hip.h"
+#include "gr_copy.h"
 #include "gr_error.h"
-#include "gr_internal.h"
 
 namespace {
 

@@ -6,6 +6,7 @@
 #include <stddef.h>
 
 #include "gorender_hip.h"
+#include "gr_copy.h"
 
 namespace gr_internal {
 
@@ -33,8 +34,6 @@ void grow_refs_to(gr_context* c, unsigned long long needed);
 // and message a batch holding it would fail with.
 gr_status check_request(gr_context* c, const gr_frame* frame, const gr_object* objects,
                         int32_t num_objects);
-// Copy of host memory, shared by several threads when it is large (gr_copy.cpp).
-void host_copy(void* dst, const void* src, size_t n);
 // Pinned memory that host_copy reads, its pages mapped by this thread. Left to the
 // first copy, its threads take the faults of the same 2 MB pages at once and each
 // does all of the work: the first copy of a 1280x720 frame took 310-450 us, 130 so.

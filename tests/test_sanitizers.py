@@ -8,6 +8,8 @@ import os
 import subprocess
 import sys
 
+import pytest
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SAN_LIB = os.path.join(ROOT, "gorender_amd", "csrc", "_sanitize", "libgorender_host_san.so")
 SAN_ORACLE = os.path.join(ROOT, "oracle", "build", "librefcpu_san.so")
@@ -40,3 +42,17 @@ def test_host_code_under_asan_and_ubsan():
     for marker in ("AddressSanitizer", "runtime error:", "LeakSanitizer"):
         assert marker not in out, out[-6000:]
     assert " passed" in out, out[-2000:]
+
+
+@pytest.mark.parametrize("kind", ["thread", "address"])
+def test_host_copy_under_sanitizers(kind):
+    """The copy that several threads share (gr_copy.cpp): callers at once, sizes
+    around its pieces, a forked child. Any report fails the program."""
+    subprocess.run(["make", "-s", "-C", os.path.join(ROOT, "gorender_amd", "csrc"), "sanitize"],
+                   check=True)
+    prog = os.path.join(ROOT, "gorender_amd", "csrc", "_sanitize", f"copy_check_{kind}")
+    env = dict(os.environ, TSAN_OPTIONS="halt_on_error=1", ASAN_OPTIONS="detect_leaks=0",
+               UBSAN_OPTIONS="halt_on_error=1")
+    r = subprocess.run([prog], env=env, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and r.stdout == "0 wrong\n", (r.stdout + r.stderr)[-6000:]
+    assert "Sanitizer" not in r.stderr, r.stderr[-6000:]
