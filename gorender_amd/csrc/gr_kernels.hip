@@ -600,8 +600,10 @@ __device__ __forceinline__ bool ov_line(const DevFrame& fr, int64_t x0, int64_t 
     const float xs = (float)dx / (float)side, ys = (float)dy / (float)side;
     float cx = (float)x0, cy = (float)y0;
     if (near_origin(x0, y0) && near_origin(x1, y1)) {
-        // The positions stay within a pixel of the endpoints' range, where
-        // int() is the 32-bit conversion (and one position if side is 0).
+        // At most 2^16 steps, each rounded by half a unit in the last place of a
+        // number below 2^17 (2^-8): the positions drift by 257 pixels at most, so
+        // int() is the 32-bit conversion and y * W + x, with W <= 2^14, stays
+        // below 2^31 (one position if side is 0).
         for (int i = 0; i <= (int)side; i++) {
             ov_pixel32(fr, (int)cx, (int)cy, code);
             cx += xs;

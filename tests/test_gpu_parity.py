@@ -579,3 +579,26 @@ def test_face_stage_forms_by_tiles(ctx, size, grid):
         assert_same(scene, ctx.draw(scene), refcpu.draw(scene))
     finally:
         ctx.set_config(tile_w=old.tile_w, tile_h=old.tile_h)
+
+
+@pytest.mark.parametrize("size", [(16384, 9), (9, 16384), (8191, 65)])
+def test_overlays_long_lines(ctx, size):
+    """Edges of tens of thousands of steps whose float32 positions drift by many
+    pixels, shallow and steep, across wide and tall frames and far beside them."""
+    w, h = size
+    far = 45000.0
+    px = np.array([[-far, 3], [5000, h - 2], [w / 2, -far],
+                   [w / 3, far], [w + 20000.0, h / 2], [-20000.0, 2],
+                   [-40000, -40000], [3000, 4000], [w - 3, h - 3],
+                   [-32768, 32768], [32000, 49221], [w / 2, h / 2]], np.float64)
+    v = np.ones((12, 4), np.float32)
+    v[:, 0], v[:, 1] = (px[:, 0] - w / 2) / (w / 2), (px[:, 1] - h / 2) / (h / 2)
+    v[:, 2] = 0.5
+    flags = _lib.GR_SHOW_FACES | _lib.GR_SHOW_EDGES | _lib.GR_SHOW_VERTICES
+    f = np.arange(12, dtype=np.int32).reshape(4, 3)
+    eye = np.eye(4, dtype=np.float32)
+    scene = S.SceneData(S.FrameData(w, h, flags=flags), [S.MeshData(v, f)], [],
+                        [S.ObjectData(0, eye, eye)], name=f"long-{w}")
+    want = refcpu.draw(scene)
+    assert (want[0][..., :3] == 0).all(-1).sum() > 50  # edge pixels in the frame
+    assert_same(scene, ctx.draw(scene), want)
