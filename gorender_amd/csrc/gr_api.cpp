@@ -497,7 +497,6 @@ gr_status make_plan(gr_context* c, const gr_batch_frame* bf, int nf, const gr_ob
             d.okey = (uint32_t*)(uintptr_t)(P.okey_words * 4 + 1);
             P.okey_words += (size_t)fr.width * fr.height;
         }
-        int seq = 0;
         d.obj_begin = nobj;
         d.obj_count = bf[f].num_objects;
         for (int k = 0; k < bf[f].num_objects; k++) {
@@ -508,16 +507,13 @@ gr_status make_plan(gr_context* c, const gr_batch_frame* bf, int nf, const gr_ob
             o.m = mr.dm;
             std::memcpy(o.mvp, ob.mvp, sizeof o.mvp);
             std::memcpy(o.world, ob.world, sizeof o.world);
-            o.frame = f;
             o.gouraud = (fr.flags & GR_LIGHTING) && !(fr.flags & GR_FLAT_SHADING) && mr.dm.N > 0;
             o.dense = dense_on_screen(ob.mvp, mr.dm.bbox, mr.dm.F, fr.width, fr.height) ? 1 : 0;
             o.vis = gr_box_visibility(ob.mvp, &mr.dm.bbox[0][0], fr.znear, fr.zfar);
             o.face_blocks = (mr.dm.F + gr::kFacesPerWg - 1) / gr::kFacesPerWg;
             o.face_block = P.fblocks;
-            o.seq_block = seq;
             P.fblocks += o.face_blocks;
             if (o.dense) P.dense_blocks += o.face_blocks;
-            seq += o.face_blocks;
         }
         d.face_blocks = P.fblocks - d.face_block_begin;
         // Set to the batch's record arrays by write_header (orec: 1 = overlays).
@@ -985,9 +981,8 @@ void free_pipe_bufs(Pipe& pp) {
 }  // namespace
 
 // One batch's launch sequence captured in two HIP graphs, with its own device
-// buffers: counter zeroing, k_face, k_bin_scan, k_bin_fill, k_overlay and
-// k_overlay in the geometry graph; k_raster and k_decorate in the raster
-// graph, so that a replay's raster can wait for the previous batch's between
+// buffers: counter zeroing, k_face, k_bin_scan, k_bin_fill and k_overlay in the
+// geometry graph; k_raster and k_decorate in the raster graph, so that a replay's raster can wait for the previous batch's between
 // the two graph launches while its geometry overlaps that raster.
 struct gr_batch_graph {
     gr_context* c = nullptr;
@@ -1280,9 +1275,9 @@ gr_status check_request(gr_context* c, const gr_frame* frame, const gr_object* o
 
 // The no-allocation draw. Layout of [base, base + bytes): control words (sticky
 // until gr_synchronize reads them), batch header, texture table, tile counters,
-// tile offsets/cursors/slabs, 8 bytes per face block, then what remains shared
-// between triangle records and tile-list entries, as many of each (fewer records
-// when the frame has fewer slots). Behind the array's `bytes`, which decide what
+// tile offsets/cursors/slabs, a gap of 8 bytes per face block, then what remains
+// shared between triangle records and tile-list entries, as many of each (fewer
+// records when the frame has fewer slots). Behind the array's `bytes`, which decide what
 // fits a draw, its tail of kNoAllocTail bytes holds the face blocks' state and the
 // slabs of split tiles; frames of more tiles than slabs are drawn without splits.
 // Host data reaches the array through kernel arguments, and what must start at
@@ -1328,6 +1323,8 @@ gr_status enqueue_noalloc(gr_context* c, const gr_frame* frame, const gr_object*
         B.tile_counts = (uint32_t*)take((size_t)P.tiles * 4);
         B.tiles = (uint32_t*)take(3 * (size_t)P.tiles * 4);
         B.rec_pool = (uint32_t*)take(kPoolWords * 4);
+        // Nothing is here: the face blocks' state is in the tail, but what remains
+        // for lists, and so which frames fit, stays what it was with it here.
         off += 2 * align256((size_t)std::max(P.fblocks, 1) * 4);
         B.blocks = (gr::FaceBlock*)((char*)base + bytes);
         constexpr size_t kRecBytes =

@@ -73,11 +73,9 @@ struct DevObject {
     DevMesh m;
     float mvp[16];
     float world[16];
-    int32_t frame;          // index in the batch
     int32_t gouraud;        // vertex-normal lighting in use
     int32_t face_block;     // first k_face block (batch-global)
     int32_t face_blocks;    // number of k_face blocks
-    int32_t seq_block;      // first face block index within the frame (draw order)
     int32_t dense;          // >= 1 face per 4 pixels of the projected bounding box
     int32_t vis;            // BoxVisibility of the object (kBoxOutside/Intersect/Inside)
 };

@@ -47,24 +47,6 @@ __device__ __forceinline__ uint32_t go_uint8(float x) {
     return __builtin_fabsf(x) < 2147483648.0f ? (uint32_t)(int32_t)x & 0xFFu : 0u;
 }
 
-__device__ __forceinline__ bool f_signbit(float a) { return (__float_as_uint(a) >> 31) != 0; }
-
-// Go builtin min/max on floats: NaN wins, min(-0,+0) = -0.
-__device__ __forceinline__ float go_min(float a, float b) {
-    if (a != a) return a;
-    if (b != b) return b;
-    if (a < b) return a;
-    if (b < a) return b;
-    return f_signbit(a) ? a : b;
-}
-__device__ __forceinline__ float go_max(float a, float b) {
-    if (a != a) return a;
-    if (b != b) return b;
-    if (a > b) return a;
-    if (b > a) return b;
-    return f_signbit(a) ? b : a;
-}
-
 __device__ __forceinline__ int64_t wadd(int64_t a, int64_t b) {
     return (int64_t)((uint64_t)a + (uint64_t)b);
 }
@@ -2605,7 +2587,9 @@ __device__ __forceinline__ void raster_part(
         }
         // Device-scope atomics are performed at memory, and counted as complete
         // only then: every wave's merges are in the slab before its workgroup
-        // counts itself done. (A device-scope fence would write back and
+        // counts itself done. This rests on gfx950, not on the memory model, which
+        // promises an order between the relaxed atomics of the slab and of its
+        // counter only with a release and an acquire. (Those write back and
         // invalidate the XCD's L2 in every part: 458 -> 1,220 us for 8 dense
         // requests.)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

@@ -244,11 +244,13 @@ gr_status gr_draw_batch(gr_context *ctx, const gr_batch_frame *frames, int32_t n
 /* gr_draw_device that allocates nothing: no counterpart in the reference, for
  * callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc). Every per-draw buffer
- * lives in one fixed 32 MiB device array per GPU, held until the process ends;
+ * lives in one fixed device array per GPU (49 MiB: 32 for the draw, the rest for
+ * the parts of long tile lists), which every process that loads the library holds
+ * until it ends;
  * host data reaches it through kernel arguments, and the draw calls no
  * allocation, free or memset. Limits: one frame of at most 16 objects, no edge
  * or vertex overlays (GR_ERR_UNSUPPORTED), and the frame's tile counters, 320
- * triangle records per 256 faces and 2^16 tile-list entries within 32 MiB
+ * triangle records per 256 faces and 2^16 tile-list entries within those 32 MiB
  * (about 130k faces at 1080p): larger frames -> GR_ERR_INVALID_ARGUMENT. Tile
  * lists or clipped triangles beyond what is left of the array ->
  * GR_ERR_CAPACITY from gr_synchronize. The array is
