@@ -1743,7 +1743,6 @@ __global__ __launch_bounds__(kFillThreads) void k_bin_fill(const DevFrame* __res
     constexpr uint32_t kFillKeep = 256;
     __shared__ uint2 lrange[kFillKeep];  // tx0 | tx1 << 16, ty0 | ty1 << 16
     uint32_t ux = 0u, uy = 0u;  // union: last + 1 | (0xFFFF - first) << 16
-    uint32_t nrefs = 0u;        // references
     for (uint32_t i = threadIdx.x; i < cnt; i += kFillThreads) {
         const uint32_t ri = block_rec(b, ovf, i);
         const TileRect t = rec_tiles(&fr.rrec[ri], twl, thl);
@@ -1753,7 +1752,6 @@ __global__ __launch_bounds__(kFillThreads) void k_bin_fill(const DevFrame* __res
         if (t.tx0 > t.tx1) continue;
         ux = max_u16x2(ux, (uint32_t)(t.tx1 + 1) | (uint32_t)(0xFFFF - t.tx0) << 16);
         uy = max_u16x2(uy, (uint32_t)(t.ty1 + 1) | (uint32_t)(0xFFFF - t.ty0) << 16);
-        nrefs += (uint32_t)((t.tx1 - t.tx0 + 1) * (t.ty1 - t.ty0 + 1));
     }
     // fn(t, i) for the tile range of every record i, 64 records at a time by all
     // lanes of the wave (empty past the last record).
@@ -1816,18 +1814,31 @@ __global__ __launch_bounds__(kFillThreads) void k_bin_fill(const DevFrame* __res
     // The union in windows of at most kLdsTiles tiles.
     const int ww = min(rx1 - rx0 + 1, kLdsTiles), wh = min(ry1 - ry0 + 1, kLdsTiles / ww);
     const uint32_t windows = (uint32_t)((rx1 - rx0) / ww + 1) * (uint32_t)((ry1 - ry0) / wh + 1);
-    nrefs = wave_sum_u32(nrefs);
-    // Triangles scattered over a large frame: one global atomic per reference, where
-    // that is less than what the further windows cost (each clears and scans its
-    // counters and goes through all records twice, some 8 us). The line falls with
-    // the blocks of the frame, whose atomics queue up at the same cache lines. us by
-    // windows | by references, 32x32 tiles but where stated: 20,000 triangles of 8
-    // pixels at 3840x2160 90 | 14, at 7680x4320 238 | 14, of 60 pixels 154 | 49 and
-    // 437 | 49; 200,000 of 30 pixels at 1920x1080 78 | 176, at 2560x1440 83 | 111, at
-    // 3840x2160 137 | 60; 2,000 of 150 pixels at 1920x1080 87 | 121, at 2560x1440
-    // 180 | 149; 20,000 of 60 pixels at 1280x720 in 8x8 tiles 498 | 351.
-    const uint32_t sparse = max(64u, min(8192u, 300000u / (uint32_t)max(fr.face_blocks, 1)));
-    if (nrefs < sparse * (windows - 1u)) {
+    bool sparse = false;
+    if (windows > 1u) {
+        // Triangles scattered over a large frame: one global atomic per reference,
+        // where that is less than the windows cost. A lane's atomics in a row take
+        // some 0.4 us each; a window some 8 us, and 0.06 for every step of those rows
+        // that falls into it (about half do). Many atomics queue up at the cache
+        // lines of the frame's tiles, so the more face blocks, the fewer references.
+        // us by windows | by references, 32x32 tiles but where stated: 20,000
+        // triangles of 8 pixels at 3840x2160 90 | 14, at 7680x4320 238 | 14, of 60
+        // pixels 154 | 49 and 437 | 49; 200,000 of 30 pixels at 1920x1080 78 | 176,
+        // at 2560x1440 83 | 111, at 3840x2160 137 | 60; 2,000 of 150 pixels at
+        // 1920x1080 87 | 121, at 3840x2160 304 | 154; 20,000 of 60 pixels at 1280x720
+        // in 8x8 tiles 498 | 351; a sphere of 212 faces at 1920x1080 43 | 77.
+        uint32_t row = 0u, nrefs = 0u;  // atomics in a row; references
+        each_range([&](const TileRect& t, uint32_t) {
+            const uint32_t m = (uint32_t)((t.tx1 - t.tx0 + 1) * (t.ty1 - t.ty0 + 1));
+            row += wave_reduce(m, 0u, [](uint32_t a, uint32_t b) { return a > b ? a : b; });
+            nrefs += m;
+        });
+        nrefs = wave_sum_u32(nrefs);
+        const uint32_t most = min(8192u, 300000u / (uint32_t)max(fr.face_blocks, 1));
+        sparse = nrefs < max(64u, most) * (windows - 1u) &&
+                 0.4f * (float)row < (float)windows * (8.f + 0.06f * (float)row);
+    }
+    if (sparse) {
         each_ref(rx0, ry0, rx1, ry1, [&](int tx, int ty, uint32_t i) {
             refs[atomicAdd(&tile_cursor[fr.tile_begin + ty * fr.tiles_x + tx], 1u)] = slot0 + i;
         });
