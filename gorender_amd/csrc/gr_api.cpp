@@ -1229,8 +1229,7 @@ gr_status fail(gr_status s, const std::string& msg) { return ::fail(s, msg); }
 
 hipError_t pinned_alloc(void** p, size_t bytes) {
     const hipError_t e = hipHostMalloc(p, bytes, hipHostMallocDefault);
-    if (e == hipSuccess)
-        for (size_t b = 0; b < bytes; b += 4096) ((volatile char*)*p)[b] = 0;
+    if (e == hipSuccess) host_touch(*p, bytes);
     return e;
 }
 

@@ -2,7 +2,8 @@
 // moves ~28 GB/s, half the rate at which the GPU delivers frames over PCIe, so a
 // large copy is shared by the caller and a few helper threads (with reused result
 // arrays: 8 requests delivered to the host 6.5 -> 3.0 ms, two presented 1280x720
-// frames 571 -> 358 us; five or seven helpers gave no more).
+// frames 571 -> 358 us; five or seven helpers gave no more). New pinned memory is
+// mapped by the same threads, each taking large pages of its own.
 #include <sched.h>
 #include <unistd.h>
 
@@ -21,6 +22,7 @@ namespace {
 
 constexpr size_t kShared = 512u << 10;  // least bytes worth waking the helpers for
 constexpr size_t kPiece = 128u << 10;   // bytes a thread takes at a time
+constexpr size_t kPage = 2u << 20;      // bytes a fault of pinned memory maps at most
 constexpr int kHelpers = 3;
 
 // The helper threads of the process. They live until it ends: the pool is never
@@ -31,14 +33,40 @@ constexpr int kHelpers = 3;
 class CopyPool {
 public:
     void copy(char* dst, const char* src, size_t n) {
-        // One shared copy at a time; another thread's is not waited for. A forked
+        run(Job{dst, src, n, 0, kPiece, (n + kPiece - 1) / kPiece, 0});
+    }
+    // Clears a byte of every page of [p, p + n), large page by large page.
+    void touch(char* p, size_t n) {
+        const size_t skew = (uintptr_t)p % kPage;
+        run(Job{p, nullptr, n, skew, kPage, (skew + n + kPage - 1) / kPage, 0});
+    }
+
+private:
+    // Piece k is what lies in [0, n) of [k * piece - skew, (k + 1) * piece - skew).
+    struct Job {
+        char* dst;
+        const char* src;  // null: dst is touched
+        size_t n, skew, piece, pieces;
+        uint64_t id;
+        void one(size_t k) const {
+            const size_t b = k == 0 ? 0 : k * piece - skew;
+            const size_t e = (k + 1) * piece - skew < n ? (k + 1) * piece - skew : n;
+            if (src)
+                std::memcpy(dst + b, src + b, e - b);
+            else
+                for (size_t i = b; i < e; i += 4096 - (uintptr_t)(dst + i) % 4096)
+                    ((volatile char*)dst)[i] = 0;
+        }
+    };
+
+    void run(Job job) {
+        // One shared job at a time; another thread's is not waited for. A forked
         // child has no helpers.
         std::unique_lock<std::mutex> turn(turn_, std::try_to_lock);
         if (!turn.owns_lock() || !start() || getpid() != owner_) {
-            std::memcpy(dst, src, n);
+            for (size_t k = 0; k < job.pieces; k++) job.one(k);
             return;
         }
-        Job job{dst, src, n, (n + kPiece - 1) / kPiece, 0};
         {
             std::lock_guard<std::mutex> lk(mu_);
             job.id = ++id_;
@@ -51,14 +79,6 @@ public:
         while (done_.load(std::memory_order_acquire) != job.pieces) std::this_thread::yield();
     }
 
-private:
-    struct Job {
-        char* dst;
-        const char* src;
-        size_t n, pieces;
-        uint64_t id;
-    };
-
     // Takes pieces of `job` until none is left. `next_` holds the job's number with
     // the next piece's, so a helper that comes late takes none of a later job's.
     void work(const Job& job) {
@@ -67,8 +87,7 @@ private:
             do {
                 if (at >> 32 != (job.id & 0xFFFFFFFFu) || (at & 0xFFFFFFFFu) >= job.pieces) return;
             } while (!next_.compare_exchange_weak(at, at + 1, std::memory_order_acq_rel));
-            const size_t b = (at & 0xFFFFFFFFu) * kPiece;
-            std::memcpy(job.dst + b, job.src + b, b + kPiece < job.n ? kPiece : job.n - b);
+            job.one((size_t)(at & 0xFFFFFFFFu));
             done_.fetch_add(1, std::memory_order_acq_rel);
         }
     }
@@ -129,6 +148,10 @@ void host_copy(void* dst, const void* src, size_t n) {
         std::memcpy(dst, src, n);
     else
         pool().copy((char*)dst, (const char*)src, n);
+}
+
+void host_touch(void* p, size_t n) {
+    if (n) pool().touch((char*)p, n);
 }
 
 }  // namespace gr_internal

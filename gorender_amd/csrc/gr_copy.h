@@ -6,5 +6,8 @@
 namespace gr_internal {
 
 void host_copy(void* dst, const void* src, size_t n);
+// Zeroes a byte in every page of memory that nothing has been written to, so that its
+// pages are mapped.
+void host_touch(void* p, size_t n);
 
 }  // namespace gr_internal

@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "gorender_hip.h"
+#include "gr_copy.h"
 #include "gr_error.h"
 
 namespace gr_internal {
@@ -30,6 +31,25 @@ bool copies(size_t n, uint32_t seed) {
     return std::memcmp(src.data(), dst.data(), n) == 0;
 }
 
+// host_touch of [skew, skew + n) of a buffer: a byte of every page of it cleared,
+// nothing around it.
+bool touches(size_t skew, size_t n) {
+    std::vector<unsigned char> buf(skew + n + 4096, 1);
+    gr_internal::host_touch(buf.data() + skew, n);
+    for (size_t i = 0; i < skew; i++)
+        if (!buf[i]) return false;
+    for (size_t i = skew + n; i < buf.size(); i++)
+        if (!buf[i]) return false;
+    const uintptr_t at = (uintptr_t)buf.data() + skew;
+    for (uintptr_t page = at / 4096; n && page <= (at + n - 1) / 4096; page++) {
+        bool any = false;
+        for (uintptr_t i = page * 4096; i < (page + 1) * 4096; i++)
+            if (i >= at && i < at + n) any = any || !buf[skew + (i - at)];
+        if (!any) return false;
+    }
+    return true;
+}
+
 }  // namespace
 
 int main() {
@@ -38,6 +58,10 @@ int main() {
                             kShared + 1, 8 * kPiece + 3, 9u << 20, 2 * kPiece + 77};
     int bad = 0;
     for (size_t n : sizes) bad += !copies(n, (uint32_t)n);
+    for (size_t skew : {(size_t)0, (size_t)1, (size_t)4096, (size_t)2000000})
+        for (size_t n : {(size_t)0, (size_t)1, (size_t)4096, (size_t)4097, (size_t)2u << 20,
+                         ((size_t)2u << 20) + 1, (size_t)11u << 20})
+            bad += !touches(skew, n);
     std::vector<std::thread> callers;
     std::vector<int> wrong(4, 0);
     for (uint32_t t = 0; t < 4; t++)

@@ -34,7 +34,7 @@ void grow_refs_to(gr_context* c, unsigned long long needed);
 // and message a batch holding it would fail with.
 gr_status check_request(gr_context* c, const gr_frame* frame, const gr_object* objects,
                         int32_t num_objects);
-// Pinned memory that host_copy reads, its pages mapped by this thread. Left to the
+// Pinned memory that host_copy reads, with its pages mapped (host_touch). Left to the
 // first copy, its threads take the faults of the same 2 MB pages at once and each
 // does all of the work: the first copy of a 1280x720 frame took 310-450 us, 130 so.
 hipError_t pinned_alloc(void** p, size_t bytes);
