@@ -1573,9 +1573,9 @@ __global__ __launch_bounds__(kScanThreads) void k_bin_scan(
         const int i = (int)threadIdx.x + k * kScanThreads;
         v0[k] = i < ntiles ? gld(&cnt[i]) : 0u;
     }
-    // The launch's references, where parts are smaller than split_refs (launches of
-    // few tiles). A frame that overflowed may be clearing its own counts: its batch
-    // is drawn again.
+    // The launch's references (in 32 bits: with more it overflows), where parts are
+    // smaller than split_refs (launches of few tiles). A frame that overflowed may be
+    // clearing its own counts: its batch is drawn again.
     const bool shared = nframes > 1 && part_refs < split_refs;  // at most kAllTiles tiles
     constexpr int kAllTiles = 4 * kScanThreads;
     uint4 all4 = make_uint4(0u, 0u, 0u, 0u);
@@ -1633,20 +1633,19 @@ __global__ __launch_bounds__(kScanThreads) void k_bin_scan(
     for (int i = (int)threadIdx.x + kKeep * kScanThreads; i < ntiles; i += kScanThreads)
         local += gld(&cnt[i]);
     local = wave_sum_u64(local);
-    unsigned long long all = local;
-    if (shared)
-        all = wave_sum_u64((unsigned long long)all4.x + all4.y + all4.z + all4.w + all1);
-    if (lane == 0) {
-        wsum[wave] = local;
-        wsplit[wave] = all;
+    if (lane == 0) wsum[wave] = local;
+    if (shared) {
+        const uint32_t all = wave_sum_u32(all4.x + all4.y + all4.z + all4.w + all1);
+        if (lane == 0) wsplit[wave] = all;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
         unsigned long long tot = 0;
-        all = 0;
-        for (int w = 0; w < NW; w++) {
-            tot += wsum[w];
-            all += wsplit[w];
+        for (int w = 0; w < NW; w++) tot += wsum[w];
+        uint32_t all = (uint32_t)tot;
+        if (shared) {
+            all = 0u;
+            for (int w = 0; w < NW; w++) all += (uint32_t)wsplit[w];
         }
         longest_s = min(split_refs, max(part_refs, (uint32_t)((float)all * inv_held)));
         // One frame starts at 0, without waiting for the counter.
