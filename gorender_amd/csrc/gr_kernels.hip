@@ -1824,7 +1824,7 @@ __global__ __launch_bounds__(kFillThreads) void k_bin_fill(const DevFrame* __res
         // triangles of 8 pixels at 3840x2160 90 | 14, at 7680x4320 238 | 14, of 60
         // pixels 154 | 49 and 437 | 49; 200,000 of 30 pixels at 1920x1080 78 | 176,
         // at 2560x1440 83 | 111, at 3840x2160 137 | 60; 2,000 of 150 pixels at
-        // 1920x1080 87 | 121, at 3840x2160 304 | 154; 20,000 of 60 pixels at 1280x720
+        // 1920x1080 87 | 152, at 3840x2160 304 | 154; 20,000 of 60 pixels at 1280x720
         // in 8x8 tiles 498 | 351; a sphere of 212 faces at 1920x1080 43 | 77.
         uint32_t row = 0u, nrefs = 0u;  // atomics in a row; references
         each_range([&](const TileRect& t, uint32_t) {
